@@ -218,10 +218,12 @@ def run_paths(isg, args, wl, common, otrue, mes, paths, warmup, steps, timing):
                 continue
             ptime = timing
             fused = fused or s.tuning_get(fast_prec, 1, "leaf") == 1
-            # the split-FP16 near field: k_near_h16 (tuning value 128) serves launches of >= 4
-            # right-hand sides on a grid of >= 8 x 8 leaf boxes, k_near_h16w (256) grids of >= 16 x 8
+            # the split-FP16 near field k_near_h16 (tuning values 128 and 256) serves grids of >= 8 x 8
+            # leaf boxes; the built-in rule (-1) takes it from 256 workgroups of 64 boxes on
             nv = s.tuning_get(1, 1 if batch >= 16 else 0, "near")
-            if fast_prec == 1 and ((nv == 128 and batch >= 4 and wl["level"] >= 4) or (nv == 256 and wl["level"] >= 5)):
+            if nv == -1 and 4 ** (wl["level"] - 1) // 64 * batch >= 256:
+                nv = 128
+            if fast_prec == 1 and nv in (128, 256) and wl["level"] >= 4:
                 split = split or nv
         res[p] = run_path(s, d, warmup, steps, p, ptime)
         contrast[p] = d.get("o")
@@ -451,9 +453,9 @@ def main():
             "kernel_tuning": args.tuning,
         },
         "roofline": {
-            "kernel": ("%s (P2P + L2P on v_mfma_f32_16x16x32_f16, FP32 operands split into FP16 hi + lo)"
-                       % ("k_near_h16w" if split == 256 else "k_near_h16")
-                       if split else "k_near_mfma (P2P + L2P on v_mfma_%s_16x16x4)" % prec),
+            "kernel": ("%s (P2P + L2P in the mirror-symmetric basis on v_mfma_f32_16x16x32_f16, FP32 operands split "
+                       "into FP16 hi + lo)" % ("k_near_h16w (= k_near_h16)" if split == 256 else "k_near_h16")
+                       if split else "k_near_mfma (P2P + L2P in the mirror-symmetric basis on v_mfma_%s_16x16x4)" % prec),
             "bound": "mfma",
             "achieved": round(achieved, 2),
             "peak": peak,
@@ -464,12 +466,13 @@ def main():
                               "(rocprofv3 FETCH_SIZE x2 + WRITE_SIZE x1, copy-calibrated)"
                               if traffic else None,
             "flops_per_rhs_launch": flops_mv,
-            "note": ("achieved counts 8 flops per complex multiply-add; the split kernel executes each real product "
-                     "as three FP16 products (hi.hi + hi.lo + lo.hi) in the four-product complex form, 24 FP16 "
-                     "flops per complex multiply-add, so its executed MFMA rate is 3 x achieved and its ceiling "
-                     "for this arithmetic is peak / 3" if split else
-                     "complex products in the three-product form: the matrix cores execute 6 of the 8 "
-                     "algorithmic flops per complex multiply-add, so the executed MFMA rate is 0.75 x achieved"),
+            "note": ("achieved counts the dense blocks' 8 flops per complex multiply-add; the mirror-symmetric basis "
+                     "needs a quarter of those multiplications, and the split kernel executes each real product as "
+                     "three FP16 products (hi.hi + hi.lo + lo.hi) in the four-product complex form: its executed MFMA "
+                     "rate is 0.75 x achieved (0.83 x with the padding of its k-chunks)" if split else
+                     "achieved counts the dense blocks' 8 flops per complex multiply-add; the mirror-symmetric basis "
+                     "needs a quarter of those multiplications, the three-product form 6 of the 8 flops: the executed "
+                     "MFMA rate is 0.19 x achieved"),
             "frac_of_split_ceiling": round(3 * achieved / peak, 4) if split else None,
             "avg_launch_ms": round(near_ms / max(near_n, 1), 4),
             "launches": near_n,

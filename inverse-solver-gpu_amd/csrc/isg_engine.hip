@@ -15,6 +15,7 @@
 
 #include "isg_kernels.hpp"
 #include "isg_near_h16.hpp"
+#include "isg_near_sym.hpp"
 #include "isg_setup_kernels.hpp"
 #include "isg_solver_kernels.hpp"
 
@@ -218,6 +219,15 @@ void Engine::upload(DevOp<T>& d) {
       if (op64_.shiftL[i]) d.shiftL[i] = cvt(op64_.shiftL[i], (size_t)4 * P_.nsamp[i]);
       if (op64_.trans[i]) d.trans[i] = cvt(op64_.trans[i], (size_t)49 * P_.nsamp[i]);
     }
+    ISG_HIP(hipGetLastError());
+    ISG_HIP(hipStreamSynchronize(stream_));
+  }
+  // mirror-symmetric near-field and L2P tables, from the FP64 ones
+  const int Sl = P_.nsamp[L - 1];
+  d.sym_near = (cplx<T>*)dalloc((size_t)4 * kSymK * 16 * sizeof(cplx<T>));
+  d.sym_l2p = (cplx<T>*)dalloc((size_t)4 * sym_reps(Sl) * 16 * sizeof(cplx<T>));
+  if (ok()) {
+    k_sym_tables<T><<<64, 256, 0, stream_>>>(op64_.near, op64_.basisT, Sl, d.sym_near, d.sym_l2p);
     ISG_HIP(hipGetLastError());
     ISG_HIP(hipStreamSynchronize(stream_));
   }
@@ -470,14 +480,14 @@ Engine::~Engine() {
 }
 
 // Split-FP16 tables of k_near_h16 and k_p2m_h16 from the FP32 operator's
-// near-field, L2P and P2M tables, each with the power-of-two scale that puts
-// its largest component just below 2^14.
+// symmetric near-field and L2P tables and its P2M table, each with the
+// power-of-two scale that puts its largest component just below 2^14.
 void Engine::build_split16() {
   if (!ok()) return;
-  const int S = P_.nsamp[P_.L - 1], nlc = (S + 31) / 32, ncolp = 16 * ((S + 15) / 16);
-  std::vector<zf> nf((size_t)9 * 4096), bf((size_t)S * 64), cf((size_t)64 * S);
-  ISG_HIP(hipMemcpy(nf.data(), op32_.near, nf.size() * sizeof(zf), hipMemcpyDeviceToHost));
-  ISG_HIP(hipMemcpy(bf.data(), op32_.basisT, bf.size() * sizeof(zf), hipMemcpyDeviceToHost));
+  const int S = P_.nsamp[P_.L - 1], nrep = sym_reps(S), ncolp = 16 * ((S + 15) / 16);
+  std::vector<zf> nf((size_t)4 * kSymK * 16), bf((size_t)4 * nrep * 16), cf((size_t)64 * S);
+  ISG_HIP(hipMemcpy(nf.data(), op32_.sym_near, nf.size() * sizeof(zf), hipMemcpyDeviceToHost));
+  ISG_HIP(hipMemcpy(bf.data(), op32_.sym_l2p, bf.size() * sizeof(zf), hipMemcpyDeviceToHost));
   ISG_HIP(hipMemcpy(cf.data(), op32_.coeffT, cf.size() * sizeof(zf), hipMemcpyDeviceToHost));
   if (!ok()) return;
   auto absmax = [](const std::vector<zf>& v) {
@@ -488,15 +498,11 @@ void Engine::build_split16() {
   near16_et_ = h16_scale_exp(absmax(nf));
   bas16_eb_ = h16_scale_exp(absmax(bf));
   p2m16_ec_ = h16_scale_exp(absmax(cf));
-  near16_ = dalloc((size_t)18 * 1024 * 16);
-  bas16_ = dalloc((size_t)nlc * 1024 * 16);
+  near16_ = S <= kS16MaxS ? dalloc((size_t)(kS16Chunks + 1) * 1024 * 16) : nullptr;
   p2m16_ = S <= 16 * kP2mH16MaxCB ? dalloc((size_t)2 * 16 * ncolp * 16) : nullptr;
-  if (!near16_ || !bas16_) return;
-  // near[s][k][m] (k = source pixel), basisT[k][m] (k = local sample), coeffT[n][s] (n = pixel)
-  k_split16<<<(18 * 256 + 255) / 256, 256, 0, stream_>>>(op32_.near, 2, 4096, 64, 64, 64, 64, near16_et_, 18,
-                                                          (v8h*)near16_);
-  k_split16<<<(nlc * 256 + 255) / 256, 256, 0, stream_>>>(op32_.basisT, nlc, 0, S, 64, 64, 64, bas16_eb_, nlc,
-                                                          (v8h*)bas16_);
+  if (near16_)
+    k_split16_sym<<<(kS16Chunks + 1), 256, 0, stream_>>>(op32_.sym_near, near16_et_, op32_.sym_l2p, nrep, bas16_eb_,
+                                                         (v8h*)near16_);
   if (p2m16_)
     k_split16<<<(2 * 4 * ncolp + 255) / 256, 256, 0, stream_>>>(op32_.coeffT, 2, 0, 64, S, S, ncolp, p2m16_ec_, 2,
                                                                 (v8h*)p2m16_);
@@ -585,7 +591,8 @@ template <typename T, typename TI>
 void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, const NearPost<TI>* prep) {
   const int Lf = P_.L - 1, S = P_.nsamp[Lf], B = P_.B;
   const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).p2m_nb;
-  int nb = force > 0 ? force : (tuned > 0 ? tuned : (B >= 32 ? 32 : 16));
+  // built-in rule: 32-box tiles once they fill the chip, else 16 (64 px, one system: 12.9 -> 9.6 us)
+  int nb = force > 0 ? force : (tuned > 0 ? tuned : ((long)(B / 32) * nrhs >= 256 ? 32 : 16));
   DevOp<T>& d = ops<T>();
   cplx<T>* out = d.agm + lvl_off_[Lf];
   long as = (long)lvl_size_[Lf];
@@ -792,45 +799,23 @@ int Engine::launch_near(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act
   const int Lf = P_.L - 1, S = P_.nsamp[Lf], B = P_.B;
   const long N = P_.N, ls = (long)lvl_size_[Lf];
   const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).near_nb;
-  int nb = force > 0 ? force : (tuned > 0 ? tuned : (B >= 32 ? 32 : 16));
+  // Built-in rule: the split kernel once its 64-box workgroups fill the chip (one per CU), else 16-box
+  // tiles.  Measured (us per launch, 16-box / split): 112 workgroups 15.2 / 17.7, 256 22.1 / 19.2,
+  // 960 57 / 39, 16384 877 / 498; wider tiles of k_near_mfma were never faster (64 px 13.6 / 21.5 at 32).
+  int nb = force > 0 ? force : (tuned > 0 ? tuned : (sizeof(T) == 4 && (long)(B / 64) * nrhs >= 256 ? kNearSplit : 16));
   DevOp<T>& d = ops<T>();
   const cplx<T>* loc = d.agl + lvl_off_[Lf];
   const NearPost<TI> pp = post ? *post : NearPost<TI>();
   const int kt = sizeof(T) == 4 ? KT_NEAR32 : KT_NEAR;
-  if (nb == kNearSplitWide) {
-    // split-FP16 kernel with 128-box tiles of one right-hand side
-    if constexpr (sizeof(T) == 4 && sizeof(TI) == 4) {
-      if (with_near && B % 128 == 0 && near16_ && bas16_ && pp.mode != 3) {
-        dim3 grid(B / 128, nrhs), blk(kBlock);
-        auto go = [&](auto modec) {
-          k_near_h16w<decltype(modec)::value><<<grid, blk, kH16WLds, stream_>>>(
-              y, N, loc, ls, r, N, (const v8h*)near16_, near16_et_, (const v8h*)bas16_, bas16_eb_, S, 1 << Lf, act,
-              pp);
-        };
-        prof_begin(kt);
-        if (pp.mode == 1)
-          go(std::integral_constant<int, 1>());
-        else if (pp.mode == 2)
-          go(std::integral_constant<int, 2>());
-        else
-          go(std::integral_constant<int, 0>());
-        prof_end(kt);
-        return B / 128;
-      }
-    }
-    nb = kNearSplit;
-  }
-  if (nb == kNearSplit) {
+  if (nb == kNearSplit || nb == kNearSplitWide) {
     // split-FP16 kernel: FP32 operator on FP32 vectors, near field included,
     // 64-box tiles, BiCGSTAB post steps (not the FP64 residual check)
     if constexpr (sizeof(T) == 4 && sizeof(TI) == 4) {
-      // (pairs of right-hand sides: below 4 the workgroups are few and half idle)
-      if (with_near && B % 64 == 0 && near16_ && bas16_ && pp.mode != 3 && (nrhs >= 4 || force == kNearSplit)) {
-        dim3 grid(B / 64, (nrhs + 1) / 2), blk(kBlock);
+      if (with_near && B % 64 == 0 && near16_ && pp.mode != 3) {
+        dim3 grid(B / 64, nrhs), blk(kBlock);
         auto go = [&](auto modec) {
-          k_near_h16<decltype(modec)::value><<<grid, blk, kH16Lds, stream_>>>(
-              y, N, loc, ls, r, N, (const v8h*)near16_, near16_et_, (const v8h*)bas16_, bas16_eb_, S, 1 << Lf, nrhs,
-              act, pp);
+          k_near_h16<decltype(modec)::value><<<grid, blk, s16_lds(S), stream_>>>(
+              y, N, loc, ls, r, N, (const v8h*)near16_, near16_et_, bas16_eb_, S, 1 << Lf, act, pp);
         };
         prof_begin(kt);
         if (pp.mode == 1)
@@ -843,11 +828,12 @@ int Engine::launch_near(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act
         return B / 64;
       }
     }
-    nb = B >= 32 ? 32 : 16;
+    nb = 16;
   }
   if (nb == 64 && sizeof(T) != 4) nb = 32;  // 64-box tiles: FP32 only (LDS)
   if (B % nb != 0) nb = 16;
-  size_t lds = (size_t)near_lds_elems(nb, S) * sizeof(cplx<T>);
+  while (nb > 16 && (size_t)near_sym_elems<T>(nb, S, with_near) * sizeof(cplx<T>) > kLdsLimit) nb /= 2;
+  size_t lds = (size_t)near_sym_elems<T>(nb, S, with_near) * sizeof(cplx<T>);
   dim3 grid(B / nb, nrhs), blk(kBlock);
   if (pp.mode == 3 && !(sizeof(T) == 8 && sizeof(TI) == 8 && nb <= 32)) {
     set_error("near field: the residual-check epilogue is FP64 only");
@@ -858,7 +844,7 @@ int Engine::launch_near(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act
   // budget (and occupancy) of a kernel without the post epilogue
   auto go = [&](auto nbc, auto modec) {
     k_near_mfma<T, TI, decltype(nbc)::value, decltype(modec)::value>
-        <<<grid, blk, lds, stream_>>>(y, N, loc, ls, r, N, d.near, d.basisT, S, lv, wn, act, pp);
+        <<<grid, blk, lds, stream_>>>(y, N, loc, ls, r, N, d.sym_near, d.sym_l2p, S, lv, wn, act, pp);
   };
   using I16 = std::integral_constant<int, 16>;
   using I32 = std::integral_constant<int, 32>;
@@ -1446,7 +1432,7 @@ void Engine::autotune_prec(int nrhs, int reps) {
   const int widths[5] = {16, 32, 64, kNearSplit, kNearSplitWide};
   auto width_ok = [&](int c) {
     if (c == 3) return sizeof(T) == 4 && P_.B % 64 == 0 && near16_ != nullptr;
-    if (c == 4) return sizeof(T) == 4 && P_.B % 128 == 0 && near16_ != nullptr;
+    if (c == 4) return false;  // the same kernel as 128
     return P_.B % widths[c] == 0 && (widths[c] < 64 || sizeof(T) == 4);
   };
   int c = pick(5, width_ok, [&](int c) {

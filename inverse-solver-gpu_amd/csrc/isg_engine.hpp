@@ -64,6 +64,8 @@ struct DevOp {
   cplx<T>* near = nullptr;     // [9][64][64]
   cplx<T>* coeffT = nullptr;   // [64][S_leaf]
   cplx<T>* basisT = nullptr;   // [S_leaf][64]
+  cplx<T>* sym_near = nullptr;  // mirror-symmetric classes of both (k_sym_tables)
+  cplx<T>* sym_l2p = nullptr;
   std::vector<T*> interpT, anterpT, band_m2m, band_l2l;  // band blocks [nrb][KB][16]
   std::vector<int*> bs0_m2m, bs0_l2l;                    // window start of each band block
   std::vector<cplx<T>*> shiftM, shiftL, trans;
@@ -194,7 +196,7 @@ class Engine {
   void upload(DevOp<T>& d);
   template <typename T>
   void plan_interp(DevOp<T>& d, std::vector<InterpShape>& m2m, std::vector<InterpShape>& l2l);
-  // split-FP16 near-field and L2P tables of the FP32 operator (k_near_h16)
+  // split-FP16 tables of the FP32 operator (k_near_h16, k_p2m_h16)
   void build_split16();
   // operator with tables / multipoles of type T on vectors of type TI
   template <typename T, typename TI>
@@ -266,10 +268,9 @@ class Engine {
   bool checked_h_ = false;
   DevOp<double> op64_;
   DevOp<float> op32_;
-  // k_near_h16 tables ([9 x 2][4][4][64] and [ceil(S / 32)][4][4][64] groups
-  // of 8 FP16) and their power-of-two scale exponents
+  // k_near_h16 table (k_split16_sym: 6 chunks of 1024 groups of 8 FP16; null
+  // for S > kS16MaxS) and the power-of-two scale exponents of its two parts
   void* near16_ = nullptr;
-  void* bas16_ = nullptr;
   int near16_et_ = 0, bas16_eb_ = 0;
   // k_p2m_h16 table ([2][4][4][16 ceil(S / 16)] groups of 8 FP16; null for S > 96) and its exponent
   void* p2m16_ = nullptr;

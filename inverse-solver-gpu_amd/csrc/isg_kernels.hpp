@@ -6,8 +6,8 @@
 //   k_m2m_lds    child -> parent interpolate+shift  (kernels.cu:83-136)
 //   k_m2l_tile   diagonal translation               (kernels.cu:239-266)
 //   k_l2l_lds    parent -> child shift+anterpolate  (kernels.cu:137-238)
-//   k_near_mfma  near field + leaf receiving patterns on the matrix cores
-//                                                (kernels.cu:32-81, :292-319)
+//   k_near_mfma (isg_near_sym.hpp)  near field + leaf receiving patterns on the
+//                matrix cores                     (kernels.cu:32-81, :292-319)
 //   k_rx_*    receiver interpolation / anterpolation (matvec_gpu.cu:351-361, :395-401)
 // Grids are (work items / 256, right-hand sides); blockIdx.y selects the
 // right-hand side and an optional `act` mask skips converged ones.
@@ -119,13 +119,7 @@ __global__ void __launch_bounds__(kBlock) k_l2l(const cplx<T>* __restrict__ par,
 }
 
 // ---------------------------------------------------------------------------
-// Matrix-core (MFMA) near field.  For a tile of NB Morton-consecutive leaf
-// boxes the output r[box][m] (64 rows m = test pixel, NB columns) is one
-// complex GEMM over K = 9*64 (near blocks times the gathered neighbour
-// pixels) + S (leaf receiving pattern times the leaf locals, i.e. L2P), so
-// the near field and L2P are fused and r is written once.
-// Wave w owns rows 16w..16w+15; each 16x16 output block accumulates four real
-// products (re*re, -im*im, re*im, im*re) with v_mfma_*_16x16x4.  Operand
+// Matrix-core products.  Operand
 // layout of the 16x16x4 instructions (checked on gfx950): A[i][k] in lane
 // i + 16k, B[k][j] in lane j + 16k; the 16x16 result D[i][j] is in lane
 // j + 16(i/4), register i%4 for f32 and in lane j + 16(i%4), register i/4
@@ -231,165 +225,12 @@ __device__ __forceinline__ zd stv(cplx<V>* a, long i, zd v) {
   return ccast<double>(w);  // the value as stored
 }
 
-// LDS row length (complex elements) of the near/L2P tile: 64 pixels or S
-// locals, plus one element of padding so 16 lanes reading 16 different rows
-// hit 16 different banks.
-// LDS elements of k_near_mfma<NB>: the (TX+2) x (TY+2) halo boxes of 65
-// elements, later reused for NB rows of S + 1 leaf locals.
-__host__ __device__ inline int near_lds_elems(int NB, int S) {
-  int tx = (NB == 16) ? 4 : 8, ty = NB / tx;
-  int halo = (tx + 2) * (ty + 2) * 65, l2p = NB * (S + 1);
-  return halo > l2p ? halo : l2p;
-}
-
+// Output of a near-field kernel whose NB x 64 products are in LDS: stored, or
+// the BiCGSTAB post step / residual check of NearPost.
 template <typename T, typename TI, int NB, int POST>
-__global__ void __launch_bounds__(kBlock) k_near_mfma(const cplx<TI>* __restrict__ y, long ys,
-                                                      const cplx<T>* __restrict__ loc, long ls,
-                                                      cplx<TI>* __restrict__ r, long rs,
-                                                      const cplx<T>* __restrict__ near,
-                                                      const cplx<T>* __restrict__ basisT, int S, int nbs,
-                                                      int with_near, const int* __restrict__ act,
-                                                      NearPost<TI> post) {
-  typedef typename Mfma<T>::v4 v4;
-  constexpr int NN = NB / 16;
-  // Morton-consecutive NB boxes form a TX x TY block; with its one-box halo
-  // the nine near slots of every box in the tile lie in HX x HY boxes, staged
-  // once (each input pixel enters LDS once per tile instead of once per slot).
-  constexpr int TX = (NB == 16) ? 4 : 8, TY = NB / TX, HX = TX + 2, HY = TY + 2;
-  constexpr int HROW = 65;  // 64 pixels + 1 padding element
-  constexpr int PRE = sizeof(T) == 4 ? 8 : 4;  // L2P table values loaded ahead per MFMA group
-  extern __shared__ char smem_raw[];
-  cplx<T>* tile = reinterpret_cast<cplx<T>*>(smem_raw);
-  const int row = S + 1;    // L2P rows: S locals + 1 padding element
-  int rhs = blockIdx.y;
-  if (rhs_off(act, rhs)) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const long b0 = (long)xcd_block() * NB;
-  // complex products in the three-product form (Mfma::cmac3)
-  v4 p1[NN], p2[NN], p3[NN];
-#pragma unroll
-  for (int j = 0; j < NN; j++) {
-    p1[j] = v4{0, 0, 0, 0};
-    p2[j] = v4{0, 0, 0, 0};
-    p3[j] = v4{0, 0, 0, 0};
-  }
-  const cplx<TI>* yr = y + rhs * ys;
-  if (with_near) {
-    const int X0 = (int)compact2((unsigned)b0), Y0 = (int)compact2((unsigned)b0 >> 1);
-    // pixel offset of each halo box (Morton index * 64), -1 outside the grid:
-    // one Morton conversion per box instead of one per pixel
-    __shared__ int hoff[HX * HY];
-    for (int h = tid; h < HX * HY; h += kBlock) {
-      const int sx = X0 - 1 + h % HX, sy = Y0 - 1 + h / HX;
-      hoff[h] = (sx >= 0 && sy >= 0 && sx < nbs && sy < nbs) ? (int)morton2(sx, sy) * 64 : -1;
-    }
-    __syncthreads();
-    stage<sizeof(T) == 4 ? 8 : 4, cplx<TI>>(
-        HX * HY * 64,
-        [&](int idx) {
-          const int off = hoff[idx >> 6];
-          cplx<TI> v = mkc<TI>(0, 0);
-          if (off >= 0) {
-            v = yr[(long)off + (idx & 63)];
-            // residual check: the input is the iterate x, contrast-weighted here
-            if constexpr (POST == 3) v = prep_val(v, post.g, rhs * post.gs + off + (idx & 63), post.herm != 0);
-          }
-          return v;
-        },
-        [&](int idx, cplx<TI> v) { tile[(idx >> 6) * HROW + (idx & 63)] = ccast<T>(v); });
-    // halo row of column 16 j + li for the centre slot
-    int hc[NN];
-#pragma unroll
-    for (int j = 0; j < NN; j++) {
-      unsigned c = (unsigned)(16 * j + li);
-      hc[j] = ((int)compact2(c >> 1) + 1) * HX + (int)compact2(c) + 1;
-    }
-    __syncthreads();
-    for (int s = 0; s < 9; s++) {
-      const int off = (s / 3 - 1) * HX + (s % 3 - 1);
-      const cplx<T>* A = near + (long)s * 4096 + 16 * w + li;
-#pragma unroll 8
-      for (int kk = 0; kk < 16; kk++) {
-        const int k = 4 * kk + lk;
-        cplx<T> a = A[k * 64];
-        T asum = a.x + a.y;
-#pragma unroll
-        for (int j = 0; j < NN; j++) {
-          cplx<T> bv = tile[(hc[j] + off) * HROW + k];
-          Mfma<T>::cmac3(bv, a, asum, p1[j], p2[j], p3[j]);
-        }
-      }
-    }
-  }
-  // leaf locals -> pixels (L2P) as the last K block
-  __syncthreads();
-  const cplx<T>* lr = loc + rhs * ls + b0 * S;
-  {
-    // element idx = j * S + k goes to tile[j * (S + 1) + k] = tile[idx + j];
-    // j is stepped rather than divided out of idx
-    constexpr int U = sizeof(T) == 4 ? 8 : 4;
-    const int n = NB * S, dj = kBlock / S, dk = kBlock - dj * S;
-    int jb = tid / S, kq = tid - jb * S;
-    for (int e0 = tid; e0 < n; e0 += U * kBlock) {
-      cplx<T> v[U];
-      int ju[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int e = e0 + u * kBlock;
-        ju[u] = jb;
-        v[u] = lr[e < n ? e : n - 1];  // unconditional (clamped) load: the array stays in registers
-        kq += dk;
-        jb += dj;
-        if (kq >= S) {
-          kq -= S;
-          jb++;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int e = e0 + u * kBlock;
-        if (e < n) tile[e + ju[u]] = v[u];
-      }
-    }
-  }
-  __syncthreads();
-  const cplx<T>* A = basisT + 16 * w + li;
-  const int nk = S / 4;  // S is a multiple of 4
-#pragma unroll 1
-  for (int k0 = 0; k0 < nk; k0 += PRE) {
-    cplx<T> a[PRE];
-#pragma unroll
-    for (int u = 0; u < PRE; u++)
-      if (k0 + u < nk) a[u] = A[(4 * (k0 + u) + lk) * 64];
-#pragma unroll
-    for (int u = 0; u < PRE; u++) {
-      if (k0 + u < nk) {
-        const int k = 4 * (k0 + u) + lk;
-        const T asum = a[u].x + a[u].y;
-#pragma unroll
-        for (int j = 0; j < NN; j++) {
-          cplx<T> bv = tile[(16 * j + li) * row + k];
-          Mfma<T>::cmac3(bv, a[u], asum, p1[j], p2[j], p3[j]);
-        }
-      }
-    }
-  }
-  // D[box][m]: lane li holds pixel m = 16w + li.  The product goes through
-  // LDS (the L2P tile is free once every wave has passed the barrier) so
-  // that each thread then takes consecutive elements of the workgroup's
-  // contiguous output range [b0*64, (b0+NB)*64): coalesced stores, and for a
-  // post step coalesced loads and few live registers.
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < NN; j++) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const T re = p1[j][q] - p2[j][q], im = p3[j][q] - p1[j][q] - p2[j][q];
-      tile[(16 * j + Mfma<T>::row(lk, q)) * 64 + 16 * w + li] = mkc<T>(re, im);
-    }
-  }
-  __syncthreads();
+__device__ __forceinline__ void near_epilogue(const cplx<T>* tile, cplx<TI>* __restrict__ r, long rs, long b0, int rhs,
+                                              const NearPost<TI>& post) {
+  const int tid = threadIdx.x;
   if constexpr (POST == 0) {
     cplx<TI>* out = r + rhs * rs + b0 * 64;
 #pragma unroll 4

@@ -14,21 +14,17 @@
 // block.  The scales are exact powers of two and are divided out of the FP32
 // accumulators at the end.
 //
-// Workgroup: 8 x 8 Morton-consecutive leaf boxes (64) of two right-hand sides
-// = 128 MFMA rows, so each table fragment read from L2 feeds 8 row blocks
-// (the table, 8 B per complex entry in its four FP16 parts, is what limits a
-// split kernel: the matrix cores consume it ~5 times faster than the FP32
-// kernel does, which reads the same 8 B per entry for 16 or 32 rows).  Wave w
-// owns right-hand side w / 2 of the pair (its 4 row blocks of 16 boxes) and
-// output pixels 32 (w % 2) .. +31 (2 column blocks): every A fragment read
-// from LDS feeds 2 column blocks, every B fragment 4 row blocks.
+// The near field and L2P run in the mirror-symmetric basis of a leaf box
+// (isg_near_sym.hpp: a quarter of the multiplications): the data operand is
+// the folded quarter window, formed in FP32 and then split.
 //
 // Reference counterpart: the near-field and L2P stages of matvec_gpu.cu
-// (kernels.cu:32-81, :292-319); the result equals the FP32 kernel's to the
+// (kernels.cu:32-81, :292-319); the results equal the FP32 kernels' to the
 // split's 2^-22.
 #pragma once
 
 #include "isg_kernels.hpp"
+#include "isg_near_sym.hpp"
 
 namespace isg {
 
@@ -36,22 +32,10 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
-// Tuning value of the near stage that selects this kernel (FP32 operator).
+// Tuning values of the near and P2M stages that select the split kernels
+// (FP32 operator); the near stage has one kernel for both.
 constexpr int kNearSplit = 128;
-// Halo of the 8 x 8 box tile: 10 x 10 boxes at a row pitch of 12 positions,
-// so the 16 boxes of a row block (a 4 x 4 block) read by 16 lanes fall in 16
-// different 16-byte bank groups.  Positions (and the boxes of the L2P chunk)
-// are stored XOR 2 g for k group g, so that the four groups of one box, which
-// consecutive lanes write, also fall in different bank groups (a bijection on
-// the low bits: readers of one group keep distinct banks; 119 ^ 6 < 120).
-constexpr int kH16Pitch = 12;
-constexpr int kH16Pos = kH16Pitch * 10;
-// LDS (bytes): half of the halo (32 of the 64 pixels of each box) as
-// [rhs 2][part 4][k group 4][position 120] x 8 FP16; reused for a 32-local
-// chunk of the L2P ([rhs][part][k group][box 64] x 8 FP16) and for one
-// right-hand side's 64 x 64 complex output tile.
-constexpr size_t kH16Lds = (size_t)2 * 4 * 4 * kH16Pos * 16;
-static_assert(kH16Lds >= (size_t)64 * 64 * 8 && kH16Lds >= (size_t)2 * 4 * 4 * 64 * 16, "LDS reuse");
+constexpr int kNearSplitWide = 256;
 
 // Power-of-two exponent e with |2^e m| < 2^14 for the largest magnitude m
 // (0 for m = 0 or m not finite: Inf / NaN then propagate as in FP32).
@@ -164,636 +148,311 @@ static __global__ void __launch_bounds__(256) k_split16(const zf* __restrict__ s
   for (int P = 0; P < 4; P++) out[((long)(b * 4 + P) * 4 + g) * ncolp + m] = ph[P];
 }
 
-// As h16_cmac with the negation on the data side: na = -a2, -a3 (the table
-// fragments are then used as loaded; fewer live registers when one table
-// fragment serves several data fragments one after another).
-__device__ __forceinline__ void h16_cmac_na(const v8h (&a)[4], const v8h (&na)[2], const v8h (&b)[4], v4f& cr,
-                                            v4f& ci) {
-  cr = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[0], cr, 0, 0, 0);
-  ci = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[2], ci, 0, 0, 0);
-  cr = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[1], cr, 0, 0, 0);
-  ci = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[3], ci, 0, 0, 0);
-  cr = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[1], b[0], cr, 0, 0, 0);
-  ci = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[1], b[2], ci, 0, 0, 0);
-  cr = __builtin_amdgcn_mfma_f32_16x16x32_f16(na[0], b[2], cr, 0, 0, 0);
-  ci = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[2], b[0], ci, 0, 0, 0);
-  cr = __builtin_amdgcn_mfma_f32_16x16x32_f16(na[0], b[3], cr, 0, 0, 0);
-  ci = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[2], b[1], ci, 0, 0, 0);
-  cr = __builtin_amdgcn_mfma_f32_16x16x32_f16(na[1], b[2], cr, 0, 0, 0);
-  ci = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[3], b[0], ci, 0, 0, 0);
+// Split tables of k_near_h16, from the FP32 symmetric ones: chunk b of 32
+// k-slots, out[b][c][part][lk][col] = 8 FP16 parts (slots 8 lk .. +7).
+//   near (tn, 5 chunks): slot (b, lk, e) is quarter-window pixel (i, j): b < 3:
+//     (4 + e, 4 b + lk), eight pixels of a neighbour box's row; then
+//     (e % 4, 2 (4 (b - 3) + lk) + e / 4), two rows of the box's own half; zero past 144
+//   l2p (tl, 1 chunk): slot (lk, e) is direction orbit 8 lk + e, zero past nrep
+constexpr int kS16Chunks = 5;
+static __global__ void __launch_bounds__(256) k_split16_sym(const zf* __restrict__ tn, int et,
+                                                            const zf* __restrict__ tl, int nrep, int eb,
+                                                            v8h* __restrict__ out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (kS16Chunks + 1) * 4 * 4 * 16) return;
+  const int col = t & 15, lk = (t >> 4) & 3, c = (t >> 6) & 3, b = t >> 8;
+  const float s = ldexpf(1.f, b < kS16Chunks ? et : eb);
+  v8h ph[4];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    zf v = mkc<float>(0.f, 0.f);
+    if (b < kS16Chunks) {
+      const int i = b < 3 ? 4 + e : e & 3, j = b < 3 ? 4 * b + lk : 2 * (4 * (b - 3) + lk) + (e >> 2);
+      if (j < 12) v = tn[(c * kSymK + 12 * j + i) * 16 + col];
+    } else if (8 * lk + e < nrep) {
+      v = tl[(c * nrep + 8 * lk + e) * 16 + col];
+    }
+    h16_split(v.x * s, ph[0], ph[1], e);
+    h16_split(v.y * s, ph[2], ph[3], e);
+  }
+#pragma unroll
+  for (int P = 0; P < 4; P++) out[(((b * 4 + c) * 4 + P) * 4 + lk) * 16 + col] = ph[P];
 }
 
-// Split tables, built once per operator (k_split16):
-//   tab[s][kc][part][g][m] (8 FP16 each): 2^et near[s][32 kc + 8 g + e][m], e = 0..7
-//   bas[kc][part][g][m]    (8 FP16 each): 2^eb basisT[32 kc + 8 g + e][m] (0 for k >= S)
-// Grid (B / 64, ceil(nrhs / 2)), kBlock threads, kH16Lds bytes of dynamic LDS.
+// Near field + L2P of the FP32 operator, split FP16, symmetric classes.
+// Workgroup: 64 Morton-consecutive boxes (8 x 8) of one right-hand side.  The
+// 10 x 10-box halo is loaded once into registers, its largest component sets
+// the data scale (two bits of headroom: a folded value sums four), and the
+// scaled FP32 pixels are staged in LDS.  Wave w owns row
+// blocks 2 (w / 2), +1 (16 boxes each) and the classes odd or even in y by
+// w % 2, even and odd in x: a table fragment then serves two row blocks and a
+// halo pixel is read by two waves.  Per chunk and row block a lane reads the
+// four mirror images of its 8 slots (16-byte reads; the 16 boxes of a block
+// fall in distinct banks), folds them (4 FP32 operations per operand) and
+// splits them (about as many), for 24 MFMAs.
+// What bounds it (1024^2 x 64 right-hand sides, 498 us; the dense split kernel took
+// 900): vector work 320 us, MFMA 123, memory 1.65 GB = 350 us; three workgroups per
+// CU instead of two were worth 572 -> 498 us, hence the 664-element pitch and the
+// 168-register limit.
+constexpr int kS16Box = 66, kS16Row = 664;  // halo layout: 16-byte reads need box / 2 odd, row / 2 = 4 mod 8
+constexpr int kS16Rows = 10 * kS16Row;       // LDS elements of the halo: with the static part 53.7 KB, three workgroups per CU
+// LDS bytes for S leaf directions; the kernel takes S <= 124 (one L2P chunk)
+__host__ __device__ inline size_t s16_lds(int S) {
+  const int l2p = 64 * (S + 1), out = 64 * 64;
+  const int m = l2p > out ? l2p : out;
+  return (size_t)(kS16Rows > m ? kS16Rows : m) * sizeof(zf);
+}
+constexpr int kS16MaxS = 124;
+
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+
+// v - hi, exact, as one mixed-precision multiply-add per element (the compiler
+// would convert hi back and subtract)
+__device__ __forceinline__ v2f h16_rest(v2f v, v2h hi) {
+  v2f r;
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r.x) : "v"(hi), "v"(v.x));
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(hi), "v"(v.y));
+  return r;
+}
+
+// elements e, e + 1 of the four parts of a pair of complex values
+__device__ __forceinline__ void h16_split_pair(v2f re, v2f im, v8h (&a)[4], int e) {
+  const v2h rh = __builtin_convertvector(re, v2h), mh = __builtin_convertvector(im, v2h);
+  const v2h rl = __builtin_convertvector(h16_rest(re, rh), v2h), ml = __builtin_convertvector(h16_rest(im, mh), v2h);
+  a[0][e] = rh.x;
+  a[0][e + 1] = rh.y;
+  a[1][e] = rl.x;
+  a[1][e + 1] = rl.y;
+  a[2][e] = mh.x;
+  a[2][e + 1] = mh.y;
+  a[3][e] = ml.x;
+  a[3][e + 1] = ml.y;
+}
+
 template <int POST>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
 k_near_h16(const zf* __restrict__ y, long ys, const zf* __restrict__ loc, long ls, zf* __restrict__ r, long rs,
-           const v8h* __restrict__ tab, int et, const v8h* __restrict__ bas, int eb, int S, int nbs, int nrhs,
-           const int* __restrict__ act, NearPost<float> post) {
+           const v8h* __restrict__ tab, int et, int eb, int S, int nbs, const int* __restrict__ act,
+           NearPost<float> post) {
+  constexpr int BS = kS16Box, RS = kS16Row;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  v8h* hal = reinterpret_cast<v8h*>(smem_raw);
-  __shared__ int hoff[100];
-  __shared__ float red[4][kBlock / 64];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const int rw = w >> 1, mb0 = 2 * (w & 1);
-  const int rhs[2] = {2 * (int)blockIdx.y, 2 * (int)blockIdx.y + 1};
-  bool on[2];
-#pragma unroll
-  for (int q = 0; q < 2; q++) on[q] = rhs[q] < nrhs && !rhs_off(act, rhs[q]);
-  if (!on[0] && !on[1]) return;
-  const bool mine = sel2(on, rw);  // wave-uniform
-  // a right-hand side that loads may use when its own is off (never read then)
-  const int rv[2] = {on[0] ? rhs[0] : rhs[1], on[1] ? rhs[1] : rhs[0]};
-  const long b0 = (long)xcd_block() * 64;
-  const int X0 = (int)compact2((unsigned)b0), Y0 = (int)compact2((unsigned)b0 >> 1);
-  for (int h = tid; h < 100; h += kBlock) {
-    const int sx = X0 - 1 + h % 10, sy = Y0 - 1 + h / 10;
-    hoff[h] = (sx >= 0 && sy >= 0 && sx < nbs && sy < nbs) ? (int)morton2(sx, sy) * 64 : -1;
-  }
-  __syncthreads();
-
-  // data scale of each right-hand side: largest |re|, |im| over the halo,
-  // from one pass whose loads are all issued before the first comparison
-  // (the accumulators are not live yet)
-  int es[2], el[2];
-  {
-    constexpr int NU = (3200 + kBlock - 1) / kBlock;  // 100 boxes x 32 float4 per right-hand side
-    float m[2] = {0.f, 0.f};
-    float4 v[2][NU];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const float4* yq = reinterpret_cast<const float4*>(y + (long)sel2(rv, q) * ys);
-#pragma unroll
-      for (int u = 0; u < NU; u++) {
-        const int e = tid + u * kBlock, ec = e < 3200 ? e : 3199;
-        const int off = hoff[ec >> 5];
-        v[q][u] = yq[((off < 0 ? 0 : off) >> 1) + (ec & 31)];
-        if (!(sel2(on, q) && e < 3200 && off >= 0)) v[q][u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-#pragma unroll
-      for (int u = 0; u < NU; u++) m[q] = fmaxf(m[q], h16_absmax(v[q][u]));
-    block_max<2>(m, red);
-#pragma unroll
-    for (int q = 0; q < 2; q++) es[q] = h16_scale_exp(m[q]);
-  }
-
-  v4f cr[4][2], ci[4][2];
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      cr[j][c] = v4f{0, 0, 0, 0};
-      ci[j][c] = v4f{0, 0, 0, 0};
-    }
-  // halo position of box 16 j + li (this lane's A row) for the centre slot
-  int hc[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const unsigned c = (unsigned)(16 * j + li);
-    hc[j] = ((int)compact2(c >> 1) + 1) * kH16Pitch + (int)compact2(c) + 1;
-  }
-
-  // ---- near field: two halves of the source pixels (k = 32 kc .. +31)
-  // B fragments of slot s (this lane's 8 k of column li, for both column
-  // blocks); the next slot's are loaded while the current slot's MFMAs run
-  const v8h* tl = tab + lk * 64 + 16 * mb0 + li;  // + (s * 2 + kc) * 1024 + P * 256 + 16 c
-  auto load_b = [&](v8h (&b)[2][4], const v8h* t) {
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-      for (int P = 0; P < 4; P++) b[c][P] = t[P * 256 + 16 * c];
-  };
-  v8h bn[2][4];
-#pragma unroll 1
-  for (int kc = 0; kc < 2; kc++) {
-    __syncthreads();  // the previous half is no longer read
-    if (mine) load_b(bn, tl + (long)kc * 1024);  // in flight during the staging
-    {
-      // units (q, h, g) of 8 source pixels 32 kc + 8 g .. +7 of halo box h
-      float4 v[4][4];
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int u = tid + t * kBlock, uc = u < 800 ? u : 799;
-        const int q = uc / 400, h = (uc >> 2) % 100, g = uc & 3;
-        const int off = hoff[h];
-        const float4* src = reinterpret_cast<const float4*>(y + (long)sel2(rv, q) * ys + (off < 0 ? 0 : off) + 32 * kc + 8 * g);
-#pragma unroll
-        for (int c = 0; c < 4; c++) v[t][c] = src[c];
-      }
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int u = tid + t * kBlock;
-        if (u < 800) {
-          const int q = u / 400, h = (u >> 2) % 100, g = u & 3;
-          const float s = ldexpf(1.f, sel2(es, q));
-          // zero outside the grid and for a right-hand side that is off (its loads used stand-in addresses)
-          const bool ok = sel2(on, q) && hoff[h] >= 0;
-          const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-          v8h ph[4];
-          h16_split4(ok ? v[t][0] : z, ok ? v[t][1] : z, s, ph, 0);
-          h16_split4(ok ? v[t][2] : z, ok ? v[t][3] : z, s, ph, 4);
-          const int p = (h / 10) * kH16Pitch + h % 10;
-#pragma unroll
-          for (int P = 0; P < 4; P++) hal[((q * 4 + P) * 4 + g) * kH16Pos + (p ^ (2 * g))] = ph[P];
-        }
-      }
-    }
-    __syncthreads();
-    if (mine) {
-      const v8h* hb = hal + (rw * 16 + lk) * kH16Pos;  // + P * 4 * kH16Pos + position
-#pragma unroll 1
-      for (int s = 0; s < 9; s++) {
-        const int off = (s / 3 - 1) * kH16Pitch + (s % 3 - 1);
-        v8h b[2][4], nb[2][2];
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-          for (int P = 0; P < 4; P++) b[c][P] = bn[c][P];
-        if (s + 1 < 9) load_b(bn, tl + (long)((s + 1) * 2 + kc) * 1024);
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-          nb[c][0] = h16_neg(b[c][2]);
-          nb[c][1] = h16_neg(b[c][3]);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int p = (hc[j] + off) ^ (2 * lk);
-          v8h a[4];
-#pragma unroll
-          for (int P = 0; P < 4; P++) a[P] = hb[P * 4 * kH16Pos + p];
-#pragma unroll
-          for (int c = 0; c < 2; c++) h16_cmac(a, b[c], nb[c], cr[j][c], ci[j][c]);
-        }
-      }
-    }
-  }
-
-  // ---- L2P: locals of the tile's boxes, in chunks of 32; units (q, box, g):
-  // locals 32 kc + 8 g .. +7 of box b0 + box, loaded a chunk ahead
-  float4 lv[2][4];
-  auto load_loc = [&](int kc) {
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
-      const int u = tid + t * kBlock;
-      const int q = u >> 8, bx = (u >> 2) & 63, g = u & 3;
-      const zf* lb = loc + (long)sel2(rv, q) * ls + (b0 + bx) * S;
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const int k = 32 * kc + 8 * g + 2 * c;
-        lv[t][c] = *reinterpret_cast<const float4*>(lb + (k < S ? k : S - 2));
-      }
-    }
-  };
-  load_loc(0);
-  // locals scale of each right-hand side, read after the near field so that the
-  // staging below finds them in L2
-  {
-    float m[2] = {0.f, 0.f};
-    const int n4 = 32 * S;  // 64 boxes x S locals = 32 S float4 (S even), per right-hand side
-    constexpr int U = 9;
-    for (int e0 = tid; e0 < 2 * n4; e0 += U * kBlock) {
-      float4 t[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int e = e0 + u * kBlock, q = e >= n4 ? 1 : 0, ei = e - q * n4;
-        const float4* lq = reinterpret_cast<const float4*>(loc + (long)sel2(rv, q) * ls + b0 * S);
-        t[u] = lq[ei < n4 ? ei : n4 - 1];
-        if (!(sel2(on, q) && e < 2 * n4)) t[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const float a = h16_absmax(t[u]);
-        if (e0 + u * kBlock >= n4)
-          m[1] = fmaxf(m[1], a);
-        else
-          m[0] = fmaxf(m[0], a);
-      }
-    }
-    __syncthreads();  // red is read by the data scale above
-    block_max<2>(m, red);
-#pragma unroll
-    for (int q = 0; q < 2; q++) el[q] = h16_scale_exp(m[q]);
-  }
-  if (mine) {
-    // near accumulators carry 2^(es + et); bring them to the L2P's 2^(el + eb)
-    const int n = (sel2(el, rw) + eb) - (sel2(es, rw) + et);
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          cr[j][c][i] = ldexpf(cr[j][c][i], n);
-          ci[j][c][i] = ldexpf(ci[j][c][i], n);
-        }
-  }
-  const int nlc = (S + 31) / 32;
-#pragma unroll 1
-  for (int kc = 0; kc < nlc; kc++) {
-    __syncthreads();
-    if (mine) load_b(bn, bas + (long)kc * 1024 + lk * 64 + 16 * mb0 + li);  // in flight during the staging
-    {
-      // converts the chunk's locals, loaded during the previous chunk's MFMAs
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        const int u = tid + t * kBlock;
-        const int q = u >> 8, bx = (u >> 2) & 63, g = u & 3;
-        const float s = ldexpf(1.f, sel2(el, q));
-        float4 v[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const int k = 32 * kc + 8 * g + 2 * c;  // pairs (k, k + 1) lie within S or beyond it together
-          v[c] = (sel2(on, q) && k < S) ? lv[t][c] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        v8h ph[4];
-        h16_split4(v[0], v[1], s, ph, 0);
-        h16_split4(v[2], v[3], s, ph, 4);
-#pragma unroll
-        for (int P = 0; P < 4; P++) hal[((q * 4 + P) * 4 + g) * 64 + (bx ^ (2 * g))] = ph[P];
-      }
-    }
-    __syncthreads();
-    if (kc + 1 < nlc) load_loc(kc + 1);
-    if (mine) {
-      const v8h* hb = hal + (rw * 16 + lk) * 64;  // + P * 256 + box
-      v8h nb[2][2];
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        nb[c][0] = h16_neg(bn[c][2]);
-        nb[c][1] = h16_neg(bn[c][3]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        v8h a[4];
-#pragma unroll
-        for (int P = 0; P < 4; P++) a[P] = hb[P * 256 + ((16 * j + li) ^ (2 * lk))];
-#pragma unroll
-        for (int c = 0; c < 2; c++) h16_cmac(a, bn[c], nb[c], cr[j][c], ci[j][c]);
-      }
-    }
-  }
-
-  // ---- output, one right-hand side at a time through LDS (coalesced stores
-  // and, for a post step, coalesced loads); D[box][m]: box 16 j + 4 lk + i
-  // (register i), pixel m = 16 (mb0 + c) + li
   zf* tile = reinterpret_cast<zf*>(smem_raw);
-#pragma unroll 1
-  for (int q = 0; q < 2; q++) {
-    if (!sel2(on, q)) continue;  // uniform
-    __syncthreads();
-    if (rw == q) {
-      const int n = -(sel2(el, q) + eb);
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-          for (int i = 0; i < 4; i++)
-            tile[(16 * j + 4 * lk + i) * 64 + 16 * (mb0 + c) + li] =
-                mkc<float>(ldexpf(cr[j][c][i], n), ldexpf(ci[j][c][i], n));
-    }
-    __syncthreads();
-    const long o = (long)sel2(rhs, q) * rs + b0 * 64;
-    if constexpr (POST == 0) {
-#pragma unroll 4
-      for (int e = tid; e < 64 * 64; e += kBlock) r[o + e] = tile[e];
-    } else {
-      const zd* gr = post.g + (long)sel2(rhs, q) * post.gs + b0 * 64;
-      zd acc[2] = {mkc<double>(0, 0), mkc<double>(0, 0)};
-      struct In {
-        zf x, aux;  // aux: r~ (mode 1)
-        zd g;
-      };
-      const bool herm = post.herm != 0;
-      stage<2, In>(
-          64 * 64,
-          [&](int e) {
-            In v;
-            v.x = post.x[o + e];
-            if (POST == 1) v.aux = post.rt[o + e];
-            if (herm) v.g = gr[e];  // the forward post step does not use g
-            return v;
-          },
-          [&](int e, In v) {
-            const zf gt = tile[e];
-            const zd gy = mkc<double>((double)gt.x, (double)gt.y);
-            const zd xv = ccast<double>(v.x);
-            const zd px = herm ? csub(xv, cconj(cmul(v.g, gy))) : csub(xv, gy);
-            const zd res = stv(r, o + e, px);
-            if (POST == 1) {
-              const zd a = ccast<double>(v.aux);
-              acc[0].x += a.x * res.x + a.y * res.y;
-              acc[0].y += a.x * res.y - a.y * res.x;
-            } else {
-              acc[0].x += res.x * xv.x + res.y * xv.y;
-              acc[0].y += res.x * xv.y - res.y * xv.x;
-              acc[1].x += res.x * res.x + res.y * res.y;
-            }
-          });
-      block_store<2>(acc, post.part + (long)sel2(rhs, q) * kSlots * gridDim.x, gridDim.x, blockIdx.x);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Split-FP16 near field + L2P with 128-box tiles of ONE right-hand side
-// (tuning value kNearSplitWide): the same arithmetic and table as k_near_h16,
-// the same 128 MFMA rows per table fragment, but a 16 x 8 box tile (halo
-// 18 x 10 boxes: 1.41 x the tile's pixels staged instead of 1.56 x), no
-// half-idle pairs when systems of a batch have converged, and 51 KB of LDS
-// and at most 168 registers, so three workgroups share a CU (k_near_h16: two).
-// Wave w owns row blocks 4 (w / 2) .. +3 (16 boxes each) and column blocks
-// 2 (w % 2), +1.  Halo positions at a row pitch of 20 (= 4 mod 8, as 12 is),
-// stored XOR 2 g as in k_near_h16.  Grid (B / 128, nrhs).
-constexpr int kNearSplitWide = 256;
-constexpr int kH16WPitch = 20;
-constexpr int kH16WPos = kH16WPitch * 10;
-constexpr size_t kH16WLds = (size_t)4 * 4 * kH16WPos * 16;
-static_assert(kH16WLds >= (size_t)64 * 64 * 8 && kH16WLds >= (size_t)4 * 4 * 128 * 16, "LDS reuse");
-
-template <int POST>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
-k_near_h16w(const zf* __restrict__ y, long ys, const zf* __restrict__ loc, long ls, zf* __restrict__ r, long rs,
-            const v8h* __restrict__ tab, int et, const v8h* __restrict__ bas, int eb, int S, int nbs,
-            const int* __restrict__ act, NearPost<float> post) {
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  v8h* hal = reinterpret_cast<v8h*>(smem_raw);
-  __shared__ int hoff[180];
-  __shared__ float red[4][kBlock / 64];
+  __shared__ int hoff[100];
+  __shared__ float red[2][kBlock / 64];
   const int rhs = blockIdx.y;
   if (rhs_off(act, rhs)) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  const int rbh = w >> 1, mb0 = 2 * (w & 1);
-  const long b0 = (long)xcd_block() * 128;
+  const int oy = w & 1, rb0 = 2 * (w >> 1);
+  const float sy = oy ? -1.f : 1.f;
+  const long b0 = (long)xcd_block() * 64;
   const int X0 = (int)compact2((unsigned)b0), Y0 = (int)compact2((unsigned)b0 >> 1);
-  for (int h = tid; h < 180; h += kBlock) {
-    const int sx = X0 - 1 + h % 18, sy = Y0 - 1 + h / 18;
-    hoff[h] = (sx >= 0 && sy >= 0 && sx < nbs && sy < nbs) ? (int)morton2(sx, sy) * 64 : -1;
+  if (tid < 100) {
+    const int hx = tid % 10, hy = tid / 10, sxb = X0 - 1 + hx, syb = Y0 - 1 + hy;
+    hoff[tid] = (sxb >= 0 && syb >= 0 && sxb < nbs && syb < nbs) ? (int)morton2(sxb, syb) * 64 : -1;
   }
   __syncthreads();
-  const zf* yr = y + (long)rhs * ys;
-
-  // data scale: largest |re|, |im| over the halo, all loads issued first
-  int es;
-  {
-    constexpr int NU = 12;  // 180 boxes x 32 float4 = 5760 in two batches of 12 per thread
-    float m[1] = {0.f};
-    const float4* yq = reinterpret_cast<const float4*>(yr);
-#pragma unroll 1
-    for (int e0 = tid; e0 < 5760; e0 += NU * kBlock) {
-      float4 v[NU];
-#pragma unroll
-      for (int u = 0; u < NU; u++) {
-        const int e = e0 + u * kBlock, ec = e < 5760 ? e : 5759;
-        const int off = hoff[ec >> 5];
-        v[u] = yq[((off < 0 ? 0 : off) >> 1) + (ec & 31)];
-        if (!(e < 5760 && off >= 0)) v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int u = 0; u < NU; u++) m[0] = fmaxf(m[0], h16_absmax(v[u]));
-    }
-    block_max<1>(m, red);
-    es = h16_scale_exp(m[0]);
-  }
-
-  v4f cr[4][2], ci[4][2];
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      cr[j][c] = v4f{0, 0, 0, 0};
-      ci[j][c] = v4f{0, 0, 0, 0};
-    }
-  // halo position of box 16 (4 rbh + j) + li for the centre slot
-  int hc[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const unsigned c = (unsigned)(16 * (4 * rbh + j) + li);
-    hc[j] = ((int)compact2(c >> 1) + 1) * kH16WPitch + (int)compact2(c) + 1;
-  }
-
-  const v8h* tl = tab + lk * 64 + 16 * mb0 + li;  // + (s * 2 + kc) * 1024 + P * 256 + 16 c
-  auto load_b = [&](v8h (&b)[2][4], const v8h* t) {
+  // table fragments of this wave's two classes (2 oy, 2 oy + 1)
+  const v8h* tl = tab + (2 * oy * 4 * 4 + lk) * 16 + li;  // + chunk * 1024 + class * 256 + part * 64
+  auto load_b = [&](v8h (&b)[2][4], int chunk) {
 #pragma unroll
     for (int c = 0; c < 2; c++)
 #pragma unroll
-      for (int P = 0; P < 4; P++) b[c][P] = t[P * 256 + 16 * c];
+      for (int P = 0; P < 4; P++) b[c][P] = tl[chunk * 1024 + c * 256 + P * 64];
   };
-  const float sd = ldexpf(1.f, es);
-  v8h bn[2][4];
-#pragma unroll 1
-  for (int kc = 0; kc < 2; kc++) {
-    __syncthreads();  // the previous half is no longer read
-    load_b(bn, tl + (long)kc * 1024);  // in flight during the staging
-    {
-      // units (h, g) of 8 source pixels 32 kc + 8 g .. +7 of halo box h
-      float4 v[3][4];
+  v8h bt[2][2][4];
+  load_b(bt[0], 0);
+  int es;
+  {
+    constexpr int NU = 13;  // 100 boxes x 32 float4
+    const float4* yq = reinterpret_cast<const float4*>(y + (long)rhs * ys);
+    float4 v[NU];
+    float m[1] = {0.f};
 #pragma unroll
-      for (int t = 0; t < 3; t++) {
-        const int u = tid + t * kBlock, uc = u < 720 ? u : 719;
-        const int h = uc >> 2, g = uc & 3;
-        const int off = hoff[h];
-        const float4* src = reinterpret_cast<const float4*>(yr + (off < 0 ? 0 : off) + 32 * kc + 8 * g);
-#pragma unroll
-        for (int c = 0; c < 4; c++) v[t][c] = src[c];
-      }
-#pragma unroll
-      for (int t = 0; t < 3; t++) {
-        const int u = tid + t * kBlock;
-        if (u < 720) {
-          const int h = u >> 2, g = u & 3;
-          const bool ok = hoff[h] >= 0;  // zero outside the grid
-          const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-          v8h ph[4];
-          h16_split4(ok ? v[t][0] : z, ok ? v[t][1] : z, sd, ph, 0);
-          h16_split4(ok ? v[t][2] : z, ok ? v[t][3] : z, sd, ph, 4);
-          const int p = (h / 18) * kH16WPitch + h % 18;
-#pragma unroll
-          for (int P = 0; P < 4; P++) hal[(P * 4 + g) * kH16WPos + (p ^ (2 * g))] = ph[P];
-        }
-      }
+    for (int u = 0; u < NU; u++) {
+      const int e = tid + u * kBlock, ec = e < 3200 ? e : 3199;
+      const int off = hoff[ec >> 5];
+      v[u] = yq[((off < 0 ? 0 : off) >> 1) + (ec & 31)];
+      if (off < 0) v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    __syncthreads();
-    const v8h* hb = hal + lk * kH16WPos;  // + P * 4 * kH16WPos + position
-#pragma unroll 1
-    for (int s = 0; s < 9; s++) {
-      const int off = (s / 3 - 1) * kH16WPitch + (s % 3 - 1);
-      v8h b[2][4];
 #pragma unroll
-      for (int c = 0; c < 2; c++)
+    for (int u = 0; u < NU; u++) m[0] = fmaxf(m[0], h16_absmax(v[u]));  // clamped repeats change no maximum
+    block_max<1>(m, red);
+    es = h16_scale_exp(m[0]) - 2;
+    const float s = ldexpf(1.f, es);
 #pragma unroll
-        for (int P = 0; P < 4; P++) b[c][P] = bn[c][P];
-      if (s + 1 < 9) load_b(bn, tl + (long)((s + 1) * 2 + kc) * 1024);  // the next slot's, during these MFMAs
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int p = (hc[j] + off) ^ (2 * lk);
-        v8h a[4], na[2];
-#pragma unroll
-        for (int P = 0; P < 4; P++) a[P] = hb[P * 4 * kH16WPos + p];
-        na[0] = h16_neg(a[2]);
-        na[1] = h16_neg(a[3]);
-#pragma unroll
-        for (int c = 0; c < 2; c++) h16_cmac_na(a, na, b[c], cr[j][c], ci[j][c]);
-      }
+    for (int u = 0; u < NU; u++) {
+      const int e = tid + u * kBlock;
+      const int h = e >> 5;
+      if (e < 3200)
+        *reinterpret_cast<float4*>(&tile[h * BS + h / 10 * (RS - 10 * BS) + 2 * (e & 31)]) =
+            make_float4(v[u].x * s, v[u].y * s, v[u].z * s, v[u].w * s);
     }
   }
-
-  // ---- L2P: locals of the tile's 128 boxes in chunks of 32; units (box, g):
-  // locals 32 kc + 8 g .. +7 of box b0 + box, loaded a chunk ahead
-  const zf* lr = loc + (long)rhs * ls + b0 * S;
-  float4 lv[2][4];
-  auto load_loc = [&](int kc) {
+  v4f cr[2][2], cn[2][2], ci[2][2];  // [row block][class]: real part cr - cn, imaginary part ci
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      const int u = tid + t * kBlock;
-      const int bx = u >> 2, g = u & 3;
-      const zf* lb = lr + (long)bx * S;
+  for (int j = 0; j < 2; j++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const int k = 32 * kc + 8 * g + 2 * c;
-        lv[t][c] = *reinterpret_cast<const float4*>(lb + (k < S ? k : S - 2));
-      }
+    for (int c = 0; c < 2; c++) {
+      cr[j][c] = v4f{0, 0, 0, 0};
+      cn[j][c] = v4f{0, 0, 0, 0};
+      ci[j][c] = v4f{0, 0, 0, 0};
     }
+  int base[2];  // window corner (upper left neighbour) of box 16 (rb0 + j) + li
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const unsigned c = (unsigned)(16 * (rb0 + j) + li);
+    base[j] = (int)compact2(c >> 1) * RS + (int)compact2(c) * BS;
+  }
+  // a pair of slots folded: rows first (sign sy), then both column parities
+  auto fold2 = [&](float4 pp, float4 mp, float4 pm, float4 mm, v8h (&a)[2][4], int e) {
+    // (pp, pm: columns ascending; mp, mm: descending)
+    const float ex0 = fmaf(sy, pm.x, pp.x), ey0 = fmaf(sy, pm.y, pp.y), ex1 = fmaf(sy, pm.z, pp.z),
+                ey1 = fmaf(sy, pm.w, pp.w);
+    const float fx0 = fmaf(sy, mm.z, mp.z), fy0 = fmaf(sy, mm.w, mp.w), fx1 = fmaf(sy, mm.x, mp.x),
+                fy1 = fmaf(sy, mm.y, mp.y);
+    h16_split_pair(v2f{ex0 + fx0, ex1 + fx1}, v2f{ey0 + fy0, ey1 + fy1}, a[0], e);
+    h16_split_pair(v2f{ex0 - fx0, ex1 - fx1}, v2f{ey0 - fy0, ey1 - fy1}, a[1], e);
   };
-  load_loc(0);
+  // both classes' chains interleaved: six independent accumulators
+  auto mac = [&](const v8h (&a)[2][4], const v8h (&b)[2][4], int j) {
+#define ISG_S16(ACC, P, Q)                \
+  _Pragma("unroll") for (int c = 0; c < 2; c++) ACC[j][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[c][P], b[c][Q], ACC[j][c], 0, 0, 0);
+    ISG_S16(cr, 0, 0)
+    ISG_S16(ci, 0, 2)
+    ISG_S16(cn, 2, 2)
+    ISG_S16(cr, 0, 1)
+    ISG_S16(ci, 0, 3)
+    ISG_S16(cn, 2, 3)
+    ISG_S16(cr, 1, 0)
+    ISG_S16(ci, 1, 2)
+    ISG_S16(cn, 3, 2)
+    ISG_S16(ci, 2, 0)
+    ISG_S16(ci, 2, 1)
+    ISG_S16(ci, 3, 0)
+#undef ISG_S16
+  };
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < kS16Chunks; b++) {
+    load_b(bt[(b + 1) & 1], b + 1);  // (the last one is the L2P's)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      v8h a[2][4];
+      if (b < 3) {
+        // rows 12 + 4 b + lk and 11 - 4 b - lk of the window, eight columns of the right and left neighbours
+        const zf* p = tile + base[j] + 8 * lk + (b == 0 ? RS + 32 : (b == 1 ? 2 * RS : 2 * RS + 32));
+        const zf* q = tile + base[j] + 8 * (3 - lk) + (b == 0 ? RS : (b == 1 ? 32 : 0));
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          auto at = [&](const zf* s, int o) { return *reinterpret_cast<const float4*>(s + o); };
+          fold2(at(p, 2 * BS + 2 * t), at(p, 6 - 2 * t), at(q, 2 * BS + 2 * t), at(q, 6 - 2 * t), a, 2 * t);
+        }
+      } else {
+        // the box's own columns: quarter-window rows j0, j0 + 1 (two slots' worth of lanes idle in the last chunk)
+        const int j0 = b == 3 ? 2 * lk : 8 + 2 * (lk & 1);
+        const zf* p = tile + base[j] + BS + (j0 < 4 ? RS + (4 + j0) * 8 : 2 * RS + (j0 - 4) * 8);
+        const zf* q = tile + base[j] + BS + (j0 < 4 ? RS + (3 - j0) * 8 : (11 - j0) * 8);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          auto at = [&](const zf* s, int o) { return *reinterpret_cast<const float4*>(s + o); };
+          const int up = (t >> 1) * 8, e = 2 * (t & 1);  // second row; column pair
+          fold2(at(p, up + 4 + e), at(p, up + 2 - e), at(q, 4 + e - up), at(q, 2 - e - up), a, 2 * t);
+        }
+      }
+      mac(a, bt[b & 1], j);
+    }
+  }
+  // ---- L2P: the tile's locals staged raw, rows of S + 1; orbits m = 8 lk + e
+  __syncthreads();
   int el;
   {
     float m[1] = {0.f};
-    const int n4 = 64 * S;  // 128 boxes x S locals = 64 S float4 (S even)
+    const int n4 = 32 * S;  // 64 boxes x S locals in float4 (S even)
     constexpr int U = 9;
-    const float4* lq = reinterpret_cast<const float4*>(lr);
+    const float4* lq = reinterpret_cast<const float4*>(loc + (long)rhs * ls + b0 * S);
+    const int hs = S >> 1, db = kBlock / hs, dk = kBlock - db * hs;  // box and pair of element e, stepped
+    int bx = tid / hs, kp = tid - bx * hs;
     for (int e0 = tid; e0 < n4; e0 += U * kBlock) {
       float4 t[U];
+      int at[U];
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int e = e0 + u * kBlock;
         t[u] = lq[e < n4 ? e : n4 - 1];
+        at[u] = bx * (S + 1) + 2 * kp;
+        bx += db;
+        kp += dk;
+        if (kp >= hs) {
+          kp -= hs;
+          bx++;
+        }
       }
 #pragma unroll
-      for (int u = 0; u < U; u++) m[0] = fmaxf(m[0], h16_absmax(t[u]));  // clamped repeats change no maximum
+      for (int u = 0; u < U; u++) {
+        m[0] = fmaxf(m[0], h16_absmax(t[u]));  // clamped repeats change no maximum
+        if (e0 + u * kBlock < n4) {
+          tile[at[u]] = mkc<float>(t[u].x, t[u].y);
+          tile[at[u] + 1] = mkc<float>(t[u].z, t[u].w);
+        }
+      }
     }
-    __syncthreads();  // red is read by the data scale above
-    block_max<1>(m, red);
-    el = h16_scale_exp(m[0]);
+    block_max<1>(m, red + 1);  // (its barrier also covers the staging)
+    el = h16_scale_exp(m[0]) - 2;
   }
   {
     // near accumulators carry 2^(es + et); bring them to the L2P's 2^(el + eb)
     const int n = (el + eb) - (es + et);
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < 2; j++)
 #pragma unroll
       for (int c = 0; c < 2; c++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          cr[j][c][i] = ldexpf(cr[j][c][i], n);
+          cr[j][c][i] = ldexpf(cr[j][c][i] - cn[j][c][i], n);
+          cn[j][c][i] = 0.f;
           ci[j][c][i] = ldexpf(ci[j][c][i], n);
         }
   }
   const float sl = ldexpf(1.f, el);
-  const int nlc = (S + 31) / 32;
-#pragma unroll 1
-  for (int kc = 0; kc < nlc; kc++) {
-    __syncthreads();
-    v8h b[2][4];
-    load_b(b, bas + (long)kc * 1024 + lk * 64 + 16 * mb0 + li);  // in flight during the staging
-    {
 #pragma unroll
-      for (int t = 0; t < 2; t++) {
-        const int u = tid + t * kBlock;
-        const int bx = u >> 2, g = u & 3;
-        float4 v[4];
+  for (int j = 0; j < 2; j++) {
+    const zf* t = tile + (16 * (rb0 + j) + li) * (S + 1);
+    v8h a[2][4];
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const int k = 32 * kc + 8 * g + 2 * c;  // pairs (k, k + 1) lie within S or beyond it together
-          v[c] = k < S ? lv[t][c] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        v8h ph[4];
-        h16_split4(v[0], v[1], sl, ph, 0);
-        h16_split4(v[2], v[3], sl, ph, 4);
+    for (int e = 0; e < 8; e += 2) {
+      zf g[2], h[2];
 #pragma unroll
-        for (int P = 0; P < 4; P++) hal[(P * 4 + g) * 128 + (bx ^ (2 * g))] = ph[P];
+      for (int u = 0; u < 2; u++) {
+        const int m = min(8 * lk + e + u, S >> 2);  // (past S / 4 the table is zero)
+        const zf v0 = t[m], v1 = t[(S >> 1) - m], v2 = t[m ? S - m : 0], v3 = t[(S >> 1) + m];
+        g[u] = mkc<float>(fmaf(sy, v2.x, v0.x) * sl, fmaf(sy, v2.y, v0.y) * sl);
+        h[u] = mkc<float>(fmaf(sy, v3.x, v1.x) * sl, fmaf(sy, v3.y, v1.y) * sl);
       }
+      h16_split_pair(v2f{g[0].x + h[0].x, g[1].x + h[1].x}, v2f{g[0].y + h[0].y, g[1].y + h[1].y}, a[0], e);
+      h16_split_pair(v2f{g[0].x - h[0].x, g[1].x - h[1].x}, v2f{g[0].y - h[0].y, g[1].y - h[1].y}, a[1], e);
     }
-    __syncthreads();
-    if (kc + 1 < nlc) load_loc(kc + 1);
-    const v8h* hb = hal + lk * 128;  // + P * 512 + box
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      v8h a[4], na[2];
-#pragma unroll
-      for (int P = 0; P < 4; P++) a[P] = hb[P * 512 + ((16 * (4 * rbh + j) + li) ^ (2 * lk))];
-      na[0] = h16_neg(a[2]);
-      na[1] = h16_neg(a[3]);
-#pragma unroll
-      for (int c = 0; c < 2; c++) h16_cmac_na(a, na, b[c], cr[j][c], ci[j][c]);
-    }
+    mac(a, bt[kS16Chunks & 1], j);
   }
-
-  // ---- output in two halves of 64 boxes through LDS; D[box][m]: box
-  // 16 (4 rbh + j) + 4 lk + i (register i), pixel m = 16 (mb0 + c) + li
-  zf* tile = reinterpret_cast<zf*>(smem_raw);
-  const int n = -(el + eb);
-  zd acc[2] = {mkc<double>(0, 0), mkc<double>(0, 0)};
-  const bool herm = post.herm != 0;
-#pragma unroll 1
-  for (int hh = 0; hh < 2; hh++) {
-    __syncthreads();
-    if (rbh == hh) {
+  // ---- back to pixels through LDS (as k_near_mfma)
+  __syncthreads();
+  {
+    const int n = -(el + eb), p = li & 3, q = li >> 2;
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+    for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int c = 0; c < 2; c++)
+      for (int c = 0; c < 2; c++) {
+        const int px = (oy ? 3 - q : 4 + q) * 8 + (c ? 3 - p : 4 + p);
 #pragma unroll
-          for (int i = 0; i < 4; i++)
-            tile[(16 * j + 4 * lk + i) * 64 + 16 * (mb0 + c) + li] =
-                mkc<float>(ldexpf(cr[j][c][i], n), ldexpf(ci[j][c][i], n));
-    }
-    __syncthreads();
-    const long o = (long)rhs * rs + (b0 + 64 * hh) * 64;
-    if constexpr (POST == 0) {
-#pragma unroll 4
-      for (int e = tid; e < 64 * 64; e += kBlock) r[o + e] = tile[e];
-    } else {
-      const zd* gr = post.g + (long)rhs * post.gs + (b0 + 64 * hh) * 64;
-      struct In {
-        zf x, aux;  // aux: r~ (mode 1)
-        zd g;
-      };
-      stage<2, In>(
-          64 * 64,
-          [&](int e) {
-            In v;
-            v.x = post.x[o + e];
-            if (POST == 1) v.aux = post.rt[o + e];
-            if (herm) v.g = gr[e];  // the forward post step does not use g
-            return v;
-          },
-          [&](int e, In v) {
-            const zf gt = tile[e];
-            const zd gy = mkc<double>((double)gt.x, (double)gt.y);
-            const zd xv = ccast<double>(v.x);
-            const zd px = herm ? csub(xv, cconj(cmul(v.g, gy))) : csub(xv, gy);
-            const zd res = stv(r, o + e, px);
-            if (POST == 1) {
-              const zd a = ccast<double>(v.aux);
-              acc[0].x += a.x * res.x + a.y * res.y;
-              acc[0].y += a.x * res.y - a.y * res.x;
-            } else {
-              acc[0].x += res.x * xv.x + res.y * xv.y;
-              acc[0].y += res.x * xv.y - res.y * xv.x;
-              acc[1].x += res.x * res.x + res.y * res.y;
-            }
-          });
-    }
+        for (int i = 0; i < 4; i++)
+          tile[(16 * (rb0 + j) + 4 * lk + i) * 64 + px] = mkc<float>(ldexpf(cr[j][c][i] - cn[j][c][i], n), ldexpf(ci[j][c][i], n));
+      }
   }
-  if constexpr (POST != 0) block_store<2>(acc, post.part + (long)rhs * kSlots * gridDim.x, gridDim.x, blockIdx.x);
+  __syncthreads();
+  sym_unfold<float, 64>(tile);
+  __syncthreads();
+  near_epilogue<float, float, 64, POST>(tile, r, rs, b0, rhs, post);
 }
 
 // P2M of the FP32 operator on split FP16: agm[box][s] = sum_n coeffT[n][s]

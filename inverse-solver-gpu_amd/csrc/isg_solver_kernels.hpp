@@ -6,7 +6,7 @@
 // fused pass that also produces the dot products the next scalar needs:
 //   k_bi_init   r = b - A x, r~ = r, partial <b,b>, <r,r>
 //   k_bi_pupd   p = r + beta (p - omega v), y = prep(p)
-//   (near)      v = post(p, G y), partial <r~,v>    -- epilogue of k_near_mfma
+//   (near)      v = post(p, G y), partial <r~,v>    -- epilogue of the near-field kernel
 //   k_bi_supd   s = r - alpha v, y = prep(s)
 //   (near)      t = post(s, G y), partial <t,s>, <t,t>    -- likewise
 //   k_bi_xrupd  x += alpha p; x += omega s; r = s - omega t; partial <r,r>, <r~,r>
