@@ -661,8 +661,14 @@ void Engine::launch_m2m(int i, int nrhs, const int* act, int force) {
   } else if (kind == 1) {
     int nch = (Sp + sh.kch - 1) / sh.kch;
     dim3 grid(np / sh.g * nch, nrhs);
-    k_m2m_chunk<T><<<grid, blk, sh.lds_chunk, stream_>>>(child, cs, par, ps, d.interpT[i], interp0_[i], d.shiftM[i],
-                                                         Sp, Sc, sh.g, sh.kch, nch, nt, act);
+    auto go = [&](auto ntc) {
+      k_m2m_chunk<T, decltype(ntc)::value><<<grid, blk, sh.lds_chunk, stream_>>>(
+          child, cs, par, ps, d.interpT[i], interp0_[i], d.shiftM[i], Sp, Sc, sh.g, sh.kch, nch, nt, act);
+    };
+    if (nt == 30)
+      go(std::integral_constant<int, 30>());
+    else
+      go(std::integral_constant<int, 0>());
   } else {
     k_m2m<T><<<dim3(nblocks((long)np * Sp), nrhs), blk, 0, stream_>>>(child, cs, par, ps, d.interpT[i], interp0_[i],
                                                                        d.shiftM[i], Sp, Sc, np, nt, act);
@@ -700,8 +706,14 @@ void Engine::launch_l2l(int i, bool accumulate, int nrhs, const int* act, int fo
   } else if (kind == 1) {
     int nch = (Sc + sh.kch - 1) / sh.kch;
     dim3 grid(np * nch, nrhs);
-    k_l2l_chunk<T><<<grid, blk, sh.lds_chunk, stream_>>>(par, ps, child, cs, d.anterpT[i + 1], anterp0_[i + 1],
-                                                         d.shiftL[i], Sp, Sc, sh.kch, nch, nt, acc, act);
+    auto go = [&](auto ntc) {
+      k_l2l_chunk<T, decltype(ntc)::value><<<grid, blk, sh.lds_chunk, stream_>>>(
+          par, ps, child, cs, d.anterpT[i + 1], anterp0_[i + 1], d.shiftL[i], Sp, Sc, sh.kch, nch, nt, acc, act);
+    };
+    if (nt == 60)
+      go(std::integral_constant<int, 60>());
+    else
+      go(std::integral_constant<int, 0>());
   } else {
     k_l2l<T><<<dim3(nblocks((long)4 * np * Sc), nrhs), blk, 0, stream_>>>(par, ps, child, cs, d.anterpT[i + 1],
                                                                            anterp0_[i + 1], d.shiftL[i], Sp, Sc, np,
@@ -712,7 +724,7 @@ void Engine::launch_l2l(int i, bool accumulate, int nrhs, const int* act, int fo
 // M2L variants: TS x TS target boxes and KC samples per workgroup; 0-5
 // k_m2l_tile, 6-8 k_m2l_reg (operators in registers), 9 k_m2l_par (one
 // thread per parent and sample, sources in registers)
-constexpr int kM2LVariants = 10;
+constexpr int kM2LVariants = 10, kM2LPar = 9;
 constexpr int kM2LShape[kM2LVariants][2] = {{4, 8}, {8, 8}, {8, 16}, {16, 8}, {8, 32}, {16, 16},
                                             {8, 16}, {8, 32}, {8, 8}, {8, 16}};
 
@@ -724,14 +736,45 @@ bool Engine::m2l_ok(int v, int i) const {
   return (1 << i) >= TS && lds <= kLdsLimit;
 }
 
-// translations of level i.  Built-in rule: 8x8 tiles of 8 samples, 4x4 when
-// 8x8 tiles would leave fewer than 1024 workgroups.
+// Translations of levels lo..hi.  Levels without a tuned variant (or with the
+// per-parent one) go into one k_m2l_par launch, the finest first: its
+// workgroups fill the chip and those of the small levels run beside them,
+// instead of one launch of a few workgroups each (a launch costs the host
+// ~3.5 us, the smallest kernels 5).
 template <typename T>
-void Engine::launch_m2l(int i, int nrhs, const int* act, int force) {
+void Engine::launch_m2l(int lo, int hi, int nrhs, const int* act, int force) {
+  M2LSet<T> set;
+  set.n = 0;
+  int blocks = 0;
+  DevOp<T>& d = ops<T>();
+  for (int i = hi; i >= lo; i--) {
+    const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).m2l[i];
+    const int v = force >= 0 && m2l_ok<T>(force, i) ? force : tuned;
+    if (m2l_ok<T>(v, i) && v != kM2LPar) {
+      launch_m2l_variant<T>(i, nrhs, act, v);
+      continue;
+    }
+    if (set.n == kM2LMaxLevels) {
+      k_m2l_par<T><<<dim3(blocks, nrhs), dim3(kBlock), 0, stream_>>>(set, act);
+      set.n = blocks = 0;
+    }
+    const int S = P_.nsamp[i], nb = 1 << i;
+    M2LLevel<T>& e = set.lv[set.n++];
+    e.m = d.agm + lvl_off_[i];
+    e.l = d.agl + lvl_off_[i];
+    e.trans = d.trans[i];
+    e.st = (long)lvl_size_[i];
+    e.first = blocks;
+    e.lev = i;
+    e.S = S;
+    blocks += std::max(1, nb * nb / (kParTS * kParTS)) * ((S + kParKC - 1) / kParKC);
+  }
+  if (set.n > 0) k_m2l_par<T><<<dim3(blocks, nrhs), dim3(kBlock), 0, stream_>>>(set, act);
+}
+
+template <typename T>
+void Engine::launch_m2l_variant(int i, int nrhs, const int* act, int v) {
   const int S = P_.nsamp[i], nb = 1 << i;
-  int v = force;
-  if (!m2l_ok<T>(v, i)) v = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).m2l[i];
-  if (!m2l_ok<T>(v, i)) v = (nb >= 8 && (long)(nb * nb / 64) * ((S + 7) / 8) * nrhs >= 1024) ? 1 : 0;
   const int TS = kM2LShape[v][0], KC = kM2LShape[v][1];
   const int nchunk = (S + KC - 1) / KC;
   const int ntile = nb * nb / (TS * TS);
@@ -747,7 +790,6 @@ void Engine::launch_m2l(int i, int nrhs, const int* act, int force) {
     case 3: k_m2l_tile<T, 16, 8><<<grid, blk, 0, stream_>>>(m, l, st, d.trans[i], i, S, act); break;
     case 6: k_m2l_reg<T, 16><<<grid, blk, 0, stream_>>>(m, l, st, d.trans[i], i, S, act); break;
     case 8: k_m2l_reg<T, 8><<<grid, blk, 0, stream_>>>(m, l, st, d.trans[i], i, S, act); break;
-    case 9: k_m2l_par<T><<<grid, blk, 0, stream_>>>(m, l, st, d.trans[i], i, S, act); break;
     case 7:
       if constexpr (sizeof(T) == 4) k_m2l_reg<T, 32><<<grid, blk, 0, stream_>>>(m, l, st, d.trans[i], i, S, act);
       break;
@@ -905,7 +947,7 @@ void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, con
   const bool fuse = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).leaf == 1 && leaf_fuse_ok<T>();
   const int mtop = fuse ? Lf - 1 : Lf, ltop = fuse ? L - 3 : L - 2;
   prof_begin(kt);
-  for (int i = 2; i <= mtop; i++) launch_m2l<T>(i, nrhs, act);
+  launch_m2l<T>(2, mtop, nrhs, act);
   prof_end(kt);
   prof_begin(KT_INTERP, false);  // timed with the M2M launch set of this product
   for (int i = 2; i <= ltop; i++) launch_l2l<T>(i, true, nrhs, act);
@@ -1447,7 +1489,15 @@ void Engine::autotune_prec(int nrhs, int reps) {
   tu.p2m_nb = c < 0 ? -1 : widths[c];
   for (int i = 2; i <= Lf; i++)
     tu.m2l[i] = pick(
-        kM2LVariants, [&](int v) { return m2l_ok<T>(v, i); }, [&](int v) { launch_m2l<T>(i, nrhs, nullptr, v); });
+        kM2LVariants, [&](int v) { return m2l_ok<T>(v, i); }, [&](int v) { launch_m2l<T>(i, i, nrhs, nullptr, v); });
+  // the per-level choices against every level in one per-parent launch
+  {
+    const std::vector<int> chosen = tu.m2l;
+    const float t_sep = timed([&] { launch_m2l<T>(2, Lf, nrhs, nullptr); });
+    std::fill(tu.m2l.begin(), tu.m2l.end(), -1);
+    const float t_one = timed([&] { launch_m2l<T>(2, Lf, nrhs, nullptr); });
+    if (t_sep < t_one) tu.m2l = chosen;
+  }
   const std::vector<InterpShape>& sm = sizeof(T) == 4 ? m2m32_ : m2m64_;
   const std::vector<InterpShape>& sl = sizeof(T) == 4 ? l2l32_ : l2l64_;
   for (int i = 0; i + 1 < L; i++) {
@@ -1466,7 +1516,7 @@ void Engine::autotune_prec(int nrhs, int reps) {
           if (f == 1) {
             launch_m2l_leaf<T>(nrhs, nullptr);
           } else {
-            launch_m2l<T>(Lf, nrhs, nullptr, vm);
+            launch_m2l<T>(Lf, Lf, nrhs, nullptr, vm);
             launch_l2l<T>(L - 2, true, nrhs, nullptr, kl);
           }
         });

@@ -210,7 +210,9 @@ class Engine {
   template <typename T>
   void launch_l2l(int i, bool accumulate, int nrhs, const int* act, int force = -1);
   template <typename T>
-  void launch_m2l(int i, int nrhs, const int* act, int force = -1);
+  void launch_m2l(int lo, int hi, int nrhs, const int* act, int force = -1);
+  template <typename T>
+  void launch_m2l_variant(int i, int nrhs, const int* act, int v);
   template <typename T>
   void launch_m2l_leaf(int nrhs, const int* act);
   template <typename T>

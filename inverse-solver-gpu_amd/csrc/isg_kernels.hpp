@@ -293,8 +293,35 @@ __device__ __forceinline__ void near_epilogue(const cplx<T>* tile, cplx<TI>* __r
 // first[k0]) mod Ssrc.  All four windows (children, or shifted parent copies)
 // go to LDS once; each thread then forms one target from LDS.
 
+// The upper levels have little work (16 parents of 1036 samples at 1024^2) and
+// these kernels were bound by the latency of their serial tap loop, each tap
+// waiting for its weight from L2: the weights, shifts and first-tap indices of a
+// thread are now loaded into registers before the staging (NT taps, compiled in;
+// 0: any count, loaded tap by tap), and the staging steps its indices instead of
+// dividing.  Per launch at 512^2 x 15 right-hand sides (FP32): M2M 14.5 -> 8.5 us,
+// L2L 19.6 -> 17.4 us.
+
+// Window staging: the calling wave loads elements j0, j0 + 1, .. of n (mod K),
+// lane by lane, all loads (up to 4 x 64) issued before the first store.
+template <typename Ld, typename St>
+__device__ __forceinline__ void stage_window(int n, int j0, int K, Ld ld, St st) {
+  const int lane = threadIdx.x & 63;
+  for (int t0 = lane; t0 < n; t0 += 256) {
+    decltype(ld(0)) v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      int j = j0 + min(t0 + 64 * u, n - 1);
+      while (j >= K) j -= K;
+      v[u] = ld(j);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (t0 + 64 * u < n) st(t0 + 64 * u, v[u]);
+  }
+}
+
 // M2M: parent[p][k] = sum_c shiftM[c][k] sum_t w[t][k] child[4p+c][first[k]+t]
-template <typename T>
+template <typename T, int NT>
 __global__ void __launch_bounds__(kBlock) k_m2m_chunk(const cplx<T>* __restrict__ child, long cs,
                                                       cplx<T>* __restrict__ par, long ps, const T* __restrict__ wT,
                                                       const int* __restrict__ i0, const cplx<T>* __restrict__ shift,
@@ -311,38 +338,51 @@ __global__ void __launch_bounds__(kBlock) k_m2m_chunk(const cplx<T>* __restrict_
   int W = i0[k0 + kn - 1] - base;
   if (W < 0) W += Sc;
   W += ntap;
+  const int o = min((int)threadIdx.x, G * kn - 1);
+  const int g = o / kn, k = k0 + (o - g * kn);
+  const int ik = i0[k];
+  T w[NT ? NT : 1];
+  cplx<T> sh[4];
+  if constexpr (NT > 0) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) w[t] = wT[t * Sp + k];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; c++) sh[c] = shift[c * Sp + k];
   const cplx<T>* cr = child + rhs * cs + 4 * p0 * Sc;
-  stage<sizeof(T) == 4 ? 8 : 4, cplx<T>>(
-      4 * G * W,
-      [&](int e) {
-        int v = e / W, t = e - v * W;  // v = 4 g + c (consecutive children)
-        int j = base + t;
-        while (j >= Sc) j -= Sc;
-        return cr[(long)v * Sc + j];
-      },
-      [&](int e, cplx<T> v) { lds[e] = v; });
+  for (int v = threadIdx.x >> 6; v < 4 * G; v += kBlock / 64)  // v = 4 g + c (consecutive children)
+    stage_window(
+        W, base, Sc, [&](int j) { return cr[(long)v * Sc + j]; }, [&](int t, cplx<T> x) { lds[v * W + t] = x; });
   __syncthreads();
-  int o = threadIdx.x;
-  if (o >= G * kn) return;
-  int g = o / kn, k = k0 + (o - g * kn);
-  int d = i0[k] - base;
+  if ((int)threadIdx.x >= G * kn) return;
+  int d = ik - base;
   if (d < 0) d += Sc;
   cplx<T> acc = mkc<T>(0, 0);
+#pragma unroll
   for (int c = 0; c < 4; c++) {
     const cplx<T>* src = lds + (4 * g + c) * W + d;
     cplx<T> red = mkc<T>(0, 0);
-    for (int t = 0; t < ntap; t++) {
-      T w = wT[t * Sp + k];
-      red.x += w * src[t].x;
-      red.y += w * src[t].y;
+    if constexpr (NT > 0) {
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        red.x += w[t] * src[t].x;
+        red.y += w[t] * src[t].y;
+      }
+    } else {
+      for (int t = 0; t < ntap; t++) {
+        const T wt = wT[t * Sp + k];
+        red.x += wt * src[t].x;
+        red.y += wt * src[t].y;
+      }
     }
-    acc = cfma(red, shift[c * Sp + k], acc);
+    acc = cfma(red, sh[c], acc);
   }
   par[rhs * ps + (p0 + g) * Sp + k] = acc;
 }
 
-// L2L: child[4p+c][k] (+)= sum_t a[t][k] (shiftL[c] o par[p])[first[k]+t]
-template <typename T>
+// L2L: child[4p+c][k] (+)= sum_t a[t][k] (shiftL[c] o par[p])[first[k]+t];
+// wave c forms child c's window and its kch <= 64 samples
+template <typename T, int NT>
 __global__ void __launch_bounds__(kBlock) k_l2l_chunk(const cplx<T>* __restrict__ par, long ps,
                                                       cplx<T>* __restrict__ child, long cs, const T* __restrict__ aT,
                                                       const int* __restrict__ j0s, const cplx<T>* __restrict__ shift,
@@ -358,31 +398,42 @@ __global__ void __launch_bounds__(kBlock) k_l2l_chunk(const cplx<T>* __restrict_
   int W = j0s[k0 + kn - 1] - base;
   if (W < 0) W += Sp;
   W += ntap;
-  const cplx<T>* pv = par + rhs * ps + (long)p * Sp;
-  stage<4, CPair<T>>(
-      4 * W,
-      [&](int e) {
-        int c = e / W, t = e - c * W;
-        int j = base + t;
-        while (j >= Sp) j -= Sp;
-        return CPair<T>{shift[c * Sp + j], pv[j]};
-      },
-      [&](int e, CPair<T> v) { lds[e] = cmul(v.a, v.b); });
-  __syncthreads();
-  for (int o = threadIdx.x; o < 4 * kn; o += kBlock) {
-    int c = o / kn, k = k0 + (o - c * kn);
-    int d = j0s[k] - base;
-    if (d < 0) d += Sp;
-    const cplx<T>* src = lds + c * W + d;
-    cplx<T> red = mkc<T>(0, 0);
-    for (int t = 0; t < ntap; t++) {
-      T w = aT[t * Sc + k];
-      red.x += w * src[t].x;
-      red.y += w * src[t].y;
-    }
-    cplx<T>* dst = child + rhs * cs + (4L * p + c) * Sc + k;
-    *dst = accumulate ? cadd(*dst, red) : red;
+  const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;
+  const int k = k0 + min(lane, kn - 1);
+  const int jk = j0s[k];
+  T w[NT ? NT : 1];
+  if constexpr (NT > 0) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) w[t] = aT[t * Sc + k];
   }
+  cplx<T>* dst = child + rhs * cs + (4L * p + c) * Sc + k;
+  cplx<T> old = mkc<T>(0, 0);
+  if (accumulate) old = *dst;
+  const cplx<T>* pv = par + rhs * ps + (long)p * Sp;
+  cplx<T>* win = lds + c * W;
+  stage_window(
+      W, base, Sp, [&](int j) { return CPair<T>{shift[c * Sp + j], pv[j]}; },
+      [&](int t, CPair<T> x) { win[t] = cmul(x.a, x.b); });
+  __syncthreads();
+  if (lane >= kn) return;
+  int d = jk - base;
+  if (d < 0) d += Sp;
+  const cplx<T>* src = win + d;
+  cplx<T> red = mkc<T>(0, 0);
+  if constexpr (NT > 0) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      red.x += w[t] * src[t].x;
+      red.y += w[t] * src[t].y;
+    }
+  } else {
+    for (int t = 0; t < ntap; t++) {
+      const T wt = aT[t * Sc + k];
+      red.x += wt * src[t].x;
+      red.y += wt * src[t].y;
+    }
+  }
+  *dst = accumulate ? cadd(old, red) : red;
 }
 
 // Interpolation (M2M) and anterpolation (L2L) on the matrix cores, for the
@@ -732,9 +783,8 @@ constexpr int kParTS = 8, kParSB = kParTS + 4, kParKC = 16;
 struct ParBlock {
   int chunk, k0, X0, Y0;
   unsigned m0;
-  __device__ __forceinline__ ParBlock(int S) {
+  __device__ __forceinline__ ParBlock(int S, int lb) {
     const int nchunk = (S + kParKC - 1) / kParKC;
-    const int lb = xcd_block();
     const int tile = lb / nchunk;
     chunk = lb - tile * nchunk;
     k0 = chunk * kParKC;
@@ -797,21 +847,46 @@ __device__ __forceinline__ void par_translate_stream(const cplx<T> (*src)[kParKC
     }
 }
 
+// One level of a merged M2L launch: its multipoles, locals, operators and
+// first workgroup (per right-hand side).
+template <typename T>
+struct M2LLevel {
+  const cplx<T>* m;
+  cplx<T>* l;
+  const cplx<T>* trans;
+  long st;
+  int first, lev, S;
+};
+constexpr int kM2LMaxLevels = 10;
+template <typename T>
+struct M2LSet {
+  M2LLevel<T> lv[kM2LMaxLevels];
+  int n;
+};
+
+// M2L of several levels in one launch (they are independent once the
+// multipoles are there): workgroups first[q] .. of the grid belong to set
+// entry q.  A level of 4 x 4 boxes fills a quarter of its one tile.
 // (at least 2 waves per SIMD: the FP64 instantiation otherwise takes 256+ registers
 // and runs one wave per SIMD; measured 2.00 -> 1.52 ms per FP64 launch set)
 template <typename T>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) k_m2l_par(const cplx<T>* __restrict__ agm, cplx<T>* __restrict__ agl,
-                                                    long st, const cplx<T>* __restrict__ trans, int lev, int S,
-                                                    const int* __restrict__ act) {
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+k_m2l_par(M2LSet<T> set, const int* __restrict__ act) {
   __shared__ cplx<T> src[kParSB * kParSB][kParKC];
   __shared__ cplx<T> tr[49][kParKC];
   const int rhs = blockIdx.y;
   if (rhs_off(act, rhs)) return;
-  const ParBlock B(S);
-  m2l_stage<T, kParTS, kParKC>(src, tr, agm + rhs * st, trans, B.X0, B.Y0, B.k0, 1 << lev, S);
+  const int lb = xcd_block();
+  M2LLevel<T> L = set.lv[0];
+  for (int q = 1; q < set.n; q++)
+    if (lb >= set.lv[q].first) L = set.lv[q];
+  const int S = L.S, nb = 1 << L.lev;
+  const ParBlock B(S, lb - L.first);
+  m2l_stage<T, kParTS, kParKC>(src, tr, L.m + rhs * L.st, L.trans, B.X0, B.Y0, B.k0, nb, S);
   __syncthreads();
   const int kk = threadIdx.x % kParKC, pp = threadIdx.x / kParKC;
   const int lx0 = 2 * (pp & 3), ly0 = 2 * (pp >> 2);  // first child of the parent, tile coordinates
+  if (lx0 >= nb || ly0 >= nb || B.k0 + kk >= S) return;
   cplx<T> acc[4];
   if constexpr (sizeof(T) == 8) {
     par_translate_stream<T>(src, tr, lx0, ly0, kk, acc);
@@ -820,11 +895,9 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
     par_load<T>(src, lx0, ly0, kk, sv);
     par_translate<T>(tr, kk, sv, acc);
   }
-  if (B.k0 + kk < S) {
-    cplx<T>* out = agl + rhs * st + (long)(B.m0 + 4 * morton2((unsigned)(pp & 3), (unsigned)(pp >> 2))) * S;
+  cplx<T>* out = L.l + rhs * L.st + (long)(B.m0 + 4 * morton2((unsigned)(pp & 3), (unsigned)(pp >> 2))) * S;
 #pragma unroll
-    for (int c = 0; c < 4; c++) out[(long)c * S + B.k0 + kk] = acc[c];
-  }
+  for (int c = 0; c < 4; c++) out[(long)c * S + B.k0 + kk] = acc[c];
 }
 
 // Leaf M2L fused with the last L2L (parent level lev-1 -> leaf level lev):
@@ -854,7 +927,7 @@ __global__ void __launch_bounds__(kBlock) k_m2l_leaf(const cplx<T>* __restrict__
   cplx<T>* sw = pw + max(16 * KB, 64 * kParKC);         // [4 children][KB]
   const int rhs = blockIdx.y;
   if (rhs_off(act, rhs)) return;
-  const ParBlock B(S);
+  const ParBlock B(S, xcd_block());
   // the band rows of the window (the interpolation's A operand; no LDS
   // needed), issued before the staging so their latency overlaps it
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
