@@ -568,9 +568,7 @@ int isg_warmnet_set_params(isg_warmnet* n, const float* in) {
 int isg_warmnet_get_grads(isg_warmnet* n, float* out) {
   if (net_check(n) != ISG_OK) return ISG_E_STATE;
   if (!out) return net_fail(n, ISG_E_ARG, "null pointer");
-  std::vector<float> g;
-  n->net->get_grads(g);
-  std::memcpy(out, g.data(), g.size() * sizeof(float));
+  n->net->get_grads(out);
   return net_check(n);
 }
 

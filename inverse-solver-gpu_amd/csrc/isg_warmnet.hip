@@ -177,54 +177,86 @@ __global__ void __launch_bounds__(kNB) __attribute__((amdgpu_waves_per_eu(2))) k
 // lane l supplies channel l % 16 and the 8 positions of tile row
 // 4 c + l / 16), B = the input shifted by the tap (columns ci, the same
 // positions); wave w owns taps w, w + 4, w + 8.  The tile's dY and input halo
-// are staged in LDS as BF16, channel-major.  Fixed order over the chunk's
-// tiles: deterministic.
+// are staged in LDS as BF16, channel-major (rows of 72 and HS + 2 so that the
+// 16 channels of a position fall in different banks).  Fixed order over the
+// chunk's tiles: deterministic.
+// A workgroup runs a few tiles in a row, each a chain of loads, staging and few
+// MFMAs, so latency bounds it: every thread loads whole float4s (4 channels of a
+// position), the next tile's while the current one is multiplied, and the bias
+// sums are spread over all threads (16 of them had summed 64 positions serially).
+// 16 x 128^2 images: 7 launches of 3x3 layers 175 -> 130 us.
 template <int KS>
 __global__ void __launch_bounds__(kNB) k_wgrad(const float* __restrict__ dY, const float* __restrict__ M,
                                                const float* __restrict__ X, const float* __restrict__ U, int cin,
                                                int cout, int H, int W, int batch, int per_chunk,
                                                float* __restrict__ part, float* __restrict__ bpart) {
   constexpr int R = KS / 2, HW = 8 + KS - 1, HS = HW * HW, NT = KS * KS, TPW = (NT + 3) / 4;
-  __shared__ __attribute__((aligned(16))) uint16_t dsm[16][64];  // dY[co][p], BF16
-  __shared__ uint16_t xsm[16][HS];                              // In[ci][halo position], BF16
+  constexpr int DP = 72, XP = HS + 2;
+  constexpr int NX = (HS * 4 + kNB - 1) / kNB;  // float4 groups of the input halo per thread
+  __shared__ __attribute__((aligned(16))) uint16_t dsm[16][DP];  // dY[co][p], BF16
+  __shared__ uint16_t xsm[16][XP];                              // In[ci][halo position], BF16
+  __shared__ float bsm[kNB];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, lk = lane >> 4;
   const int ncit = cin >> 4;
   const int co0 = (blockIdx.x / ncit) * 16, ci0 = (blockIdx.x % ncit) * 16;
   const int chunk = blockIdx.y;
   const int tiles_x = (W + 7) >> 3, tiles = ((H + 7) >> 3) * tiles_x;
   const long total = (long)tiles * batch;
+  const long t0 = (long)chunk * per_chunk, t1 = min(total, t0 + per_chunk);
   v4f acc[TPW];
 #pragma unroll
   for (int q = 0; q < TPW; q++) acc[q] = v4f{0, 0, 0, 0};
-  float bacc = 0.f;
-  for (long tt = (long)chunk * per_chunk; tt < total && tt < (long)(chunk + 1) * per_chunk; tt++) {
+  const int c4 = 4 * (tid & 3);  // this thread's channels c4 .. c4 + 3
+  float bacc[4] = {0.f, 0.f, 0.f, 0.f};
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  struct Regs {
+    float4 d, m, x[NX], u[NX];
+  } v;
+  auto load = [&](long tt) {
     const int n = (int)(tt / tiles), tl = (int)(tt % tiles);
     const int ty0 = (tl / tiles_x) * 8, tx0 = (tl % tiles_x) * 8;
     const long img = (long)n * H * W;
-    for (int e = tid; e < 64 * 16; e += kNB) {
-      const int p = e >> 4, c = e & 15;
-      const int gy = ty0 + (p >> 3), gx = tx0 + (p & 7);
-      float v = 0.f;
-      if (gy < H && gx < W) {
-        const long pix = img + (long)gy * W + gx;
-        v = dY[pix * cout + co0 + c];
-        if (M && !(M[pix * cout + co0 + c] > 0.f)) v = 0.f;
-      }
-      dsm[c][p] = f2bf(v);
+    {
+      const int p = tid >> 2, gy = ty0 + (p >> 3), gx = tx0 + (p & 7);
+      const bool in = gy < H && gx < W;
+      const long at = (in ? img + (long)gy * W + gx : 0) * cout + co0 + c4;
+      v.d = in ? *reinterpret_cast<const float4*>(dY + at) : zero;
+      if (M) v.m = *reinterpret_cast<const float4*>(M + at);
     }
-    for (int e = tid; e < HS * 16; e += kNB) {
-      const int hp = e >> 4, c = e & 15;
+#pragma unroll
+    for (int q = 0; q < NX; q++) {
+      const int hp = (tid >> 2) + q * (kNB / 4);
       const int gy = ty0 + hp / HW - R, gx = tx0 + hp % HW - R;
-      float v = 0.f;
-      if (gy >= 0 && gy < H && gx >= 0 && gx < W) {
-        v = X[(img + (long)gy * W + gx) * cin + ci0 + c];
-        if (U) v += U[((long)n * (H >> 1) * (W >> 1) + (long)(gy >> 1) * (W >> 1) + (gx >> 1)) * cin + ci0 + c];
+      const bool in = hp < HS && gy >= 0 && gy < H && gx >= 0 && gx < W;
+      v.x[q] = in ? *reinterpret_cast<const float4*>(X + (img + (long)gy * W + gx) * cin + ci0 + c4) : zero;
+      if (U)
+        v.u[q] = in ? *reinterpret_cast<const float4*>(
+                          U + ((long)n * (H >> 1) * (W >> 1) + (long)(gy >> 1) * (W >> 1) + (gx >> 1)) * cin + ci0 + c4)
+                    : zero;
+    }
+  };
+  if (t0 < t1) load(t0);
+  for (long tt = t0; tt < t1; tt++) {
+    {
+      const int p = tid >> 2;
+      const float d[4] = {v.d.x, v.d.y, v.d.z, v.d.w}, m[4] = {v.m.x, v.m.y, v.m.z, v.m.w};
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const uint16_t b = f2bf((M && !(m[c] > 0.f)) ? 0.f : d[c]);
+        dsm[c4 + c][p] = b;
+        bacc[c] += bf2f(b);
       }
-      xsm[c][hp] = f2bf(v);
+#pragma unroll
+      for (int q = 0; q < NX; q++) {
+        const int hp = (tid >> 2) + q * (kNB / 4);
+        const float x[4] = {v.x[q].x, v.x[q].y, v.x[q].z, v.x[q].w}, u[4] = {v.u[q].x, v.u[q].y, v.u[q].z, v.u[q].w};
+        if (hp < HS)
+#pragma unroll
+          for (int c = 0; c < 4; c++) xsm[c4 + c][hp] = f2bf(U ? x[c] + u[c] : x[c]);
+      }
     }
     __syncthreads();
-    if (tid < 16)
-      for (int p = 0; p < 64; p++) bacc += bf2f(dsm[tid][p]);
+    if (tt + 1 < t1) load(tt + 1);  // in flight during the products
 #pragma unroll
     for (int q = 0; q < TPW; q++) {
       const int t = w + 4 * q;
@@ -254,16 +286,55 @@ __global__ void __launch_bounds__(kNB) k_wgrad(const float* __restrict__ dY, con
       for (int i = 0; i < 4; i++) part[base + ((long)t * cout + co0 + 4 * lk + i) * cin + ci0 + li] = acc[q][i];
     }
   }
-  if (ci0 == 0 && tid < 16) bpart[(long)chunk * cout + co0 + tid] = bacc;
+  if (ci0 == 0) {
+    // bias: each thread's four channels, then the 64 positions in a fixed order
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      __syncthreads();
+      bsm[tid] = bacc[c];
+      __syncthreads();
+      if (tid < 4) {
+        float s = 0.f;
+        for (int p = 0; p < 64; p++) s += bsm[4 * p + tid];
+        bpart[(long)chunk * cout + co0 + 4 * tid + c] = s;
+      }
+    }
+  }
 }
 
-// out[i] = sum_c part[c][i], fixed order (deterministic)
-__global__ void k_chunk_sum(const float* __restrict__ part, long len, int nchunk, float* __restrict__ out) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += (long)gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int c = 0; c < nchunk; c++) s += part[(long)c * len + i];
-    out[i] = s;
+// gw[i] = sum_c part[c][i] and gb[i] = sum_c bpart[c][i], fixed order
+// (deterministic).  GRP threads share an output, each summing every GRP-th chunk
+// with 8 loads in flight, and their sums are added in order: with up to 512
+// chunks one thread per output was a serial chain of as many loads (650 us of a
+// 1.64 ms training step on 16 x 128^2 images).
+template <int GRP>
+__global__ void __launch_bounds__(kNB) k_chunk_sum(const float* __restrict__ part, long len,
+                                                   const float* __restrict__ bpart, int blen, int nchunk,
+                                                   float* __restrict__ gw, float* __restrict__ gb) {
+  constexpr int OUT = kNB / GRP;
+  __shared__ float sh[GRP][OUT];
+  const long nbw = (len + OUT - 1) / OUT;
+  const bool bias = blockIdx.x >= nbw;
+  const float* src = bias ? bpart : part;
+  const long n = bias ? blen : len;
+  const int o = threadIdx.x % OUT, g = threadIdx.x / OUT;
+  const long i = (bias ? blockIdx.x - nbw : (long)blockIdx.x) * OUT + o;
+  float s = 0.f;
+  if (i < n)
+    for (int c0 = g; c0 < nchunk; c0 += 8 * GRP) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = c0 + u * GRP < nchunk ? src[(long)(c0 + u * GRP) * n + i] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += v[u];
+    }
+  if constexpr (GRP > 1) {
+    sh[g][o] = s;
+    __syncthreads();
+    if (g > 0) return;
+    for (int q = 1; q < GRP; q++) s += sh[q][o];
   }
+  if (i < n) (bias ? gb : gw)[i] = s;
 }
 
 // Space-to-depth input: x32[n][Y][X][8 s + c] = in[n][2Y + s / 2][2X + s % 2][c] * scale[c]
@@ -538,10 +609,9 @@ void WarmNet::get_params(std::vector<float>& out) {
   WN_HIP(hipMemcpy(out.data(), w_, out.size() * 4, hipMemcpyDeviceToHost));
 }
 
-void WarmNet::get_grads(std::vector<float>& out) {
-  out.resize(num_params());
+void WarmNet::get_grads(float* out) {
   WN_HIP(hipDeviceSynchronize());
-  WN_HIP(hipMemcpy(out.data(), g_, out.size() * 4, hipMemcpyDeviceToHost));
+  WN_HIP(hipMemcpy(out, g_, num_params() * 4, hipMemcpyDeviceToHost));
 }
 
 void WarmNet::set_params(const std::vector<float>& in) {
@@ -604,8 +674,13 @@ void WarmNet::wgrad(int li, const float* dy, const float* m, const float* x, con
     k_wgrad<3><<<grid, kNB, 0, s>>>(dy, m, x, u, l.cin, l.cout, H, W, batch, per, part_, bpart);
   else
     k_wgrad<1><<<grid, kNB, 0, s>>>(dy, m, x, u, l.cin, l.cout, H, W, batch, per, part_, bpart);
-  k_chunk_sum<<<grid_for(wlen), kNB, 0, s>>>(part_, wlen, (int)nch, g_ + l.woff);
-  k_chunk_sum<<<grid_for(l.cout), kNB, 0, s>>>(bpart, l.cout, (int)nch, g_ + l.boff);
+  // 16 threads per output from 64 chunks on (the outputs are few there)
+  const int out = nch >= 64 ? 16 : kNB;
+  const unsigned gs = (unsigned)((wlen + out - 1) / out + (l.cout + out - 1) / out);
+  if (nch >= 64)
+    k_chunk_sum<16><<<gs, kNB, 0, s>>>(part_, wlen, bpart, l.cout, (int)nch, g_ + l.woff, g_ + l.boff);
+  else
+    k_chunk_sum<1><<<gs, kNB, 0, s>>>(part_, wlen, bpart, l.cout, (int)nch, g_ + l.woff, g_ + l.boff);
 }
 
 static bool shape_ok(int batch, int H, int W, int max_batch, long max_pix) {

@@ -76,7 +76,7 @@ class WarmNet {
   // resets the optimiser state.
   void get_params(std::vector<float>& out);
   void set_params(const std::vector<float>& in);
-  void get_grads(std::vector<float>& out);
+  void get_grads(float* out);  // num_params() values
   // Channel scales: in[c] multiplies input channel c, out multiplies the output.
   void set_scales(const float* s) { for (int i = 0; i < kScales; i++) scales_[i] = s[i]; }
   const float* scales() const { return scales_; }
