@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 
 namespace isg {
 
@@ -12,7 +13,6 @@ namespace {
 constexpr int kNB = 256;  // threads per block
 constexpr int kCK = 32;   // input channels staged per pass
 constexpr int kCKP = kCK + 8;  // padded LDS row: 80 bytes keep the 16-byte loads aligned
-constexpr int kCOT = 64;  // output channels per workgroup
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
@@ -35,65 +35,86 @@ __host__ __device__ __forceinline__ float bf2f(uint16_t b) {
 
 // Convolution (KS = 1 or 3, stride 1, zero padding KS/2) on the matrix cores.
 //   Y[n][p][co] = act(bias[co] + sum_{tap,ci} bf16(In[n][p+tap][ci]) bf16(Wb[tap][co][ci]))
-//   In = X (+ up2(U)) (* [M > 0])
-// One workgroup: a 16x16-position tile of one image and up to 64 output
-// channels (NCB blocks of 16).  Waves split the output blocks and the tile's
-// 16 rows: wave w owns block w / (4 / NCB) and rows w % (4 / NCB) + (4 / NCB) j,
-// one MFMA row block (16 positions of a tile row) each, so a wave keeps its
-// block's weights of one input chunk (KS * KS fragments) in registers and
-// reuses them over 16 * NCB / 4 row blocks.  The input halo is staged through
-// LDS in chunks of 32 (or 16) input channels as BF16; a chunk of 32 is one
-// v_mfma_f32_16x16x32_bf16 per tap and row block (lane l supplies position
-// or output channel l % 16 and the 8 input channels 8 (l / 16) .. +7 of both
-// operands; the same channel order on both sides, so the sum over the chunk
-// is exact in any lane-to-channel assignment), a chunk of 16 one
-// v_mfma_f32_16x16x16_bf16.  Positions outside the image are zero on input
-// and not stored (partial tiles).
-template <int KS, int NCB, int MODE>  // MODE 0: In = X, 1: X + up2(U), 2: X * [M > 0]
-__global__ void __launch_bounds__(kNB) __attribute__((amdgpu_waves_per_eu(2))) k_conv(const float* __restrict__ X, const float* __restrict__ U,
-                                              const float* __restrict__ M, const uint16_t* __restrict__ Wb,
-                                              const float* __restrict__ bias, float* __restrict__ Y, int cin,
-                                              int cout, int cstore, int H, int W, int relu) {
+// Input (MODE): 0 In = X, 1 X + up2(U), 2 X * [M > 0], 3 the network's images
+// themselves: In[Y][X][8 s + c] = X[2Y + s / 2][2X + s % 2][c] * scale[c] (KS 3,
+// 32 channels; the space-to-depth form is then never stored).
+// Output (OUT): 0 Y; 1 Y and its 2x2 averages Y2 (a pooling pass would read Y
+// again); 2 / 3 a following 1x1 layer of 16 outputs (w2, b2; cout 32, one
+// workgroup holds them all) is applied and stored instead of Y: 2 packed,
+// [p][16], 3 depth-to-space times a scale, [2y + s / 2][2x + s % 2][c] from
+// channel 2 s + c < 8.
+// One workgroup: a 16x16-position tile of one image and NCB blocks of 16 output
+// channels; wave w owns tile rows 4 w .. +3 for all of them, so that a fragment
+// of the input read from LDS serves NCB matrix products (with a block per wave,
+// every wave read the whole tile and LDS was the limit).  The input halo is
+// staged through LDS in chunks of 32 (or 16) input channels as BF16; a chunk of
+// 32 is one v_mfma_f32_16x16x32_bf16 per tap and row block (lane l supplies
+// position or output channel l % 16 and the 8 input channels 8 (l / 16) .. +7 of
+// both operands), a chunk of 16 one v_mfma_f32_16x16x16_bf16.  Every output is
+// summed chunk by chunk, tap by tap, whatever NCB.  Positions outside the image
+// are zero on input and not stored (partial tiles).
+struct ConvExtra {
+  float* y2;            // OUT 1: averages; 2, 3: the following layer's output
+  const uint16_t* w2;   // OUT 2, 3: its weights [16][32] (BF16) and bias
+  const float* b2;
+  float scale;          // OUT 3: output scale
+};
+template <int KS, int NCB, int MODE, int OUT>
+// (held to 3 or 4 waves per SIMD the skip-added layers spill: 24 -> 46 us)
+__global__ void __launch_bounds__(kNB) __attribute__((amdgpu_waves_per_eu(2)))
+k_conv(const float* __restrict__ X, const float* __restrict__ U, const float* __restrict__ M,
+       const uint16_t* __restrict__ Wb, const float* __restrict__ bias, float* __restrict__ Y, int cin, int cout,
+       int cstore, int H, int W, int relu, ConvExtra ex) {
   constexpr int TS = 16, R = KS / 2, HW = TS + KS - 1, HS = HW * HW;
-  constexpr int WPC = 4 / NCB;     // waves per output block
-  constexpr int NRB = TS / WPC;    // row blocks per wave
+  constexpr int NR = 4;  // tile rows per wave
   __shared__ __attribute__((aligned(16))) uint16_t hal[HS * kCKP];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int n = blockIdx.y;
   const int tiles_x = (W + TS - 1) / TS;  // the last tile row / column may be partial
   const int ty0 = (blockIdx.x / tiles_x) * TS, tx0 = (blockIdx.x % tiles_x) * TS;
-  const int cb = w / WPC, part = w % WPC;
-  const int co = blockIdx.z * kCOT + cb * 16 + (lane & 15);  // this lane's B column / D channel
   const int ck = (cin % kCK == 0) ? kCK : 16;
   const int li = lane & 15, kq = lane >> 4;
-  v4f acc[NRB];
+  const int co0 = blockIdx.z * (16 * NCB) + li;  // this lane's B column / D channel of block 0
+  v4f acc[NR][NCB];
 #pragma unroll
-  for (int j = 0; j < NRB; j++) acc[j] = v4f{0, 0, 0, 0};
+  for (int j = 0; j < NR; j++)
+#pragma unroll
+    for (int b = 0; b < NCB; b++) acc[j][b] = v4f{0, 0, 0, 0};
   const long img = (long)n * H * W;
-  const uint16_t* wrow = Wb + (long)co * cin;  // + tap * cout * cin + ci
   const int sh4 = ck == kCK ? 3 : 2;  // log2 of the float4 groups per position in a chunk
   for (int ci0 = 0; ci0 < cin; ci0 += ck) {
     // halo staging: every load of the thread's share is issued before the
-    // first conversion, so their latencies overlap (NE float4 groups each)
+    // first conversion, so their latencies overlap (NE float4 groups each).
+    // (Loading the next chunk during the products cost more registers, hence
+    // waves, than it hid: 24 -> 39 us for the skip-added 512^2 x 4 layers.)
     constexpr int NE = (HS * (kCK / 4) + kNB - 1) / kNB;
-    float4 v[NE], a2[MODE ? NE : 1];  // a2: the upsampled addend (MODE 1) or the mask (MODE 2)
+    constexpr bool ADD = MODE == 1 || MODE == 2;
+    float4 v[NE], a2[ADD ? NE : 1];  // a2: the upsampled addend (MODE 1) or the mask (MODE 2)
 #pragma unroll
     for (int q = 0; q < NE; q++) {
       const int e = tid + q * kNB;
       const int hp = e >> sh4, c4 = e & ((1 << sh4) - 1);
       const int gy = ty0 + hp / HW - R, gx = tx0 + hp % HW - R;
       v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if constexpr (MODE != 0) a2[q] = v[q];
+      if constexpr (ADD) a2[q] = v[q];
       if (hp < HS && gy >= 0 && gy < H && gx >= 0 && gx < W) {
-        const long pix = img + (long)gy * W + gx;
-        v[q] = *reinterpret_cast<const float4*>(X + pix * cin + ci0 + 4 * c4);
-        if constexpr (MODE == 1) {
-          const long up = (long)n * (H >> 1) * (W >> 1) + (long)(gy >> 1) * (W >> 1) + (gx >> 1);
-          a2[q] = *reinterpret_cast<const float4*>(U + up * cin + ci0 + 4 * c4);
+        if constexpr (MODE == 3) {
+          const int s = c4 >> 1;
+          v[q] = *reinterpret_cast<const float4*>(
+              X + (((long)n * 2 * H + 2 * gy + (s >> 1)) * 2 * W + 2 * gx + (s & 1)) * 8 + 4 * (c4 & 1));
+        } else {
+          const long pix = img + (long)gy * W + gx;
+          v[q] = *reinterpret_cast<const float4*>(X + pix * cin + ci0 + 4 * c4);
+          if constexpr (MODE == 1) {
+            const long up = (long)n * (H >> 1) * (W >> 1) + (long)(gy >> 1) * (W >> 1) + (gx >> 1);
+            a2[q] = *reinterpret_cast<const float4*>(U + up * cin + ci0 + 4 * c4);
+          }
+          if constexpr (MODE == 2) a2[q] = *reinterpret_cast<const float4*>(M + pix * cin + ci0 + 4 * c4);
         }
-        if constexpr (MODE == 2) a2[q] = *reinterpret_cast<const float4*>(M + pix * cin + ci0 + 4 * c4);
       }
     }
+    float4 sc = make_float4(1.f, 1.f, 1.f, 1.f);
+    if constexpr (MODE == 3) sc = *reinterpret_cast<const float4*>(M + 4 * (tid & 1));  // M: the input scales
 #pragma unroll
     for (int q = 0; q < NE; q++) {
       const int e = tid + q * kNB;
@@ -109,61 +130,127 @@ __global__ void __launch_bounds__(kNB) __attribute__((amdgpu_waves_per_eu(2))) k
         x.z = a2[q].z > 0.f ? x.z : 0.f;
         x.w = a2[q].w > 0.f ? x.w : 0.f;
       }
+      if constexpr (MODE == 3) {
+        x.x *= sc.x; x.y *= sc.y; x.z *= sc.z; x.w *= sc.w;
+      }
       uint2 pk;
       pk.x = (uint32_t)f2bf(x.x) | ((uint32_t)f2bf(x.y) << 16);
       pk.y = (uint32_t)f2bf(x.z) | ((uint32_t)f2bf(x.w) << 16);
       *reinterpret_cast<uint2*>(&hal[hp * kCKP + 4 * c4]) = pk;
     }
-    // this lane's weight fragment of one tap (8 input channels of its output
-    // channel), the next tap's loaded while the current one's MFMAs run
+    // this lane's weight fragments of one tap (8 input channels of its output
+    // channel per block), the next tap's loaded while the current one's MFMAs run
     if (ck == kCK) {
-      const uint16_t* wp = wrow + ci0 + 8 * kq;
-      v8s bn = *reinterpret_cast<const v8s*>(wp);
+      const uint16_t* wp = Wb + (long)co0 * cin + ci0 + 8 * kq;
+      v8s bn[NCB];
+#pragma unroll
+      for (int b = 0; b < NCB; b++) bn[b] = *reinterpret_cast<const v8s*>(wp + (long)16 * b * cin);
       __syncthreads();
 #pragma unroll 1
       for (int tap = 0; tap < KS * KS; tap++) {
-        const v8bf b = __builtin_bit_cast(v8bf, bn);
-        if (tap + 1 < KS * KS) bn = *reinterpret_cast<const v8s*>(wp + (long)(tap + 1) * cout * cin);
-        const int dy = tap / KS, dx = tap % KS;
-        const uint16_t* hb = &hal[(dy * HW + li + dx) * kCKP + 8 * kq];
+        v8bf bt[NCB];
 #pragma unroll
-        for (int j = 0; j < NRB; j++) {
-          const int rb = part + WPC * j;
-          const v8bf a = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8s*>(hb + rb * HW * kCKP));
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[j], 0, 0, 0);
+        for (int b = 0; b < NCB; b++) {
+          bt[b] = __builtin_bit_cast(v8bf, bn[b]);
+          if (tap + 1 < KS * KS)
+            bn[b] = *reinterpret_cast<const v8s*>(wp + ((long)(tap + 1) * cout + 16 * b) * cin);
+        }
+        const int dy = tap / KS, dx = tap % KS;
+        const uint16_t* hb = &hal[((4 * w + dy) * HW + li + dx) * kCKP + 8 * kq];
+#pragma unroll
+        for (int j = 0; j < NR; j++) {
+          const v8bf a = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8s*>(hb + j * HW * kCKP));
+#pragma unroll
+          for (int b = 0; b < NCB; b++) acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bt[b], acc[j][b], 0, 0, 0);
         }
       }
     } else {
-      const uint16_t* wp = wrow + ci0 + 4 * kq;
-      v4s bn = *reinterpret_cast<const v4s*>(wp);
+      const uint16_t* wp = Wb + (long)co0 * cin + ci0 + 4 * kq;
       __syncthreads();
 #pragma unroll 1
       for (int tap = 0; tap < KS * KS; tap++) {
-        const v4s b = bn;
-        if (tap + 1 < KS * KS) bn = *reinterpret_cast<const v4s*>(wp + (long)(tap + 1) * cout * cin);
         const int dy = tap / KS, dx = tap % KS;
-        const uint16_t* hb = &hal[(dy * HW + li + dx) * kCKP + 4 * kq];
+        const uint16_t* hb = &hal[((4 * w + dy) * HW + li + dx) * kCKP + 4 * kq];
 #pragma unroll
-        for (int j = 0; j < NRB; j++) {
-          const int rb = part + WPC * j;
-          const v4s a = *reinterpret_cast<const v4s*>(hb + rb * HW * kCKP);
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
+        for (int b = 0; b < NCB; b++) {
+          const v4s bt = *reinterpret_cast<const v4s*>(wp + ((long)tap * cout + 16 * b) * cin);
+#pragma unroll
+          for (int j = 0; j < NR; j++) {
+            const v4s a = *reinterpret_cast<const v4s*>(hb + j * HW * kCKP);
+            acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bt, acc[j][b], 0, 0, 0);
+          }
         }
       }
     }
     __syncthreads();
   }
   // D[i][j]: lane j + 16 (i / 4), register i % 4; i = position within the row block, j = channel
-  const float bv = bias ? bias[co] : 0.f;
 #pragma unroll
-  for (int j = 0; j < NRB; j++) {
-    const int gy = ty0 + part + WPC * j;
+  for (int b = 0; b < NCB; b++) {
+    const int co = co0 + 16 * b;
+    const float bv = bias ? bias[co] : 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int gx = tx0 + 4 * kq + r;
-      float v = acc[j][r] + bv;
-      if (relu) v = v > 0.f ? v : 0.f;
-      if (co < cstore && gy < H && gx < W) Y[(img + (long)gy * W + gx) * cstore + co] = v;
+    for (int j = 0; j < NR; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        float v = acc[j][b][r] + bv;
+        if (relu) v = v > 0.f ? v : 0.f;
+        acc[j][b][r] = v;
+      }
+  }
+  if constexpr (OUT <= 1) {
+#pragma unroll
+    for (int b = 0; b < NCB; b++) {
+      const int co = co0 + 16 * b;
+#pragma unroll
+      for (int j = 0; j < NR; j++) {
+        const int gy = ty0 + 4 * w + j;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int gx = tx0 + 4 * kq + r;
+          if (co < cstore && gy < H && gx < W) Y[(img + (long)gy * W + gx) * cstore + co] = acc[j][b][r];
+        }
+      }
+      if constexpr (OUT == 1) {
+        // H and W are even, so a 2x2 block lies inside the image or outside it
+#pragma unroll
+        for (int j = 0; j < NR; j += 2)
+#pragma unroll
+          for (int r = 0; r < 4; r += 2) {
+            const int gy = ty0 + 4 * w + j, gx = tx0 + 4 * kq + r;
+            if (co < cstore && gy < H && gx < W)
+              ex.y2[(((long)n * (H / 2) + gy / 2) * (W / 2) + gx / 2) * cstore + co] =
+                  0.25f * (acc[j][b][r] + acc[j][b][r + 1] + acc[j + 1][b][r] + acc[j + 1][b][r + 1]);
+          }
+      }
+    }
+  } else {
+    // the tile's 32 channels as BF16 in LDS (rows of this wave only), then the 1x1 layer
+#pragma unroll
+    for (int j = 0; j < NR; j++)
+#pragma unroll
+      for (int b = 0; b < NCB; b++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) hal[((4 * w + j) * TS + 4 * kq + r) * kCKP + 16 * b + li] = f2bf(acc[j][b][r]);
+    const v8bf b2 = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8s*>(ex.w2 + li * 32 + 8 * kq));
+    const float bv = ex.b2[li];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NR; j++) {
+      const v8bf a = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8s*>(&hal[((4 * w + j) * TS + li) * kCKP + 8 * kq]));
+      const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b2, v4f{0, 0, 0, 0}, 0, 0, 0);
+      const int gy = ty0 + 4 * w + j;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int gx = tx0 + 4 * kq + r;
+        if (gy >= H || gx >= W) continue;
+        if constexpr (OUT == 2) {
+          ex.y2[(img + (long)gy * W + gx) * 16 + li] = d[r] + bv;
+        } else if (li < 8) {
+          const int s = li >> 1;
+          ex.y2[(((long)n * 2 * H + 2 * gy + (s >> 1)) * 2 * W + 2 * gx + (s & 1)) * 2 + (li & 1)] = (d[r] + bv) * ex.scale;
+        }
+      }
     }
   }
 }
@@ -358,29 +445,9 @@ __global__ void k_net_pack(const float* __restrict__ in, int batch, int H, int W
   }
 }
 
-// Depth-to-space output: out[n][2Y + s / 2][2X + s % 2][c] = y16[n][Y][X][2 s + c] * scale, c < 2
-__global__ void k_net_unpack(const float* __restrict__ y16, int batch, int H, int W, float scale,
-                             float* __restrict__ out) {
-  constexpr int S = WarmNet::kS2D;
-  const int Wn = W / S;
-  const long total = (long)batch * H * W * 2;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(i & 1);
-    long q = i >> 1;
-    const int x = (int)(q % W);
-    q /= W;
-    const int y = (int)(q % H);
-    const long n = q / H;
-    const int sp = (y % S) * S + x % S;
-    const long pn = (n * (H / S) + y / S) * Wn + x / S;
-    out[i] = y16[pn * 16 + 2 * sp + c] * scale;
-  }
-}
-
-// 2x2 pooling: average (sum = 0) or sum (sum = 1); H, W of the input.
-__global__ void k_pool(const float* __restrict__ x, float* __restrict__ y, int batch, int H, int W, int C, int sum) {
+// 2x2 sums (backward of the upsampling); H, W of the input.
+__global__ void k_pool_sum(const float* __restrict__ x, float* __restrict__ y, int batch, int H, int W, int C) {
   const long n_out = (long)batch * (H / 2) * (W / 2) * C;
-  const float f = sum ? 1.f : 0.25f;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n_out; i += (long)gridDim.x * blockDim.x) {
     const int c = (int)(i % C);
     long p = i / C;
@@ -389,7 +456,7 @@ __global__ void k_pool(const float* __restrict__ x, float* __restrict__ y, int b
     const int oy = (int)(p % (H / 2));
     const long n = p / (H / 2);
     const long b = ((n * H + 2 * oy) * W + 2 * ox) * C + c;
-    y[i] = f * (x[b] + x[b + C] + x[b + (long)W * C] + x[b + (long)W * C + C]);
+    y[i] = (x[b] + x[b + C] + x[b + (long)W * C] + x[b + (long)W * C + C]);
   }
 }
 
@@ -629,35 +696,68 @@ void WarmNet::set_params(const std::vector<float>& in) {
   WN_HIP(hipDeviceSynchronize());
 }
 
+// out: 0 the layer alone, 1 also its 2x2 averages (into y2), 2 / 3 followed by
+// layer 10, packed / as images (into y2; layer 9 only).  x is the images
+// themselves when raw (layer 0).
 void WarmNet::conv(int li, const float* x, const float* u, const float* m, float* y, int cstore, bool transpose,
-                   int batch, int H, int W, hipStream_t s) {
+                   int batch, int H, int W, hipStream_t s, int out, float* y2, bool raw) {
   const NetLayer& l = layers()[li];
   const int cin = transpose ? l.cout : l.cin, cout = transpose ? l.cin : l.cout;
   const uint16_t* wb = (transpose ? wt_ : wb_) + l.woff;
   const float* bias = transpose ? nullptr : w_ + l.boff;
   const int relu = transpose ? 0 : l.relu;
-  dim3 grid(((H + 15) / 16) * ((W + 15) / 16), batch, (cout + kCOT - 1) / kCOT);
-  // output blocks of 16 channels per workgroup: 1, 2 or 4 (every layer's widths are 16, 32 or multiples of 64)
-  const int ncb = std::min(4, cout / 16);
-  // input mode: plain, plus the upsampled decoder input (skip connection), or masked by a ReLU output
+  // input mode: plain, plus the upsampled decoder input (skip connection), masked by a ReLU output, or images
   if (u && m) {
     if (err_.empty()) err_ = "warm-start network: a convolution input cannot be both skip-added and masked";
     return;
   }
-  const int mode = u ? 1 : (m ? 2 : 0);
-#define WN_CONV(KS, NCB, MODE) \
-  k_conv<KS, NCB, MODE><<<grid, kNB, 0, s>>>(x, u, m, wb, bias, y, cin, cout, cstore, H, W, relu)
-#define WN_CONV_NCB(KS, MODE) \
-  do { if (ncb == 4) WN_CONV(KS, 4, MODE); else if (ncb == 2) WN_CONV(KS, 2, MODE); else WN_CONV(KS, 1, MODE); } while (0)
-#define WN_CONV_MODE(KS) \
-  do { if (mode == 1) WN_CONV_NCB(KS, 1); else if (mode == 2) WN_CONV_NCB(KS, 2); else WN_CONV_NCB(KS, 0); } while (0)
-  if (l.ks == 3)
-    WN_CONV_MODE(3);
-  else
-    WN_CONV_MODE(1);
-#undef WN_CONV_MODE
-#undef WN_CONV_NCB
-#undef WN_CONV
+  const int mode = raw ? 3 : (u ? 1 : (m ? 2 : 0));
+  // 16-channel output blocks per workgroup: as many as divide the layer's
+  // width (4 at most), fewer while that leaves less than two workgroups per CU
+  // (each then stages the same halo again, from L2): the 32^2 and 64^2-position
+  // levels of a 512^2 x 4 batch were 64 and 128 workgroups of 8 and 4 serial chunks.
+  // With that and the wave split by rows: 3x3 layers 22-32 -> 13-26 us, 1x1 22 -> 12.
+  const long tiles = (long)((H + 15) / 16) * ((W + 15) / 16) * batch;
+  int ncb = std::min(4, cout / 16);
+  if (out < 2)
+    while (ncb > 1 && tiles * (cout / (16 * ncb)) < 512) ncb /= 2;
+  const ConvExtra ex{y2, wb_ + layers()[kLayers - 1].woff, w_ + layers()[kLayers - 1].boff, scales_[kInCh]};
+  auto go = [&](auto ksc, auto ncbc, auto modec, auto outc) {
+    constexpr int N = decltype(ncbc)::value;
+    dim3 grid(((H + 15) / 16) * ((W + 15) / 16), batch, cout / (16 * N));
+    k_conv<decltype(ksc)::value, N, decltype(modec)::value, decltype(outc)::value>
+        <<<grid, kNB, 0, s>>>(x, u, decltype(modec)::value == 3 ? dscale_ : m, wb, bias, y, cin, cout, cstore, H, W,
+                              relu, ex);
+  };
+#define WN_I(v) std::integral_constant<int, v>()
+  auto by_ncb = [&](auto ksc, auto modec, auto outc) {
+    if (ncb == 4)
+      go(ksc, WN_I(4), modec, outc);
+    else if (ncb == 2)
+      go(ksc, WN_I(2), modec, outc);
+    else
+      go(ksc, WN_I(1), modec, outc);
+  };
+  if (l.ks == 1) {
+    by_ncb(WN_I(1), WN_I(0), WN_I(0));  // the 1x1 layers have plain inputs
+  } else if (out >= 2) {
+    if (out == 2)
+      go(WN_I(3), WN_I(2), WN_I(1), WN_I(2));
+    else
+      go(WN_I(3), WN_I(2), WN_I(1), WN_I(3));
+  } else if (out == 1) {
+    if (mode == 3)
+      by_ncb(WN_I(3), WN_I(3), WN_I(1));
+    else
+      by_ncb(WN_I(3), WN_I(0), WN_I(1));
+  } else if (mode == 1) {
+    by_ncb(WN_I(3), WN_I(1), WN_I(0));
+  } else if (mode == 2) {
+    by_ncb(WN_I(3), WN_I(2), WN_I(0));
+  } else {
+    by_ncb(WN_I(3), WN_I(0), WN_I(0));
+  }
+#undef WN_I
 }
 
 void WarmNet::wgrad(int li, const float* dy, const float* m, const float* x, const float* u, int batch, int H,
@@ -690,13 +790,14 @@ static bool shape_ok(int batch, int H, int W, int max_batch, long max_pix) {
 
 static const char* kShapeMsg = "warm-start network: image shape outside the workspace (H, W multiples of 16)";
 
-// H, W: the image's sides; the network runs on the space-to-depth image.
+// Images to the packed input (the training step keeps it for the weight
+// gradient) and every layer; H, W: the image's sides.
 void WarmNet::forward_all(const float* in, int batch, int Hi, int Wi, hipStream_t s) {
   WN_HIP(hipMemcpyAsync(dscale_, scales_, sizeof(float) * kScales, hipMemcpyHostToDevice, s));
   const int H = Hi / kS2D, W = Wi / kS2D;
   const long np = (long)batch * H * W;
   k_net_pack<<<grid_for(np * 32), kNB, 0, s>>>(in, batch, Hi, Wi, dscale_, act_[A_X]);
-  forward_layers(batch, H, W, s);
+  forward_layers(act_[A_X], false, batch, H, W, s, 0, nullptr);
 }
 
 float* WarmNet::packed_input(int batch, int Hi, int Wi) {
@@ -714,31 +815,28 @@ void WarmNet::forward_packed(int batch, int Hi, int Wi, hipStream_t s) {
     err_ = kShapeMsg;
     return;
   }
-  forward_layers(batch, Hi / kS2D, Wi / kS2D, s);
+  forward_layers(act_[A_X], false, batch, Hi / kS2D, Wi / kS2D, s, 2, act_[A_OUT]);
   WN_HIP(hipGetLastError());
 }
 
-// every layer from the packed input act_[A_X] (H, W: the network's level-0 sides)
-void WarmNet::forward_layers(int batch, int H, int W, hipStream_t s) {
-  const long np = (long)batch * H * W;
+// Every layer from x: the packed input, or the images themselves (raw); H, W:
+// the network's level-0 sides.  last 0: layers 9 and 10 one by one, both stored
+// (training); 2 / 3: layer 10 inside layer 9, packed / images into y.
+void WarmNet::forward_layers(const float* x, bool raw, int batch, int H, int W, hipStream_t s, int last, float* y) {
   const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
-  conv(0, act_[A_X], nullptr, nullptr, act_[A_E0], 32, false, batch, H, W, s);
-  k_pool<<<grid_for(np * 32 / 4), kNB, 0, s>>>(act_[A_E0], act_[A_P0], batch, H, W, 32, 0);
-  conv(1, act_[A_P0], nullptr, nullptr, act_[A_E1], 64, false, batch, H1, W1, s);
-  k_pool<<<grid_for(np * 64 / 16), kNB, 0, s>>>(act_[A_E1], act_[A_P1], batch, H1, W1, 64, 0);
-  conv(2, act_[A_P1], nullptr, nullptr, act_[A_E2], 128, false, batch, H2, W2, s);
-  k_pool<<<grid_for(np * 128 / 64), kNB, 0, s>>>(act_[A_E2], act_[A_P2], batch, H2, W2, 128, 0);
+  conv(0, x, nullptr, nullptr, act_[A_E0], 32, false, batch, H, W, s, 1, act_[A_P0], raw);
+  conv(1, act_[A_P0], nullptr, nullptr, act_[A_E1], 64, false, batch, H1, W1, s, 1, act_[A_P1]);
+  conv(2, act_[A_P1], nullptr, nullptr, act_[A_E2], 128, false, batch, H2, W2, s, 1, act_[A_P2]);
   conv(3, act_[A_P2], nullptr, nullptr, act_[A_E3], 256, false, batch, H3, W3, s);
   conv(4, act_[A_E3], nullptr, nullptr, act_[A_U3], 128, false, batch, H3, W3, s);
   conv(5, act_[A_E2], act_[A_U3], nullptr, act_[A_D2], 128, false, batch, H2, W2, s);
   conv(6, act_[A_D2], nullptr, nullptr, act_[A_U2], 64, false, batch, H2, W2, s);
   conv(7, act_[A_E1], act_[A_U2], nullptr, act_[A_D1], 64, false, batch, H1, W1, s);
   conv(8, act_[A_D1], nullptr, nullptr, act_[A_U1], 32, false, batch, H1, W1, s);
-  conv(9, act_[A_E0], act_[A_U1], nullptr, act_[A_D0], 32, false, batch, H, W, s);
-  conv(10, act_[A_D0], nullptr, nullptr, act_[A_OUT], 16, false, batch, H, W, s);
+  conv(9, act_[A_E0], act_[A_U1], nullptr, act_[A_D0], 32, false, batch, H, W, s, last, y);
+  if (last == 0) conv(10, act_[A_D0], nullptr, nullptr, act_[A_OUT], 16, false, batch, H, W, s);
   WN_HIP(hipGetLastError());
 }
-
 
 void WarmNet::forward(const float* in, float* out, int batch, int H, int W, hipStream_t s) {
   if (!ok()) return;
@@ -746,9 +844,11 @@ void WarmNet::forward(const float* in, float* out, int batch, int H, int W, hipS
     err_ = kShapeMsg;
     return;
   }
-  forward_all(in, batch, H, W, s);
-  k_net_unpack<<<grid_for((long)batch * H * W * 2), kNB, 0, s>>>(act_[A_OUT], batch, H, W, scales_[kInCh], out);
-  WN_HIP(hipGetLastError());
+  WN_HIP(hipMemcpyAsync(dscale_, scales_, sizeof(float) * kScales, hipMemcpyHostToDevice, s));
+  const int Hn = H / kS2D, Wn = W / kS2D;
+  const bool raw = ((uintptr_t)in & 15) == 0;  // layer 0 reads the images 16 bytes at a time
+  if (!raw) k_net_pack<<<grid_for((long)batch * Hn * Wn * 32), kNB, 0, s>>>(in, batch, H, W, dscale_, act_[A_X]);
+  forward_layers(raw ? in : act_[A_X], raw, batch, Hn, Wn, s, 3, out);
 }
 
 double WarmNet::loss_grad(const float* in, const float* target, int batch, int Hi, int Wi, hipStream_t s) {
@@ -769,17 +869,17 @@ double WarmNet::loss_grad(const float* in, const float* target, int batch, int H
   conv(10, grd_[G_OUT], nullptr, nullptr, grd_[G_D0], 32, true, batch, H, W, s);
   wgrad(9, grd_[G_D0], act_[A_D0], act_[A_E0], act_[A_U1], batch, H, W, s);
   conv(9, grd_[G_D0], nullptr, act_[A_D0], grd_[G_IN0], 32, true, batch, H, W, s);
-  k_pool<<<grid_for(np * 32 / 4), kNB, 0, s>>>(grd_[G_IN0], grd_[G_U1], batch, H, W, 32, 1);
+  k_pool_sum<<<grid_for(np * 32 / 4), kNB, 0, s>>>(grd_[G_IN0], grd_[G_U1], batch, H, W, 32);
   wgrad(8, grd_[G_U1], nullptr, act_[A_D1], nullptr, batch, H1, W1, s);
   conv(8, grd_[G_U1], nullptr, nullptr, grd_[G_D1], 64, true, batch, H1, W1, s);
   wgrad(7, grd_[G_D1], act_[A_D1], act_[A_E1], act_[A_U2], batch, H1, W1, s);
   conv(7, grd_[G_D1], nullptr, act_[A_D1], grd_[G_IN1], 64, true, batch, H1, W1, s);
-  k_pool<<<grid_for(np * 64 / 16), kNB, 0, s>>>(grd_[G_IN1], grd_[G_U2], batch, H1, W1, 64, 1);
+  k_pool_sum<<<grid_for(np * 64 / 16), kNB, 0, s>>>(grd_[G_IN1], grd_[G_U2], batch, H1, W1, 64);
   wgrad(6, grd_[G_U2], nullptr, act_[A_D2], nullptr, batch, H2, W2, s);
   conv(6, grd_[G_U2], nullptr, nullptr, grd_[G_D2], 128, true, batch, H2, W2, s);
   wgrad(5, grd_[G_D2], act_[A_D2], act_[A_E2], act_[A_U3], batch, H2, W2, s);
   conv(5, grd_[G_D2], nullptr, act_[A_D2], grd_[G_IN2], 128, true, batch, H2, W2, s);
-  k_pool<<<grid_for(np * 128 / 64), kNB, 0, s>>>(grd_[G_IN2], grd_[G_U3], batch, H2, W2, 128, 1);
+  k_pool_sum<<<grid_for(np * 128 / 64), kNB, 0, s>>>(grd_[G_IN2], grd_[G_U3], batch, H2, W2, 128);
   wgrad(4, grd_[G_U3], nullptr, act_[A_E3], nullptr, batch, H3, W3, s);
   conv(4, grd_[G_U3], nullptr, nullptr, grd_[G_E3], 256, true, batch, H3, W3, s);
   // encoder, bottom-up

@@ -103,9 +103,9 @@ class WarmNet {
 
  private:
   void forward_all(const float* in, int batch, int H, int W, hipStream_t s);
-  void forward_layers(int batch, int H, int W, hipStream_t s);
+  void forward_layers(const float* x, bool raw, int batch, int H, int W, hipStream_t s, int last, float* y);
   void conv(int li, const float* x, const float* u, const float* m, float* y, int cstore, bool transpose,
-            int batch, int H, int W, hipStream_t s);
+            int batch, int H, int W, hipStream_t s, int out = 0, float* y2 = nullptr, bool raw = false);
   void wgrad(int li, const float* dy, const float* m, const float* x, const float* u, int batch, int H, int W,
              hipStream_t s);
   void refresh_bf16(hipStream_t s);
