@@ -103,12 +103,12 @@ def measured_traffic(split):
     return None
 
 
-def m2l_bytes_per_rhs(level, numsamp, cbytes, fused_leaf=False):
+def m2l_bytes_per_rhs(level, numsamp, cbytes, fused=False):
     """Read every multipole once and write every local once, levels 2..leaf;
-    with the fused leaf kernel also read the parent locals it interpolates."""
+    with the fused M2L + L2L kernels also read the parent locals they interpolate."""
     b = sum(2 * cbytes * 4 ** i * numsamp[i] for i in range(2, level))
-    if fused_leaf:
-        b += cbytes * 4 ** (level - 2) * numsamp[level - 2]
+    if fused:
+        b += sum(cbytes * 4 ** (i - 1) * numsamp[i - 1] for i in range(3, level))
     return b
 
 
@@ -217,7 +217,9 @@ def run_paths(isg, args, wl, common, otrue, mes, paths, warmup, steps, timing):
                 s.close()
                 continue
             ptime = timing
-            fused = fused or s.tuning_get(fast_prec, 1, "leaf") == 1
+            # M2L and L2L of a level in one kernel: the leaf (1) or, FP32, every level (-1, the built-in rule)
+            leaf = s.tuning_get(fast_prec, 1, "leaf")
+            fused = fused or leaf == 1 or (leaf == -1 and fast_prec == 1)
             # the split-FP16 near field k_near_h16 (tuning values 128 and 256) serves grids of >= 8 x 8
             # leaf boxes; the built-in rule (-1) takes it from 256 workgroups of 64 boxes on
             nv = s.tuning_get(1, 1 if batch >= 16 else 0, "near")

@@ -259,21 +259,20 @@ int isg_raster_bin_read(const char* path, int numunk, double* raster);
 
 /* ---- autotuner (kernel variants per stage and level, measured on the device) ----
  * stage 0 near-field tile width (16, 32 or 64 boxes; 64 for the FP32
- * operator only; 128, FP32 operator only: the split-FP16 kernel, 64-box tiles
- * of two right-hand sides on the FP16 matrix cores with FP32 operands carried
- * as hi + lo, used for launches of 4 or more right-hand sides; 256, likewise:
- * 128-box tiles of one right-hand side, grids of 16 x 8 leaf boxes or more), 1 P2M tile
- * width (16, 32 or 64; 128, FP32 operator only: the split-FP16 P2M, 32-box
+ * operator only; 128 or 256, FP32 operator only: the split-FP16 kernel, 64-box
+ * tiles on the FP16 matrix cores with FP32 operands carried as hi + lo), 1 P2M
+ * tile width (16, 32 or 64; 128, FP32 operator only: the split-FP16 P2M, 32-box
  * tiles of two right-hand sides, 4 or more right-hand sides), 2 M2L tile
  * variant of `level` (0: 4x4 boxes x 8 samples, 1: 8x8 x 8, 2: 8x8 x 16,
  * 3: 16x16 x 8, 4: 8x8 x 32, 5: 16x16 x 16; 6, 7, 8: 8x8 x 16, 32, 8 with the
- * operators held in registers; 9: 8x8 x 16, one thread per parent with its 36
- * sources in registers; 4, 5 and 7 FP32 only), 3 / 4 M2M / L2L
- * kernel of `level` (0 band MFMA, 1 chunked LDS, 2 direct, 3 / 4 band MFMA with
- * 16 / 32 columns per workgroup), 5 leaf fusion (`level` ignored; 1: the
- * leaf-level M2L and the L2L into the leaf level run as one kernel that
- * writes each leaf local expansion once, 0: separate); value -1 = built-in
- * rule (separate).  precision 0 = FP64 operator, 1 = FP32 operator of the mixed path;
+ * operators held in registers; 9: 8x8 x 16, one thread per parent, one launch
+ * for all levels that have it, and the built-in rule; 4, 5 and 7 FP32 only), 3 / 4
+ * M2M / L2L kernel of `level` (0 band MFMA, 1 chunked LDS, 2 direct, 3 / 4 band
+ * MFMA with 16 / 32 columns per workgroup), 5 fusion (`level` ignored; FP32
+ * operator: M2L and the L2L into a level as one kernel that writes each local
+ * expansion once, -1: every level from 3 on, 1: the leaf level, 0: none; the FP64
+ * operator runs them separately); value -1 = built-in
+ * rule.  precision 0 = FP64 operator, 1 = FP32 operator of the mixed path;
  * batch_class 0 for fewer than 16 right-hand sides, 1 otherwise.
  * isg_autotune times every admissible variant (reps launches each) and keeps
  * the fastest for batch_class(nrhs) and every operator precision the context has.

@@ -13,6 +13,7 @@
 
 #include <rocblas/rocblas.h>
 
+#include "isg_down_h16.hpp"
 #include "isg_kernels.hpp"
 #include "isg_near_h16.hpp"
 #include "isg_near_sym.hpp"
@@ -316,6 +317,7 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
   rxaI_ = up_i(P_.rxaI);
   plan_interp(op64_, m2m64_, l2l64_);
   if (has32_) plan_interp(op32_, m2m32_, l2l32_);
+  if (has32_) build_down16();
   for (auto& row : tune_)
     for (auto& t : row) {
       t.m2l.assign(P_.L, -1);
@@ -508,6 +510,54 @@ void Engine::build_split16() {
                                                                 (v8h*)p2m16_);
   ISG_HIP(hipGetLastError());
   ISG_HIP(hipStreamSynchronize(stream_));
+}
+
+// Tables of k_down_h16 for levels 3 .. leaf: the band blocks of each level's
+// anterpolator with the four child shifts folded in, split into FP16.  Left
+// empty (separate M2L and L2L kernels) if some level's window exceeds 96.
+void Engine::build_down16() {
+  if (!ok()) return;
+  const int L = P_.L, na = 2 * cfg_.plan.ninter;
+  std::vector<DownLevel> lv(L);
+  std::vector<double> AB;
+  std::vector<int> s0;
+  for (int i = 3; i < L; i++) {
+    const int S = P_.nsamp[i], Sp = P_.nsamp[i - 1], nrb = (S + 15) / 16;
+    const int kb = build_band(S, Sp, na, P_.anterp0[i], P_.anterpT[i], kDownK, AB, s0);
+    // (the kernel's offsets within a level of one right-hand side are 32 bits wide)
+    if (kb == 0 || lvl_size_[i] * sizeof(zf) >= 0xffffff00u) return;
+    double m = 0;
+    for (double v : AB) m = std::max(m, std::fabs(v));
+    DownLevel& d = lv[i];
+    d.kb = kb;
+    d.ec = h16_scale_exp((float)m);
+    d.tab = dalloc((size_t)nrb * 4 * kDownFrag * 16);
+    d.s0 = (int*)dalloc(s0.size() * sizeof(int));
+    double* ab = nullptr;
+    if (!ok()) return;
+    ISG_HIP(hipMalloc((void**)&ab, AB.size() * sizeof(double)));
+    if (!ok()) return;
+    ISG_HIP(hipMemcpy(ab, AB.data(), AB.size() * sizeof(double), hipMemcpyHostToDevice));
+    ISG_HIP(hipMemcpy(d.s0, s0.data(), s0.size() * sizeof(int), hipMemcpyHostToDevice));
+    k_split_l2l<<<nblocks((long)nrb * 4 * kDownG * 16), kBlock, 0, stream_>>>(ab, d.s0, kb, op64_.shiftL[i - 1], Sp, nrb,
+                                                                             d.ec, (v8h*)d.tab);
+    ISG_HIP(hipGetLastError());
+    ISG_HIP(hipStreamSynchronize(stream_));
+    (void)hipFree(ab);
+  }
+  down16_ = lv;
+}
+
+// M2L of level i and the L2L into it (FP32 operator).  Right-hand sides per
+// workgroup: as many as leave four workgroups per CU, 8 at most.
+void Engine::launch_down16(int i, int nrhs, const int* act) {
+  const int S = P_.nsamp[i], nb = 1 << i, blocks = nb * nb / (kDownTS * kDownTS) * ((S + kDownKC - 1) / kDownKC);
+  const int per = (int)std::min<long>(8, std::max<long>(1, (long)blocks * nrhs / 1024));
+  const DownLevel& d = down16_[i];
+  DevOp<float>& o = op32_;
+  k_down_h16<<<dim3(blocks, (nrhs + per - 1) / per), dim3(kBlock), 0, stream_>>>(
+      o.agm + lvl_off_[i], o.agl + lvl_off_[i], (long)lvl_size_[i], o.trans[i], i, S, o.agl + lvl_off_[i - 1],
+      (long)lvl_size_[i - 1], P_.nsamp[i - 1], (const v8h*)d.tab, d.s0, d.kb, d.ec, nrhs, per, act);
 }
 
 // ------------------------------------------------------- interpolation plan
@@ -804,35 +854,6 @@ void Engine::launch_m2l_variant(int i, int nrhs, const int* act, int v) {
   }
 }
 
-// k_m2l_leaf: leaf M2L plus the band L2L from level Lf-1, whose 16-row blocks
-// coincide with the kernel's 16-sample chunks.  Needs a leaf level of at
-// least 8x8 boxes with a parent level below it that has M2L (>= 2), the band
-// form of that L2L, and the LDS of both stages within the limit.
-template <typename T>
-bool Engine::leaf_fuse_ok() const {
-  const int Lf = P_.L - 1;
-  if (Lf < 3) return false;
-  const InterpShape& sh = (sizeof(T) == 4 ? l2l32_ : l2l64_)[Lf - 1];
-  // kb <= 96: the kernel's register window
-  if (sh.ncb <= 0 || sh.kb <= 0 || sh.kb > P_.nsamp[Lf - 1] || sh.kb > 96) return false;
-  const size_t dyn = std::max<size_t>(16 * (size_t)sh.kb, 64 * kParKC) + 4 * (size_t)sh.kb;
-  const size_t lds = ((size_t)(kParSB * kParSB + 49) * kParKC + dyn) * sizeof(cplx<T>);
-  return lds <= kLdsLimit;
-}
-
-template <typename T>
-void Engine::launch_m2l_leaf(int nrhs, const int* act) {
-  const int Lf = P_.L - 1, S = P_.nsamp[Lf], Sp = P_.nsamp[Lf - 1], nb = 1 << Lf;
-  const InterpShape& sh = (sizeof(T) == 4 ? l2l32_ : l2l64_)[Lf - 1];
-  DevOp<T>& d = ops<T>();
-  const int nchunk = (S + kParKC - 1) / kParKC;
-  dim3 grid(nb * nb / (kParTS * kParTS) * nchunk, nrhs), blk(kBlock);
-  const size_t lds = (std::max<size_t>(16 * (size_t)sh.kb, 64 * kParKC) + 4 * (size_t)sh.kb) * sizeof(cplx<T>);
-  k_m2l_leaf<T><<<grid, blk, lds, stream_>>>(d.agm + lvl_off_[Lf], d.agl + lvl_off_[Lf], (long)lvl_size_[Lf],
-                                             d.trans[Lf], Lf, S, d.agl + lvl_off_[Lf - 1], (long)lvl_size_[Lf - 1],
-                                             Sp, d.band_l2l[Lf - 1], d.bs0_l2l[Lf - 1], sh.kb, d.shiftL[Lf - 1], act);
-}
-
 // Near field + L2P on the matrix cores (k_near_mfma), or L2P alone when
 // with_near is false (receiver back-projection).
 template <typename T, typename TI>
@@ -942,19 +963,22 @@ void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, con
   for (int i = L - 2; i >= 2; i--) launch_m2m<T>(i, nrhs, act);
   prof_end(KT_INTERP);
   const int kt = sizeof(T) == 4 ? KT_M2L32 : KT_M2L;
-  // with the fused leaf kernel the last L2L (level Lf-1 -> Lf) runs inside the
-  // leaf M2L, after the L2L passes above it
-  const bool fuse = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).leaf == 1 && leaf_fuse_ok<T>();
-  const int mtop = fuse ? Lf - 1 : Lf, ltop = fuse ? L - 3 : L - 2;
+  // FP32: from level `fuse` down, M2L and the L2L into the level are one kernel (tuning stage "leaf"):
+  // -1 every level from 3 on, 1 the leaf alone, 0 none
+  int fuse = L;
+  if constexpr (sizeof(T) == 4) {
+    const int leaf = tune(PREC_MIXED, nrhs).leaf;
+    if (!down16_.empty() && leaf != 0 && L > 3) fuse = leaf == 1 ? Lf : 3;
+  }
   prof_begin(kt);
-  launch_m2l<T>(2, mtop, nrhs, act);
+  launch_m2l<T>(2, std::min(fuse, L) - 1, nrhs, act);
   prof_end(kt);
   prof_begin(KT_INTERP, false);  // timed with the M2M launch set of this product
-  for (int i = 2; i <= ltop; i++) launch_l2l<T>(i, true, nrhs, act);
+  for (int i = 2; i + 1 < fuse && i <= L - 2; i++) launch_l2l<T>(i, true, nrhs, act);
   prof_end(KT_INTERP);
-  if (fuse) {
+  if (fuse < L) {
     prof_begin(kt, false);  // timed with the M2L launch set of this product
-    launch_m2l_leaf<T>(nrhs, act);
+    for (int i = fuse; i <= Lf; i++) launch_down16(i, nrhs, act);
     prof_end(kt);
   }
   near_blocks_ = launch_near<T, TI>(y, r, nrhs, act, true, -1, post);
@@ -1506,20 +1530,20 @@ void Engine::autotune_prec(int nrhs, int reps) {
     tu.l2l[i] = pick(
         5, [&](int k) { return kind_ok(sl[i], k); }, [&](int k) { launch_l2l<T>(i, true, nrhs, nullptr, k); });
   }
-  // fused leaf kernel against the best separate leaf M2L + last L2L
+  // downward pass: fused from level 3 on (-1), at the leaf (1), or separate (0)
   tu.leaf = -1;
-  if (leaf_fuse_ok<T>()) {
-    const int vm = tu.m2l[Lf], kl = tu.l2l[L - 2];
-    tu.leaf = pick(
-        2, [](int) { return true; },
-        [&](int f) {
-          if (f == 1) {
-            launch_m2l_leaf<T>(nrhs, nullptr);
-          } else {
-            launch_m2l<T>(Lf, Lf, nrhs, nullptr, vm);
-            launch_l2l<T>(L - 2, true, nrhs, nullptr, kl);
-          }
-        });
+  if constexpr (sizeof(T) == 4) {
+    if (!down16_.empty() && L > 3) {
+      const int c = pick(
+          3, [](int) { return true; },
+          [&](int f) {
+            const int fuse = f == 0 ? 3 : (f == 1 ? Lf : L);
+            launch_m2l<T>(2, fuse - 1, nrhs, nullptr);
+            for (int i = 2; i + 1 < fuse; i++) launch_l2l<T>(i, true, nrhs, nullptr);
+            for (int i = fuse; i < L; i++) launch_down16(i, nrhs, nullptr);
+          });
+      tu.leaf = c == 0 ? -1 : (c == 1 ? 1 : 0);
+    }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

@@ -778,8 +778,7 @@ __global__ void __launch_bounds__(kBlock) k_m2l_reg(const cplx<T>* __restrict__ 
 // LDS reads per thread: 36 + 49 for 108 complex multiply-adds.
 constexpr int kParTS = 8, kParSB = kParTS + 4, kParKC = 16;
 
-// Workgroup coordinates shared by k_m2l_par and k_m2l_leaf: 8x8 boxes
-// starting at Morton index m0 (corner X0, Y0), samples k0 .. k0+15.
+// Workgroup coordinates of k_m2l_par: 8x8 boxes starting at Morton index m0 (corner X0, Y0), samples k0 .. k0+15.
 struct ParBlock {
   int chunk, k0, X0, Y0;
   unsigned m0;
@@ -898,120 +897,6 @@ k_m2l_par(M2LSet<T> set, const int* __restrict__ act) {
   cplx<T>* out = L.l + rhs * L.st + (long)(B.m0 + 4 * morton2((unsigned)(pp & 3), (unsigned)(pp >> 2))) * S;
 #pragma unroll
   for (int c = 0; c < 4; c++) out[(long)c * S + B.k0 + kk] = acc[c];
-}
-
-// Leaf M2L fused with the last L2L (parent level lev-1 -> leaf level lev):
-// the k_m2l_par workgroup (4x4 parents, 16 samples = one 16-row block of the
-// L2L band matrix) also interpolates its parents' local expansions to the
-// children's samples on the matrix cores (as k_interp_band in L2L mode,
-// columns = the 64 children, window = the row block's KB parent samples
-// from s0v[chunk], mod Sp) and writes  local = translations + interpolation
-// once.  The separate L2L pass would read the parents again and read and
-// rewrite every leaf local after the M2L wrote it.  Dynamic LDS: the parent
-// window, max(16 KB, 1024) elements (later the 64 x 16 interpolated
-// locals), and the child shifts on it, 4 x KB.
-template <typename T>
-__global__ void __launch_bounds__(kBlock) k_m2l_leaf(const cplx<T>* __restrict__ agm, cplx<T>* __restrict__ agl,
-                                                     long st, const cplx<T>* __restrict__ trans, int lev, int S,
-                                                     const cplx<T>* __restrict__ par, long ps, int Sp,
-                                                     const T* __restrict__ AB, const int* __restrict__ s0v, int KB,
-                                                     const cplx<T>* __restrict__ shift, const int* __restrict__ act) {
-  // FP64: the translation streams its sources (par_translate_stream); the
-  // neighbourhood in registers would take 256 registers, one wave per SIMD
-  constexpr bool STREAM_LEAF = sizeof(T) == 8;
-  typedef typename Mfma<T>::v4 v4;
-  __shared__ cplx<T> src[kParSB * kParSB][kParKC];
-  __shared__ cplx<T> tr[49][kParKC];
-  extern __shared__ char smem_raw[];
-  cplx<T>* pw = reinterpret_cast<cplx<T>*>(smem_raw);  // [16 parents][KB]
-  cplx<T>* sw = pw + max(16 * KB, 64 * kParKC);         // [4 children][KB]
-  const int rhs = blockIdx.y;
-  if (rhs_off(act, rhs)) return;
-  const ParBlock B(S, xcd_block());
-  // the band rows of the window (the interpolation's A operand; no LDS
-  // needed), issued before the staging so their latency overlaps it
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  constexpr int KQ = 24;  // windows of up to 96 samples (the L2L band limit)
-  const int nkq = KB >> 2;
-  T a[KQ];
-  {
-    const T* ab = AB + (long)B.chunk * KB * 16;
-#pragma unroll
-    for (int q = 0; q < KQ; q++) a[q] = (q < nkq) ? ab[(4 * q + lk) * 16 + li] : (T)0;
-  }
-  m2l_stage<T, kParTS, kParKC>(src, tr, agm + rhs * st, trans, B.X0, B.Y0, B.k0, 1 << lev, S);
-  const int s0 = s0v[B.chunk];
-  const cplx<T>* pr = par + rhs * ps + (long)(B.m0 >> 2) * Sp;  // the tile's 16 parents, Morton order
-  // window element e = p * KB + jj (parent p, or child position p for the
-  // shifts), parent sample (s0 + jj) mod Sp; (p, jj) stepped, not divided
-  {
-    const int n = 20 * KB, dp = kBlock / KB, dq = kBlock - dp * KB;
-    int p = threadIdx.x / KB, jj = threadIdx.x - p * KB;
-    for (int e0 = threadIdx.x; e0 < n; e0 += 4 * kBlock) {
-      cplx<T> v[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int e = e0 + u * kBlock;
-        int j = s0 + jj;
-        if (j >= Sp) j -= Sp;
-        // unconditional loads (past n: a clamped, unused shift element), so v stays in registers
-        v[u] = e < 16 * KB ? pr[(long)p * Sp + j] : shift[min(p - 16, 3) * Sp + j];
-        jj += dq;
-        p += dp;
-        if (jj >= KB) {
-          jj -= KB;
-          p++;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int e = e0 + u * kBlock;
-        if (e < 16 * KB)
-          pw[e] = v[u];
-        else if (e < n)
-          sw[e - 16 * KB] = v[u];
-      }
-    }
-  }
-  __syncthreads();
-  const int tid = threadIdx.x, kk = tid % kParKC, pp = tid / kParKC;
-  // interpolation first (the 36 sources of the translation phase are loaded
-  // only after it, so the two phases do not hold registers at the same time):
-  // wave w owns columns 16w .. 16w+15 (children 16w + i, i.e.
-  // parent 4w + i/4, child position i%4); lane (li, lk) feeds column li at
-  // window sample 4q + lk and receives rows Mfma::row(lk, q) at sample li
-  const int w = tid >> 6;
-  const cplx<T>* pcol = pw + (4 * w + (li >> 2)) * KB;
-  const cplx<T>* scol = sw + (li & 3) * KB;
-  v4 cr = v4{0, 0, 0, 0}, ci = v4{0, 0, 0, 0};
-#pragma unroll
-  for (int q = 0; q < KQ; q++) {
-    if (q < nkq) {
-      const int jj = 4 * q + lk;
-      const cplx<T> bv = cmul(scol[jj], pcol[jj]);
-      cr = Mfma<T>::mac(bv.x, a[q], cr);
-      ci = Mfma<T>::mac(bv.y, a[q], ci);
-    }
-  }
-  __syncthreads();  // the parent window is no longer read: it takes the result
-  cplx<T>* ll = pw;  // [64 children][16 samples]
-#pragma unroll
-  for (int q = 0; q < 4; q++) ll[(16 * w + Mfma<T>::row(lk, q)) * kParKC + li] = mkc<T>(cr[q], ci[q]);
-  __syncthreads();
-  cplx<T> acc[4];
-  if constexpr (STREAM_LEAF) {
-    par_translate_stream<T>(src, tr, 2 * (pp & 3), 2 * (pp >> 2), kk, acc);
-  } else {
-    cplx<T> sv[6][6];
-    par_load<T>(src, 2 * (pp & 3), 2 * (pp >> 2), kk, sv);
-    par_translate<T>(tr, kk, sv, acc);
-  }
-  const unsigned pm = morton2((unsigned)(pp & 3), (unsigned)(pp >> 2));
-  if (B.k0 + kk < S) {
-    cplx<T>* out = agl + rhs * st + (long)(B.m0 + 4 * pm) * S;
-#pragma unroll
-    for (int c = 0; c < 4; c++) out[(long)c * S + B.k0 + kk] = cadd(acc[c], ll[(4 * pm + c) * kParKC + kk]);
-  }
 }
 
 // P2M on the matrix cores: agm[box][k] = sum_n coeffT[n][k] y[box*64+n] for a
