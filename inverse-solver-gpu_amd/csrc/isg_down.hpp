@@ -1,4 +1,4 @@
-// isg_down_h16.hpp -- downward pass of one level of the FP32 operator: its
+// isg_down.hpp -- downward pass of one level of the FP32 operator: its
 // translations (M2L) and the interpolation of the parents' locals (L2L) in one
 // kernel, the interpolation on the FP16 matrix cores with split operands.
 //
@@ -80,8 +80,8 @@ __device__ __forceinline__ zf down_load(__amdgpu_buffer_rsrc_t rs, unsigned off)
 }
 
 // The 27 translation operators of child position (CX, CY) at one sample.
-template <int CX, int CY>
-__device__ __forceinline__ void down_load_t(const zf* __restrict__ trans, int S, int k, zf (&t)[kDownFar]) {
+template <int CX, int CY, typename T>
+__device__ __forceinline__ void down_load_t(const cplx<T>* __restrict__ trans, int S, int k, cplx<T> (&t)[kDownFar]) {
   int j = 0;
 #pragma unroll
   for (int dy = -2 - CY; dy <= 3 - CY; dy++)
@@ -93,28 +93,31 @@ __device__ __forceinline__ void down_load_t(const zf* __restrict__ trans, int S,
 // acc[i] += sum over far offsets of T * source for child position (CX, CY) of the
 // four parents i of a 2 x 2 block: their sources lie in 8 x 8 boxes, each read
 // once (s points at this lane's sample of box (-2, -2) from the block's corner).
-// A row of sources is read while the previous one is multiplied (left to
-// itself the compiler reads two at a time and waits for them); row holds the
-// first one.
-template <int CX, int CY>
-__device__ __forceinline__ void down_m2l(const zf* __restrict__ s, const zf (&t)[kDownFar], const zf (&first)[8],
-                                         zf (&acc)[4]) {
-  zf row[2][8];
+// W sources of a row are read while the previous ones are multiplied (left to
+// itself the compiler reads two at a time and waits for them); first holds the
+// first W.
+template <int CX, int CY, int W, typename T>
+__device__ __forceinline__ void down_m2l(const cplx<T>* __restrict__ s, const cplx<T> (&t)[kDownFar],
+                                         const cplx<T> (&first)[W], cplx<T> (&acc)[4]) {
+  constexpr int H = 8 / W;  // groups per row
+  cplx<T> grp[2][W];
 #pragma unroll
-  for (int x = 0; x < 8; x++) row[0][x] = first[x];
+  for (int x = 0; x < W; x++) grp[0][x] = first[x];
 #pragma unroll
-  for (int y = 0; y < 8; y++) {  // source (sx, sy) = (x - 2, y - 2)
-    if (y + 1 < 8) {
+  for (int h = 0; h < 8 * H; h++) {  // sources (sx, sy) = (x0 + x - 2, y - 2)
+    const int y = h / H, x0 = W * (h % H);
+    if (h + 1 < 8 * H) {
 #pragma unroll
-      for (int x = 0; x < 8; x++) row[(y + 1) & 1][x] = s[((y + 1) * kDownSB + x) * kDownKC];
+      for (int x = 0; x < W; x++)
+        grp[(h + 1) & 1][x] = s[((h + 1) / H * kDownSB + W * ((h + 1) % H) + x) * kDownKC];
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int x = 0; x < 8; x++) {
-      const zf v = row[y & 1][x];
+    for (int x = 0; x < W; x++) {
+      const cplx<T> v = grp[h & 1][x];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int ax = x - 2 - 2 * (i & 1), ay = y - 2 - 2 * (i >> 1);  // from the parent's first child
+        const int ax = x0 + x - 2 - 2 * (i & 1), ay = y - 2 - 2 * (i >> 1);  // from the parent's first child
         if (ax < -2 || ax > 3 || ay < -2 || ay > 3) continue;
         const int dx = ax - CX, dy = ay - CY;
         if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) continue;  // near
@@ -284,10 +287,10 @@ k_down_h16(const zf* __restrict__ agm, zf* __restrict__ agl, long st, const zf* 
 #pragma unroll
     for (int i = 0; i < 4; i++) acc[i] = mkc<float>(0.f, 0.f);
     switch (w) {
-      case 0: down_m2l<0, 0>(s, t, first, acc); break;
-      case 1: down_m2l<1, 0>(s, t, first, acc); break;
-      case 2: down_m2l<0, 1>(s, t, first, acc); break;
-      default: down_m2l<1, 1>(s, t, first, acc); break;
+      case 0: down_m2l<0, 0, 8>(s, t, first, acc); break;
+      case 1: down_m2l<1, 0, 8>(s, t, first, acc); break;
+      case 2: down_m2l<0, 1, 8>(s, t, first, acc); break;
+      default: down_m2l<1, 1, 8>(s, t, first, acc); break;
     }
     if (store) {
       char* o = reinterpret_cast<char*>(agl + (long)r * st);
@@ -300,6 +303,131 @@ k_down_h16(const zf* __restrict__ agm, zf* __restrict__ agl, long st, const zf* 
     }
     if (!more) break;
     r = rn;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same downward step in FP64: interpolation on v_mfma_f64_16x16x4 with the
+// real band block and the parents shifted as they are read (a complex table
+// would take half as many matrix products again, and FP64 products share the
+// vector ALUs' time).  Per workgroup the band block, the child shifts and, in
+// registers, the 27 operators are loaded once; per right-hand side the source
+// boxes and the parents' windows go to LDS.  Wave w owns child position w; the
+// rows of the matrix product are permuted so that a lane (li, lk) receives
+// parents 4 lk .. +3, a 2 x 2 block, as in k_down_h16.
+// FP64 work bounds it (an FP64 product of this chip's vector or matrix units
+// either way): 1024 px x 64 right-hand sides, M2L and L2L of levels 2 .. 7, 3140
+// us as separate kernels (M2L 1100, L2L 2040), 1940 here, of which about 1000 is
+// arithmetic at the rate of a large matrix product; 512 px x 16, 195 -> 168 us.
+// Grid (tiles * ceil(S / 16), ceil(nrhs / per)); level >= 3; KB <= kDownK.
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __restrict__ trans, int lev, int S,
+         const zd* __restrict__ par, long ps, int Sp, const double* __restrict__ AB, const int* __restrict__ s0v, int KB,
+         const zd* __restrict__ shift, int nrhs, int per, const int* __restrict__ act) {
+  typedef Mfma<double>::v4 v4;
+  constexpr int NS = kDownSB * kDownSB * kDownKC, NW = 16 * kDownK / kBlock, WP = kDownK + 1;
+  __shared__ zd src[NS], win[16 * WP], sh[4 * kDownK];  // win[parent][window]
+  __shared__ double ab[kDownK * 16];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  // active right-hand sides of the group, as bits
+  const int rg = blockIdx.y * per;
+  unsigned live = 0;
+  for (int q = 0; q < per && rg + q < nrhs; q++) live |= (rhs_off(act, rg + q) ? 0u : 1u) << q;
+  live = __builtin_amdgcn_readfirstlane(live);
+  if (!live) return;
+  const int nb = 1 << lev, nchunk = (S + kDownKC - 1) / kDownKC;
+  const int lb = xcd_block(), tile = lb / nchunk, chunk = lb - tile * nchunk;
+  const int k0 = chunk * kDownKC;
+  const unsigned m0 = (unsigned)tile * kDownTS * kDownTS;
+  const int X0 = (int)compact2(m0), Y0 = (int)compact2(m0 >> 1);
+  // ---- once per workgroup
+  const int ks = min(k0 + (tid & 15), S - 1);  // (samples past S are computed and not stored)
+  unsigned soff[9];  // byte offsets; past the end (zeros) for boxes outside the grid
+#pragma unroll
+  for (int u = 0; u < 9; u++) {
+    const int b = (tid >> 4) + 16 * u, bx = X0 - 2 + b % kDownSB, by = Y0 - 2 + b / kDownSB;
+    const bool ok = bx >= 0 && by >= 0 && bx < nb && by < nb;
+    soff[u] = ok ? (morton2(bx, by) * S + ks) * (unsigned)sizeof(zd) : 0xffffff00u;
+  }
+  const int s0 = s0v[chunk];
+  unsigned woff[NW], wdst[NW];  // window element e = p KB + jj of parent p
+#pragma unroll
+  for (int u = 0; u < NW; u++) {
+    const int e = min(tid + kBlock * u, 16 * KB - 1), p = e / KB, jj = e - p * KB;
+    int j = s0 + jj;
+    if (j >= Sp) j -= Sp;
+    woff[u] = (((m0 >> 2) + p) * Sp + j) * (unsigned)sizeof(zd);
+    wdst[u] = p * WP + jj;
+  }
+  for (int e = tid; e < 4 * KB; e += kBlock) {
+    const int c = e / KB;
+    int j = s0 + e - c * KB;
+    if (j >= Sp) j -= Sp;
+    sh[e] = shift[c * Sp + j];
+  }
+  for (int e = tid; e < 16 * KB; e += kBlock) ab[e] = AB[(long)chunk * KB * 16 + e];
+  zd t[kDownFar];
+  const int kt = min(k0 + li, S - 1);
+  switch (w) {
+    case 0: down_load_t<0, 0>(trans, S, kt, t); break;
+    case 1: down_load_t<1, 0>(trans, S, kt, t); break;
+    case 2: down_load_t<0, 1>(trans, S, kt, t); break;
+    default: down_load_t<1, 1>(trans, S, kt, t); break;
+  }
+  const unsigned mbytes = (unsigned)nb * nb * S * (unsigned)sizeof(zd), pbytes = (unsigned)nb * nb / 4 * Sp * (unsigned)sizeof(zd);
+  const unsigned ooff = ((m0 + 16 * lk + w) * S + k0 + li) * (unsigned)sizeof(zd), ostep = 4 * S * (unsigned)sizeof(zd);
+  const bool store = k0 + li < S;
+  const zd* wrow = win + (4 * (li & 3) + (li >> 2)) * WP + lk;  // this lane's row of the product
+  const zd* srow = sh + w * KB + lk;
+  const double* arow = ab + lk * 16 + li;
+  const int nkq = KB >> 2;
+  while (live) {
+    const int r = rg + __builtin_ctz(live);
+    live &= live - 1;
+    {
+      const __amdgpu_buffer_rsrc_t a = down_rsrc(agm + (long)r * st, mbytes), p = down_rsrc(par + (long)r * ps, pbytes);
+      zd sv[9], wv[NW];
+#pragma unroll
+      for (int u = 0; u < 9; u++)
+        sv[u] = __builtin_bit_cast(zd, __builtin_amdgcn_raw_buffer_load_b128(a, (int)soff[u], 0, 0));
+#pragma unroll
+      for (int u = 0; u < NW; u++)
+        wv[u] = __builtin_bit_cast(zd, __builtin_amdgcn_raw_buffer_load_b128(p, (int)woff[u], 0, 0));
+      __syncthreads();  // the previous right-hand side's sources are no longer read
+#pragma unroll
+      for (int u = 0; u < 9; u++) src[tid + kBlock * u] = sv[u];
+#pragma unroll
+      for (int u = 0; u < NW; u++) win[wdst[u]] = wv[u];  // (the clamped last ones repeat one element)
+    }
+    __syncthreads();
+    // ---- interpolation: rows = parents, columns = samples
+    v4 cr = v4{0, 0, 0, 0}, ci = v4{0, 0, 0, 0};
+#pragma unroll 4
+    for (int q = 0; q < nkq; q++) {
+      const zd v = cmul(srow[4 * q], wrow[4 * q]);
+      const double a = arow[64 * q];
+      cr = Mfma<double>::mac(v.x, a, cr);
+      ci = Mfma<double>::mac(v.y, a, ci);
+    }
+    // ---- translations
+    zd acc[4], first[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = mkc<double>(cr[i], ci[i]);
+    const zd* s = src + (4 * (lk >> 1) * kDownSB + 4 * (lk & 1)) * kDownKC + li;
+#pragma unroll
+    for (int x = 0; x < 4; x++) first[x] = s[x * kDownKC];
+    switch (w) {
+      case 0: down_m2l<0, 0, 4>(s, t, first, acc); break;
+      case 1: down_m2l<1, 0, 4>(s, t, first, acc); break;
+      case 2: down_m2l<0, 1, 4>(s, t, first, acc); break;
+      default: down_m2l<1, 1, 4>(s, t, first, acc); break;
+    }
+    if (store) {
+      char* o = reinterpret_cast<char*>(agl + (long)r * st);
+#pragma unroll
+      for (int i = 0; i < 4; i++) *reinterpret_cast<zd*>(o + (ooff + i * ostep)) = acc[i];
+    }
   }
 }
 

@@ -13,7 +13,7 @@
 
 #include <rocblas/rocblas.h>
 
-#include "isg_down_h16.hpp"
+#include "isg_down.hpp"
 #include "isg_kernels.hpp"
 #include "isg_near_h16.hpp"
 #include "isg_near_sym.hpp"
@@ -317,7 +317,7 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
   rxaI_ = up_i(P_.rxaI);
   plan_interp(op64_, m2m64_, l2l64_);
   if (has32_) plan_interp(op32_, m2m32_, l2l32_);
-  if (has32_) build_down16();
+  build_down();
   for (auto& row : tune_)
     for (auto& t : row) {
       t.m2l.assign(P_.L, -1);
@@ -512,10 +512,11 @@ void Engine::build_split16() {
   ISG_HIP(hipStreamSynchronize(stream_));
 }
 
-// Tables of k_down_h16 for levels 3 .. leaf: the band blocks of each level's
-// anterpolator with the four child shifts folded in, split into FP16.  Left
-// empty (separate M2L and L2L kernels) if some level's window exceeds 96.
-void Engine::build_down16() {
+// Tables of the fused downward kernels for levels 3 .. leaf: the band blocks of
+// each level's anterpolator (k_down64), and for the FP32 operator those with the
+// four child shifts folded in, split into FP16 (k_down_h16).  Left empty
+// (separate M2L and L2L kernels) if some level's window exceeds 96.
+void Engine::build_down() {
   if (!ok()) return;
   const int L = P_.L, na = 2 * cfg_.plan.ninter;
   std::vector<DownLevel> lv(L);
@@ -524,40 +525,60 @@ void Engine::build_down16() {
   for (int i = 3; i < L; i++) {
     const int S = P_.nsamp[i], Sp = P_.nsamp[i - 1], nrb = (S + 15) / 16;
     const int kb = build_band(S, Sp, na, P_.anterp0[i], P_.anterpT[i], kDownK, AB, s0);
-    // (the kernel's offsets within a level of one right-hand side are 32 bits wide)
-    if (kb == 0 || lvl_size_[i] * sizeof(zf) >= 0xffffff00u) return;
-    double m = 0;
-    for (double v : AB) m = std::max(m, std::fabs(v));
+    // (the kernels' offsets within a level of one right-hand side are 32 bits wide)
+    if (kb == 0 || lvl_size_[i] * sizeof(zd) >= 0xffffff00u) return;
     DownLevel& d = lv[i];
     d.kb = kb;
-    d.ec = h16_scale_exp((float)m);
-    d.tab = dalloc((size_t)nrb * 4 * kDownFrag * 16);
     d.s0 = (int*)dalloc(s0.size() * sizeof(int));
-    double* ab = nullptr;
+    d.ab = (double*)dalloc(AB.size() * sizeof(double));
+    if (has32_) d.tab = dalloc((size_t)nrb * 4 * kDownFrag * 16);
     if (!ok()) return;
-    ISG_HIP(hipMalloc((void**)&ab, AB.size() * sizeof(double)));
-    if (!ok()) return;
-    ISG_HIP(hipMemcpy(ab, AB.data(), AB.size() * sizeof(double), hipMemcpyHostToDevice));
+    ISG_HIP(hipMemcpy(d.ab, AB.data(), AB.size() * sizeof(double), hipMemcpyHostToDevice));
     ISG_HIP(hipMemcpy(d.s0, s0.data(), s0.size() * sizeof(int), hipMemcpyHostToDevice));
-    k_split_l2l<<<nblocks((long)nrb * 4 * kDownG * 16), kBlock, 0, stream_>>>(ab, d.s0, kb, op64_.shiftL[i - 1], Sp, nrb,
-                                                                             d.ec, (v8h*)d.tab);
-    ISG_HIP(hipGetLastError());
-    ISG_HIP(hipStreamSynchronize(stream_));
-    (void)hipFree(ab);
+    if (has32_) {
+      double m = 0;
+      for (double v : AB) m = std::max(m, std::fabs(v));
+      d.ec = h16_scale_exp((float)m);
+      k_split_l2l<<<nblocks((long)nrb * 4 * kDownG * 16), kBlock, 0, stream_>>>(d.ab, d.s0, kb, op64_.shiftL[i - 1], Sp,
+                                                                               nrb, d.ec, (v8h*)d.tab);
+    }
   }
-  down16_ = lv;
+  ISG_HIP(hipGetLastError());
+  ISG_HIP(hipStreamSynchronize(stream_));
+  if (L > 3) down_ = lv;
 }
 
-// M2L of level i and the L2L into it (FP32 operator).  Right-hand sides per
-// workgroup: as many as leave four workgroups per CU, 8 at most.
-void Engine::launch_down16(int i, int nrhs, const int* act) {
+// First level whose M2L and L2L are one kernel (L: none), for a choice of the
+// tuning stage "leaf": 0 none, 1 the leaf alone, -1 the rule.  A workgroup takes
+// 64 boxes and the levels above the leaf have few of those, each with many
+// sample chunks that repeat the set-up, so a small product fuses the leaf only.
+// All levels / the leaf / none, us a product: FP64 256 px x 1 70 / 64 / 64, x 4
+// 82 / 76 / 89, x 8 99 / 100 / 125, 512 px x 1 95 / 87 / 88, x 4 149 / 161 / 158,
+// x 16 393 / 409 / 428; FP32 256 px x 1 58 / 55 / 54, x 7 72 / 72 / 80, 512 px x 1
+// 72 / 68 / 72.
+int Engine::fuse_level(int choice, int nrhs) const {
+  if (down_.empty() || choice == 0) return P_.L;
+  return choice == 1 || (long)P_.B * nrhs < 7168 ? P_.L - 1 : 3;
+}
+
+// M2L of level i and the L2L into it.  Right-hand sides per workgroup: as many
+// as leave four workgroups per CU, 8 at most.
+template <typename T>
+void Engine::launch_down(int i, int nrhs, const int* act) {
   const int S = P_.nsamp[i], nb = 1 << i, blocks = nb * nb / (kDownTS * kDownTS) * ((S + kDownKC - 1) / kDownKC);
   const int per = (int)std::min<long>(8, std::max<long>(1, (long)blocks * nrhs / 1024));
-  const DownLevel& d = down16_[i];
-  DevOp<float>& o = op32_;
-  k_down_h16<<<dim3(blocks, (nrhs + per - 1) / per), dim3(kBlock), 0, stream_>>>(
-      o.agm + lvl_off_[i], o.agl + lvl_off_[i], (long)lvl_size_[i], o.trans[i], i, S, o.agl + lvl_off_[i - 1],
-      (long)lvl_size_[i - 1], P_.nsamp[i - 1], (const v8h*)d.tab, d.s0, d.kb, d.ec, nrhs, per, act);
+  const DownLevel& d = down_[i];
+  DevOp<T>& o = ops<T>();
+  const dim3 grid(blocks, (nrhs + per - 1) / per), blk(kBlock);
+  const cplx<T>*m = o.agm + lvl_off_[i], *par = o.agl + lvl_off_[i - 1];
+  cplx<T>* l = o.agl + lvl_off_[i];
+  const long st = (long)lvl_size_[i], ps = (long)lvl_size_[i - 1];
+  if constexpr (sizeof(T) == 4)
+    k_down_h16<<<grid, blk, 0, stream_>>>(m, l, st, o.trans[i], i, S, par, ps, P_.nsamp[i - 1], (const v8h*)d.tab, d.s0,
+                                          d.kb, d.ec, nrhs, per, act);
+  else
+    k_down64<<<grid, blk, 0, stream_>>>(m, l, st, o.trans[i], i, S, par, ps, P_.nsamp[i - 1], d.ab, d.s0,
+                                                       d.kb, o.shiftL[i - 1], nrhs, per, act);
 }
 
 // ------------------------------------------------------- interpolation plan
@@ -963,13 +984,7 @@ void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, con
   for (int i = L - 2; i >= 2; i--) launch_m2m<T>(i, nrhs, act);
   prof_end(KT_INTERP);
   const int kt = sizeof(T) == 4 ? KT_M2L32 : KT_M2L;
-  // FP32: from level `fuse` down, M2L and the L2L into the level are one kernel (tuning stage "leaf"):
-  // -1 every level from 3 on, 1 the leaf alone, 0 none
-  int fuse = L;
-  if constexpr (sizeof(T) == 4) {
-    const int leaf = tune(PREC_MIXED, nrhs).leaf;
-    if (!down16_.empty() && leaf != 0 && L > 3) fuse = leaf == 1 ? Lf : 3;
-  }
+  const int fuse = fuse_level(tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).leaf, nrhs);
   prof_begin(kt);
   launch_m2l<T>(2, std::min(fuse, L) - 1, nrhs, act);
   prof_end(kt);
@@ -978,7 +993,7 @@ void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, con
   prof_end(KT_INTERP);
   if (fuse < L) {
     prof_begin(kt, false);  // timed with the M2L launch set of this product
-    for (int i = fuse; i <= Lf; i++) launch_down16(i, nrhs, act);
+    for (int i = fuse; i <= Lf; i++) launch_down<T>(i, nrhs, act);
     prof_end(kt);
   }
   near_blocks_ = launch_near<T, TI>(y, r, nrhs, act, true, -1, post);
@@ -1530,21 +1545,18 @@ void Engine::autotune_prec(int nrhs, int reps) {
     tu.l2l[i] = pick(
         5, [&](int k) { return kind_ok(sl[i], k); }, [&](int k) { launch_l2l<T>(i, true, nrhs, nullptr, k); });
   }
-  // downward pass: fused from level 3 on (-1), at the leaf (1), or separate (0)
+  // downward pass: fused by the built-in rule (-1), at the leaf (1), or separate (0)
   tu.leaf = -1;
-  if constexpr (sizeof(T) == 4) {
-    if (!down16_.empty() && L > 3) {
-      const int c = pick(
-          3, [](int) { return true; },
-          [&](int f) {
-            const int fuse = f == 0 ? 3 : (f == 1 ? Lf : L);
-            launch_m2l<T>(2, fuse - 1, nrhs, nullptr);
-            for (int i = 2; i + 1 < fuse; i++) launch_l2l<T>(i, true, nrhs, nullptr);
-            for (int i = fuse; i < L; i++) launch_down16(i, nrhs, nullptr);
-          });
-      tu.leaf = c == 0 ? -1 : (c == 1 ? 1 : 0);
-    }
-  }
+  if (!down_.empty())
+    tu.leaf = pick(
+                  3, [](int) { return true; },
+                  [&](int f) {
+                    const int fuse = fuse_level(f - 1, nrhs);
+                    launch_m2l<T>(2, std::min(fuse, L) - 1, nrhs, nullptr);
+                    for (int i = 2; i + 1 < fuse; i++) launch_l2l<T>(i, true, nrhs, nullptr);
+                    for (int i = fuse; i < L; i++) launch_down<T>(i, nrhs, nullptr);
+                  }) -
+              1;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   ISG_HIP(hipGetLastError());

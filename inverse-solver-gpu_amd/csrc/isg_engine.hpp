@@ -156,7 +156,7 @@ class Engine {
   enum { ST_NEAR = 0, ST_P2M = 1, ST_M2L = 2, ST_M2M = 3, ST_L2L = 4, ST_LEAF = 5, ST_COUNT = 6 };
   struct Tuning {
     int near_nb = -1, p2m_nb = -1;
-    int leaf = -1;  // FP32: M2L and the L2L into a level as one kernel (k_down_h16): -1 levels >= 3, 1 the leaf, 0 none
+    int leaf = -1;  // M2L and the L2L into a level as one kernel (k_down_h16, k_down64): -1 by rule, 1 the leaf, 0 none
     std::vector<int> m2l, m2m, l2l;
   };
   static int batch_class(int nrhs) { return nrhs >= 16 ? 1 : 0; }
@@ -198,7 +198,7 @@ class Engine {
   void plan_interp(DevOp<T>& d, std::vector<InterpShape>& m2m, std::vector<InterpShape>& l2l);
   // split-FP16 tables of the FP32 operator (k_near_h16, k_p2m_h16)
   void build_split16();
-  void build_down16();
+  void build_down();
   // operator with tables / multipoles of type T on vectors of type TI
   template <typename T, typename TI>
   void apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, const NearPost<TI>* post = nullptr);
@@ -214,7 +214,9 @@ class Engine {
   void launch_m2l(int lo, int hi, int nrhs, const int* act, int force = -1);
   template <typename T>
   void launch_m2l_variant(int i, int nrhs, const int* act, int v);
-  void launch_down16(int i, int nrhs, const int* act);
+  int fuse_level(int choice, int nrhs) const;
+  template <typename T>
+  void launch_down(int i, int nrhs, const int* act);
   template <typename T, typename TI>
   // returns the number of workgroups per right-hand side (partial sums of a post step)
   int launch_near(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, bool with_near, int force = -1,
@@ -275,13 +277,15 @@ class Engine {
   // k_p2m_h16 table ([2][4][4][16 ceil(S / 16)] groups of 8 FP16; null for S > 96) and its exponent
   void* p2m16_ = nullptr;
   int p2m16_ec_ = 0;
-  // k_down_h16: per level (3 .. leaf) its split table, window starts and length, scale exponent
+  // fused downward kernels: per level (3 .. leaf) the band blocks, their window
+  // starts and length, and the FP32 operator's split table with its scale exponent
   struct DownLevel {
+    double* ab = nullptr;
     void* tab = nullptr;
     int* s0 = nullptr;
     int kb = 0, ec = 0;
   };
-  std::vector<DownLevel> down16_;  // empty: not available
+  std::vector<DownLevel> down_;  // empty: not available
   std::vector<InterpShape> m2m64_, l2l64_, m2m32_, l2l32_;  // per parent level
   std::vector<int*> interp0_, anterp0_;
   int* rx0_ = nullptr;
