@@ -116,4 +116,31 @@ struct NearPost {
   double2* part = nullptr;
 };
 
+// Scalars of one BiCGSTAB system, on the device.
+struct BiState {
+  zd rho, rho1, alpha, omega, beta;
+  double bnrm, err, tol;
+  int iter, status, active, first;
+};
+
+// What P2M does with its input vector while loading it (vectors of type V):
+//   mode 1  y = prep(r)                                  (r: the iterate)
+//   mode 2  p = r + beta (p - omega v), y = prep(p)      (p = r in the first iteration)
+//   mode 3  alpha = rho / <r~,v> from the near field's partials, s = r - alpha v, y = prep(s)
+// Modes 2 and 3 store p (mode 3: s, through the same pointer) and y.
+template <typename V>
+struct P2mStep {
+  int mode = 0;
+  const cplx<V>* r = nullptr;
+  const cplx<V>* v = nullptr;
+  cplx<V>* p = nullptr;
+  cplx<V>* y = nullptr;
+  const zd* g = nullptr;
+  long gs = 0;
+  int herm = 0;
+  BiState* st = nullptr;
+  const double2* part = nullptr;  // mode 3: nblk partial sums per system
+  int nblk = 0;
+};
+
 }  // namespace isg

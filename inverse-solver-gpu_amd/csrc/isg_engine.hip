@@ -659,7 +659,7 @@ int Engine::interp_kind(const InterpShape& sh, int np, int nrhs) const {
 // --------------------------------------------------------------- launches
 // leaf radiation patterns on the matrix cores
 template <typename T, typename TI>
-void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, const NearPost<TI>* prep) {
+void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, const P2mStep<TI>* step) {
   const int Lf = P_.L - 1, S = P_.nsamp[Lf], B = P_.B;
   const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).p2m_nb;
   // built-in rule: 32-box tiles once they fill the chip, else 16 (64 px, one system: 12.9 -> 9.6 us)
@@ -667,13 +667,17 @@ void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
   DevOp<T>& d = ops<T>();
   cplx<T>* out = d.agm + lvl_off_[Lf];
   long as = (long)lvl_size_[Lf];
+  const int mode = step ? step->mode : 0;
+  const P2mStep<TI> st = step ? *step : P2mStep<TI>();
+  const dim3 blk(kBlock);
   if (nb == kNearSplit) {
     // split-FP16 P2M: FP32 operator on FP32 vectors, 32-box tiles of two
     // right-hand sides (below 4 the workgroups are few and half idle)
     if constexpr (sizeof(T) == 4 && sizeof(TI) == 4) {
-      if (!prep && B % 32 == 0 && p2m16_ && (nrhs >= 4 || force == kNearSplit)) {
-        dim3 grid(B / 32, (nrhs + 1) / 2), blk(kBlock);
-        k_p2m_h16<<<grid, blk, 0, stream_>>>(y, P_.N, out, as, (const v8h*)p2m16_, p2m16_ec_, S, nrhs, act);
+      if (mode != 1 && B % 32 == 0 && p2m16_ && (nrhs >= 4 || force == kNearSplit)) {
+        dim3 grid(B / 32, (nrhs + 1) / 2);
+        auto k = mode == 0 ? k_p2m_h16<0> : (mode == 2 ? k_p2m_h16<2> : k_p2m_h16<3>);
+        k<<<grid, blk, 0, stream_>>>(y, P_.N, out, as, (const v8h*)p2m16_, p2m16_ec_, S, nrhs, act, st);
         return;
       }
     }
@@ -681,26 +685,23 @@ void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
   }
   if (nb == 64 && sizeof(T) != 4) nb = 32;  // 64-box tiles: FP32 only (LDS)
   if (B % nb != 0) nb = 16;
-  dim3 grid(B / nb, nrhs), blk(kBlock);
-  if (prep) {  // residual check: y is the iterate, contrast-weighted while loading (FP64 only)
-    if constexpr (sizeof(T) == 8 && sizeof(TI) == 8) {
-      if (nb == 32)
-        k_p2m_mfma<T, TI, 32, true><<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act, prep->g, prep->gs,
-                                                               prep->herm);
-      else
-        k_p2m_mfma<T, TI, 16, true><<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act, prep->g, prep->gs,
-                                                               prep->herm);
-    } else {
-      set_error("P2M: contrast weighting on load is FP64 only");
-    }
-    return;
+  const dim3 grid(B / nb, nrhs);
+  auto go = [&](auto k) { k<<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act, st); };
+  auto tile = [&](auto m) {
+    constexpr int M = decltype(m)::value;
+    if constexpr (sizeof(T) == 4)
+      if (nb == 64) return go(k_p2m_mfma<T, TI, 64, M>);
+    if (nb == 32) return go(k_p2m_mfma<T, TI, 32, M>);
+    go(k_p2m_mfma<T, TI, 16, M>);
+  };
+  if (mode == 0) return tile(std::integral_constant<int, 0>());
+  if constexpr (sizeof(T) == sizeof(TI)) {
+    // the solver's vector steps; contrast weighting alone (mode 1) serves the FP64 residual check
+    if (mode == 2) return tile(std::integral_constant<int, 2>());
+    if (mode == 3) return tile(std::integral_constant<int, 3>());
+    if constexpr (sizeof(T) == 8) return tile(std::integral_constant<int, 1>());
   }
-  if (nb == 64) {
-    if constexpr (sizeof(T) == 4) k_p2m_mfma<T, TI, 64><<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act);
-  } else if (nb == 32)
-    k_p2m_mfma<T, TI, 32><<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act);
-  else
-    k_p2m_mfma<T, TI, 16><<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act);
+  set_error("P2M: no kernel for this step on vectors of this type");
 }
 
 // child level i+1 -> parent level i
@@ -974,11 +975,21 @@ int Engine::launch_near(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act
 // P2M, M2M up to level 2, M2L on levels 2..leaf, L2L down, then near field
 // and L2P together.
 template <typename T, typename TI>
-void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, const NearPost<TI>* post) {
+void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, const NearPost<TI>* post,
+                   const P2mStep<TI>* step) {
   const int L = P_.L, Lf = L - 1;
   // post mode 3 (residual check): y is the iterate, weighted while P2M and the near field load it
+  P2mStep<TI> weight;
+  if (post && post->mode == 3) {
+    weight.mode = 1;
+    weight.r = y;
+    weight.g = post->g;
+    weight.gs = post->gs;
+    weight.herm = post->herm;
+    step = &weight;
+  }
   prof_begin(KT_P2M);
-  launch_p2m<T, TI>(y, nrhs, act, -1, (post && post->mode == 3) ? post : nullptr);
+  launch_p2m<T, TI>(y, nrhs, act, -1, step);
   prof_end(KT_P2M);
   prof_begin(KT_INTERP);
   for (int i = L - 2; i >= 2; i--) launch_m2m<T>(i, nrhs, act);
@@ -1011,15 +1022,16 @@ cplx<V>* Engine::vb(int k) {
 
 // FP32 vectors always go with the FP32 operator; FP64 vectors with either
 template <typename V>
-void Engine::apply_vec(const cplx<V>* y, cplx<V>* r, int nrhs, const int* act, int prec, const NearPost<V>* post) {
+void Engine::apply_vec(const cplx<V>* y, cplx<V>* r, int nrhs, const int* act, int prec, const NearPost<V>* post,
+                       const P2mStep<V>* step) {
   if (!ok()) return;
   if constexpr (sizeof(V) == 4) {
-    apply<float, float>(y, r, nrhs, act, post);
+    apply<float, float>(y, r, nrhs, act, post, step);
   } else {
     if (prec == PREC_MIXED && has32_)
-      apply<float, double>(y, r, nrhs, act, post);
+      apply<float, double>(y, r, nrhs, act, post, step);
     else
-      apply<double, double>(y, r, nrhs, act, post);
+      apply<double, double>(y, r, nrhs, act, post, step);
   }
   ISG_HIP(hipGetLastError());
 }
@@ -1210,31 +1222,44 @@ void Engine::bicgs_body(zd* x, const zd* g, long gs, bool herm, int nrhs, int pr
   cplx<V>*r = vb<V>(V_R), *rt = vb<V>(V_RT), *p = vb<V>(V_P), *v = vb<V>(V_V), *s = vb<V>(V_S), *t = vb<V>(V_T),
      *y = vb<V>(V_Y);
   const int h = herm ? 1 : 0;
-  const int maxit = maxit_;
   dim3 grid(nblk_, nrhs), blk(kBlock);
   // v = post(p, G y) and t = post(s, G y) with their dot products are the
-  // near-field kernel's epilogue (NearPost); its partials are per near workgroup
+  // near-field kernel's epilogue (NearPost; its partials are per near workgroup),
+  // and P2M forms p or s and y while it loads its input (P2mStep)
   NearPost<V> post;
   post.g = g;
   post.gs = gs;
   post.herm = h;
   post.part = part_;
-  k_bi_pupd<V><<<grid, blk, 0, stream_>>>(r, p, v, g, gs, y, N, h, state_);
+  P2mStep<V> step;
+  step.r = r;
+  step.v = v;
+  step.y = y;
+  step.g = g;
+  step.gs = gs;
+  step.herm = h;
+  step.st = state_;
+  step.mode = 2;
+  step.p = p;
   post.mode = 1;
   post.x = p;
   post.rt = rt;
-  apply_vec<V>(y, v, nrhs, active_, prec, &post);
-  k_bi_fin<<<dim3(nrhs), blk, 0, stream_>>>(PH_ALPHA, state_, active_, part_, near_blocks_, tolv_, maxit);
-  k_bi_supd<V><<<grid, blk, 0, stream_>>>(r, v, g, gs, s, y, N, h, state_);
+  apply_vec<V>(y, v, nrhs, active_, prec, &post, &step);
+  step.mode = 3;
+  step.p = s;
+  step.part = part_;
+  step.nblk = near_blocks_;
   post.mode = 2;
   post.x = s;
   post.rt = nullptr;
-  apply_vec<V>(y, t, nrhs, active_, prec, &post);
-  k_bi_fin<<<dim3(nrhs), blk, 0, stream_>>>(PH_OMEGA, state_, active_, part_, near_blocks_, tolv_, maxit);
+  apply_vec<V>(y, t, nrhs, active_, prec, &post, &step);
+  // omega's partials are in part_, so the residual's go to y, which is free until
+  // the next product (kSlots nblk_ of 16 bytes; N >= 1024 nblk_ or nblk_ = 1)
+  double2* rpart = reinterpret_cast<double2*>(y);
   prof_begin(KT_VEC);
-  k_bi_xrupd<V><<<grid, blk, 0, stream_>>>(x, p, s, t, r, rt, N, state_, part_);
+  k_bi_xrupd<V><<<grid, blk, 0, stream_>>>(x, p, s, t, r, rt, N, state_, part_, near_blocks_, rpart);
   prof_end(KT_VEC);
-  k_bi_fin<<<dim3(nrhs), blk, 0, stream_>>>(PH_RESID, state_, active_, part_, nblk_, tolv_, maxit);
+  k_bi_fin<<<dim3(nrhs), blk, 0, stream_>>>(PH_RESID, state_, active_, rpart, nblk_, tolv_, maxit_);
   ISG_HIP(hipMemcpyAsync(active_h_, active_, nrhs * sizeof(int), hipMemcpyDeviceToHost, stream_));
 }
 

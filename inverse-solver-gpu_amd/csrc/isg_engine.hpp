@@ -49,14 +49,6 @@ struct SolveStat {
   double relres;  // final relative residual (FP64 true residual for mixed solves)
 };
 
-// Device-resident BiCGSTAB scalars of one right-hand side.
-struct BiState {
-  zd rho, rho1, alpha, omega, beta;
-  double bnrm, err, tol;
-  int iter, status, active, first;
-};
-
-
 // Device copies of the operator tables and the multipole/local stores in
 // precision T.
 template <typename T>
@@ -201,11 +193,12 @@ class Engine {
   void build_down();
   // operator with tables / multipoles of type T on vectors of type TI
   template <typename T, typename TI>
-  void apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, const NearPost<TI>* post = nullptr);
+  void apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, const NearPost<TI>* post = nullptr,
+             const P2mStep<TI>* step = nullptr);
   // `force` >= 0 overrides the tuned / built-in choice (autotuner)
   template <typename T, typename TI>
   // prep (mode 3): y is the iterate x and P2M loads prep(x) (FP64 only)
-  void launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force = -1, const NearPost<TI>* prep = nullptr);
+  void launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force = -1, const P2mStep<TI>* step = nullptr);
   template <typename T>
   void launch_m2m(int i, int nrhs, const int* act, int force = -1);
   template <typename T>
@@ -240,7 +233,7 @@ class Engine {
   cplx<V>* vb(int k);
   template <typename V>
   void apply_vec(const cplx<V>* y, cplx<V>* r, int nrhs, const int* act, int prec,
-                 const NearPost<V>* post = nullptr);
+                 const NearPost<V>* post = nullptr, const P2mStep<V>* step = nullptr);
   // r0_in_res: the initial residual is already in vb<V>(V_RES) (blended start)
   void solve(zd* x, const zd* g, long gs, const zd* b, bool herm, int nrhs, bool x_zero, double tol, int maxit,
              std::vector<SolveStat>& out, int prec, bool r0_in_res);

@@ -225,6 +225,96 @@ __device__ __forceinline__ zd stv(cplx<V>* a, long i, zd v) {
   return ccast<double>(w);  // the value as stored
 }
 
+// Sum over blocks of one system's partials, slots 0 .. NS - 1, in a fixed order;
+// every thread gets it.  sh: LDS, reusable after the caller's next barrier.
+template <int NS>
+__device__ __forceinline__ void part_sum(const double2* __restrict__ pr, int nblk, zd (&tot)[NS],
+                                         double (*sh)[kBlock / 64]) {
+  double v[2 * NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    v[2 * s] = v[2 * s + 1] = 0;
+    for (int j = threadIdx.x; j < nblk; j += kBlock) {
+      const double2 q = pr[s * nblk + j];
+      v[2 * s] += q.x;
+      v[2 * s + 1] += q.y;
+    }
+  }
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __syncthreads();  // an earlier call's sums have been read
+#pragma unroll
+  for (int s = 0; s < 2 * NS; s++) {
+    const double a = wave_sum(v[s]);
+    if (lane == 0) sh[s][w] = a;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    tot[s] = mkc<double>(0, 0);
+    for (int i = 0; i < kBlock / 64; i++) {
+      tot[s].x += sh[2 * s][i];
+      tot[s].y += sh[2 * s + 1][i];
+    }
+  }
+}
+
+// The vector step of P2mStep, element by element (o: the system's offset,
+// element i of it; load only loads, so that a group's loads are in flight
+// together).  Every element belongs to one workgroup.  alpha is summed by each
+// workgroup from at most B / 16 partials in L2 (a kernel of one workgroup per
+// system between the two products cost 5 us of latency); the first stores it.
+template <typename V>
+struct StepIn {
+  cplx<V> r, p, v;
+  zd g;
+};
+struct StepCoef {
+  zd a, b;
+  bool first;
+};
+template <int STEP, typename V>
+__device__ __forceinline__ StepCoef step_coef(const P2mStep<V>& q, int rhs, void* lds) {
+  StepCoef c;
+  c.first = false;
+  if constexpr (STEP == 2) {
+    const BiState& S = q.st[rhs];
+    c.a = S.beta;
+    c.b = mkc<double>(-S.omega.x, -S.omega.y);
+    c.first = S.first != 0;
+  } else if constexpr (STEP == 3) {
+    zd t[1];
+    part_sum<1>(q.part + (long)rhs * kSlots * q.nblk, q.nblk, t, static_cast<double(*)[kBlock / 64]>(lds));
+    const zd al = zdiv(q.st[rhs].rho, t[0]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) q.st[rhs].alpha = al;
+    c.a = mkc<double>(-al.x, -al.y);
+  }
+  return c;
+}
+template <int STEP, typename V>
+__device__ __forceinline__ StepIn<V> step_load(const P2mStep<V>& q, const StepCoef& c, long o, long go, long i) {
+  StepIn<V> in;
+  in.r = q.r[o + i];
+  if constexpr (STEP == 2) {
+    if (!c.first) {
+      in.p = q.p[o + i];
+      in.v = q.v[o + i];
+    }
+  }
+  if constexpr (STEP == 3) in.v = q.v[o + i];
+  if (!q.herm) in.g = q.g[go + i];
+  return in;
+}
+template <int STEP, typename V>
+__device__ __forceinline__ cplx<V> step_value(const P2mStep<V>& q, const StepCoef& c, const StepIn<V>& in, cplx<V>& pv) {
+  zd x = ccast<double>(in.r);
+  if constexpr (STEP == 2)
+    if (!c.first) x = cfma(c.a, cfma(c.b, ccast<double>(in.v), ccast<double>(in.p)), x);
+  if constexpr (STEP == 3) x = cfma(c.a, ccast<double>(in.v), x);
+  pv = ccast<V>(x);
+  x = ccast<double>(pv);  // the value as stored
+  return ccast<V>(q.herm ? cconj(x) : cmul(x, in.g));
+}
+
 // Output of a near-field kernel whose NB x 64 products are in LDS: stored, or
 // the BiCGSTAB post step / residual check of NearPost.
 template <typename T, typename TI, int NB, int POST>
@@ -903,20 +993,19 @@ k_m2l_par(M2LSet<T> set, const int* __restrict__ act) {
 // tile of NB boxes.  The work is cut into units of 16 rows k x 16 boxes, dealt
 // round-robin to the 4 waves: with S = 68 (5 row blocks) and 64-box tiles
 // every wave gets 5 units (whole row blocks per wave would leave three waves
-// idle half the time).  PREP (FP64 only): y holds x and the contrast product
-// prep(x) (g x forward, conj(x) adjoint) is formed while loading it.
+// idle half the time).  STEP: the vector step of P2mStep while loading; y is
+// unused then.
 // With S <= kP2mRows (at most 5 row blocks) the units' results stay in
 // registers until every wave is done, then go through LDS so that the tile's
 // contiguous output range [b0 S, (b0 + NB) S) is written with whole,
 // coalesced lines (stored from the MFMA layout, a box's row blocks came from
 // different waves and partial lines reached HBM separately).
 constexpr int kP2mRows = 80;
-template <typename T, typename TI, int NB, bool PREP = false>
+template <typename T, typename TI, int NB, int STEP = 0>
 __global__ void __launch_bounds__(kBlock) k_p2m_mfma(const cplx<TI>* __restrict__ y, long ys,
                                                      cplx<T>* __restrict__ agm, long as,
                                                      const cplx<T>* __restrict__ coeffT, int S,
-                                                     const int* __restrict__ act, const zd* __restrict__ g = nullptr,
-                                                     long gs = 0, int herm = 0) {
+                                                     const int* __restrict__ act, P2mStep<TI> step) {
   typedef typename Mfma<T>::v4 v4;
   constexpr int NN = NB / 16;
   constexpr int MAXU = (5 * NN + 3) / 4;  // units per wave with 5 row blocks
@@ -928,14 +1017,26 @@ __global__ void __launch_bounds__(kBlock) k_p2m_mfma(const cplx<TI>* __restrict_
   const long b0 = (long)xcd_block() * NB;
   const cplx<TI>* yr = y + rhs * ys + b0 * 64;
   // loads issued in groups ahead of their LDS stores
-  stage<sizeof(T) == 4 ? 8 : 4, cplx<TI>>(
-      NB * 64,
-      [&](int idx) {
-        cplx<TI> v = yr[idx];
-        if constexpr (PREP) v = prep_val(v, g, rhs * gs + b0 * 64 + idx, herm != 0);
-        return v;
-      },
-      [&](int idx, cplx<TI> v) { tile[(idx >> 6) * 65 + (idx & 63)] = ccast<T>(v); });
+  if constexpr (STEP == 0) {
+    stage<sizeof(T) == 4 ? 8 : 4, cplx<TI>>(
+        NB * 64, [&](int idx) { return yr[idx]; },
+        [&](int idx, cplx<TI> v) { tile[(idx >> 6) * 65 + (idx & 63)] = ccast<T>(v); });
+  } else {
+    const long o = rhs * ys + b0 * 64, go = rhs * step.gs + b0 * 64;
+    const StepCoef c = step_coef<STEP>(step, rhs, tile);
+    if constexpr (STEP == 3) __syncthreads();
+    stage<4, StepIn<TI>>(
+        NB * 64, [&](int idx) { return step_load<STEP>(step, c, o, go, idx); },
+        [&](int idx, const StepIn<TI>& in) {
+          cplx<TI> pv;
+          const cplx<TI> yv = step_value<STEP>(step, c, in, pv);
+          if constexpr (STEP > 1) {
+            step.p[o + idx] = pv;
+            step.y[o + idx] = yv;
+          }
+          tile[(idx >> 6) * 65 + (idx & 63)] = ccast<T>(yv);
+        });
+  }
   __syncthreads();
   const int nrb = (S + 15) / 16, nunit = nrb * NN;
   const bool staged = S <= kP2mRows;

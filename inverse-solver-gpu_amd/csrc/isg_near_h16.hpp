@@ -458,7 +458,9 @@ k_near_h16(const zf* __restrict__ y, long ys, const zf* __restrict__ loc, long l
 // P2M of the FP32 operator on split FP16: agm[box][s] = sum_n coeffT[n][s]
 // y[box 64 + n] for 32 Morton-consecutive boxes of two right-hand sides.
 // The workgroup's input (2 x 32 boxes x 64 pixels) is loaded once into
-// registers (units of 8 pixels: 2 per thread), its largest component per
+// registers, whole lines per instruction (8 pixels per thread and 64-byte stride
+// between lanes, with three to five arrays in flight, ran from L2: 697 -> 557 us
+// for STEP 2 at 1024 px x 64), its largest component per
 // right-hand side sets the data scale, and it is staged split in LDS as
 // [rhs][part][pixel group 8][box 32] x 8 FP16 (boxes XOR 2 (g mod 4), as in
 // k_near_h16).  Wave w owns right-hand side w / 2, row block w % 2 (16
@@ -471,9 +473,10 @@ k_near_h16(const zf* __restrict__ y, long ys, const zf* __restrict__ loc, long l
 constexpr int kP2mH16MaxCB = 6;  // column blocks held per wave (S <= 96)
 // (at least 4 waves per SIMD: unbounded, the compiler hoists every
 // coefficient fragment of both K chunks and takes 256 registers)
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as,
-                                                    const v8h* __restrict__ coef, int ec, int S, int nrhs,
-                                                    const int* __restrict__ act) {
+template <int STEP>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
+k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as, const v8h* __restrict__ coef, int ec, int S,
+          int nrhs, const int* __restrict__ act, P2mStep<float> step) {
   __shared__ v8h hal[2 * 4 * 8 * 32];
   __shared__ float red[4][kBlock / 64];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -488,15 +491,58 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
   const int rv[2] = {on[0] ? rhs[0] : rhs[1], on[1] ? rhs[1] : rhs[0]};
   const long b0 = (long)xcd_block() * 32;
   const int ncb = (S + 15) / 16, ncolp = 16 * ncb;
-  // units (q, box, g8): pixels 8 g8 .. +7 of box b0 + box of right-hand side q; unit t of this thread
-  // is tid + 256 t, so q = t and g8 = tid % 8 for both
-  const int bx = (tid >> 3) & 31, g8 = tid & 7;
+  // load c of this thread: pixels 2 pr and 2 pr + 1 of group g8 of box bx + 8 c, so
+  // that a wave's load and store instructions cover whole lines
+  const int bx = tid >> 5, g8 = (tid >> 2) & 7, pr = tid & 3;
   float4 v[2][4];
 #pragma unroll
   for (int q = 0; q < 2; q++) {
-    const float4* src = reinterpret_cast<const float4*>(y + (long)sel2(rv, q) * ys + (b0 + bx) * 64 + 8 * g8);
+    const long o = (long)sel2(rv, q) * ys + b0 * 64 + 2 * tid;  // + 512 c
+    if constexpr (STEP == 0) {
 #pragma unroll
-    for (int c = 0; c < 4; c++) v[q][c] = src[c];
+      for (int c = 0; c < 4; c++) v[q][c] = *reinterpret_cast<const float4*>(y + o + 512 * c);
+    } else {
+      // (a switched-off system's vectors stay as they are)
+      if (!sel2(on, q)) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) v[q][c] = make_float4(0.f, 0.f, 0.f, 0.f);
+        continue;
+      }
+      const StepCoef cf = step_coef<STEP>(step, rhs[q], hal);  // (hal is filled behind block_max's barrier)
+      const zd* g = step.g + rhs[q] * step.gs + b0 * 64 + 2 * tid;
+      StepIn<float> in[8];
+      auto ld = [&](const zf* a, zf StepIn<float>::*f) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const float4 x = *reinterpret_cast<const float4*>(a + o + 512 * c);
+          in[2 * c].*f = mkc<float>(x.x, x.y);
+          in[2 * c + 1].*f = mkc<float>(x.z, x.w);
+        }
+      };
+      ld(step.r, &StepIn<float>::r);
+      if (STEP == 3 || !cf.first) ld(step.v, &StepIn<float>::v);
+      if (STEP == 2 && !cf.first) ld(step.p, &StepIn<float>::p);
+      if (!step.herm) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          in[2 * c].g = g[512 * c];
+          in[2 * c + 1].g = g[512 * c + 1];
+        }
+      }
+      float4 pv[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        zf p0, p1;
+        const zf y0 = step_value<STEP>(step, cf, in[2 * c], p0), y1 = step_value<STEP>(step, cf, in[2 * c + 1], p1);
+        pv[c] = make_float4(p0.x, p0.y, p1.x, p1.y);
+        v[q][c] = make_float4(y0.x, y0.y, y1.x, y1.y);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        *reinterpret_cast<float4*>(step.p + o + 512 * c) = pv[c];
+        *reinterpret_cast<float4*>(step.y + o + 512 * c) = v[q][c];
+      }
+    }
   }
   int es[2];
   {
@@ -514,14 +560,17 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
   }
 #pragma unroll
   for (int q = 0; q < 2; q++) {
-    const float s = ldexpf(1.f, sel2(es, q));
-    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-    const bool ok = sel2(on, q);
-    v8h ph[4];
-    h16_split4(ok ? v[q][0] : z, ok ? v[q][1] : z, s, ph, 0);
-    h16_split4(ok ? v[q][2] : z, ok ? v[q][3] : z, s, ph, 4);
+    const float s = sel2(on, q) ? ldexpf(1.f, sel2(es, q)) : 0.f;
 #pragma unroll
-    for (int P = 0; P < 4; P++) hal[((q * 4 + P) * 8 + g8) * 32 + (bx ^ (2 * (g8 & 3)))] = ph[P];
+    for (int c = 0; c < 4; c++) {
+      const v2f re = v2f{v[q][c].x * s, v[q][c].z * s}, im = v2f{v[q][c].y * s, v[q][c].w * s};
+      const v2h rh = __builtin_convertvector(re, v2h), mh = __builtin_convertvector(im, v2h);
+      const v2h part[4] = {rh, __builtin_convertvector(h16_rest(re, rh), v2h), mh,
+                           __builtin_convertvector(h16_rest(im, mh), v2h)};
+#pragma unroll
+      for (int P = 0; P < 4; P++)
+        reinterpret_cast<v2h*>(hal + ((q * 4 + P) * 8 + g8) * 32 + ((bx + 8 * c) ^ (2 * (g8 & 3))))[pr] = part[P];
+    }
   }
   __syncthreads();
   if (!mine) return;  // no barrier follows

@@ -5,14 +5,18 @@
 // (bicgs_gpu.cu:16-58, 116-224; kernels.cu:334-413).  Here each step is one
 // fused pass that also produces the dot products the next scalar needs:
 //   k_bi_init   r = b - A x, r~ = r, partial <b,b>, <r,r>
-//   k_bi_pupd   p = r + beta (p - omega v), y = prep(p)
-//   (near)      v = post(p, G y), partial <r~,v>    -- epilogue of the near-field kernel
-//   k_bi_supd   s = r - alpha v, y = prep(s)
-//   (near)      t = post(s, G y), partial <t,s>, <t,t>    -- likewise
-//   k_bi_xrupd  x += alpha p; x += omega s; r = s - omega t; partial <r,r>, <r~,r>
-// Partial sums are FP64, one per block, reduced in a fixed order by
-// k_bi_fin, which also advances the per-right-hand-side scalars on the
-// device (no host round trip).  prep/post are the contrast products of
+//   (P2M)       p = r + beta (p - omega v), y = prep(p)   -- while P2M loads its input
+//   (near)      v = post(p, G y), partial <r~,v>          -- epilogue of the near-field kernel
+//   (P2M)       alpha; s = r - alpha v, y = prep(s)       -- P2mStep
+//   (near)      t = post(s, G y), partial <t,s>, <t,t>    -- NearPost
+//   k_bi_xrupd  omega; x += alpha p; x += omega s; r = s - omega t; partial <r,r>, <r~,r>
+// Partial sums are FP64, one per block, reduced in a fixed order by their
+// consumers and, at the end of an iteration, by k_bi_fin, which advances the
+// per-right-hand-side scalars on the device (no host round trip).  Forming p and
+// s in kernels of their own, and alpha and omega in two more, cost 4 of 25
+// launches an iteration at 256 px (solve of 9 iterations in FP64 2.45 -> 2.1 ms)
+// and two reads of y (1024 px x 64, FP32 vectors, update and P2M: 442 + 239 ->
+// 557 us for p, 380 + 239 -> 485 us for s: 5.5 TB/s).  prep/post are the contrast products of
 // kernels.cu:394-409: forward y = g x, v = x - Gy; adjoint y = conj x,
 // v = x - conj(g Gy).
 #pragma once
@@ -23,7 +27,7 @@
 
 namespace isg {
 
-enum { PH_INIT = 0, PH_ALPHA = 1, PH_OMEGA = 2, PH_RESID = 3 };
+enum { PH_INIT = 0, PH_RESID = 1 };
 // r0 (may be null) supplies a residual computed beforehand (blended start).
 template <typename V>
 __global__ void __launch_bounds__(kBlock) k_bi_init(const zd* __restrict__ x, const cplx<V>* __restrict__ gy,
@@ -51,56 +55,26 @@ __global__ void __launch_bounds__(kBlock) k_bi_init(const zd* __restrict__ x, co
   block_store<2>(acc, part + (long)rhs * kSlots * gridDim.x, gridDim.x, blockIdx.x);
 }
 
-template <typename V>
-__global__ void __launch_bounds__(kBlock) k_bi_pupd(const cplx<V>* __restrict__ r, cplx<V>* __restrict__ p,
-                                                    const cplx<V>* __restrict__ v, const zd* __restrict__ g, long gs,
-                                                    cplx<V>* __restrict__ y, long N, int herm,
-                                                    const BiState* __restrict__ st) {
-  int rhs = blockIdx.y;
-  const BiState& S = st[rhs];
-  if (!S.active) return;
-  long o = rhs * N;
-  zd beta = S.beta, mom = mkc<double>(-S.omega.x, -S.omega.y);
-  int first = S.first;
-  ISG_VEC_LOOP(N) {
-    zd pv;
-    if (first) {
-      pv = ldv(r, o + i);
-    } else {
-      zd tmp = cfma(mom, ldv(v, o + i), ldv(p, o + i));
-      pv = cfma(beta, tmp, ldv(r, o + i));
-    }
-    pv = stv(p, o + i, pv);
-    stv(y, o + i, prep_val(pv, g, rhs * gs + i, herm));
-  }
-}
-
-template <typename V>
-__global__ void __launch_bounds__(kBlock) k_bi_supd(const cplx<V>* __restrict__ r, const cplx<V>* __restrict__ v,
-                                                    const zd* __restrict__ g, long gs, cplx<V>* __restrict__ s,
-                                                    cplx<V>* __restrict__ y, long N, int herm,
-                                                    const BiState* __restrict__ st) {
-  int rhs = blockIdx.y;
-  const BiState& S = st[rhs];
-  if (!S.active) return;
-  long o = rhs * N;
-  zd mal = mkc<double>(-S.alpha.x, -S.alpha.y);
-  ISG_VEC_LOOP(N) {
-    zd sv = stv(s, o + i, cfma(mal, ldv(v, o + i), ldv(r, o + i)));
-    stv(y, o + i, prep_val(sv, g, rhs * gs + i, herm));
-  }
-}
-
+// omega = <t,s> / <t,t> from the near field's partials (nnear per system, summed
+// by every workgroup; the first stores it).  part must not overlap them.
 template <typename V>
 __global__ void __launch_bounds__(kBlock) k_bi_xrupd(zd* __restrict__ x, const cplx<V>* __restrict__ p,
                                                      const cplx<V>* __restrict__ s, const cplx<V>* __restrict__ t,
                                                      cplx<V>* __restrict__ r, const cplx<V>* __restrict__ rt, long N,
-                                                     const BiState* __restrict__ st, double2* __restrict__ part) {
+                                                     BiState* __restrict__ st, const double2* __restrict__ near_part,
+                                                     int nnear, double2* __restrict__ part) {
   int rhs = blockIdx.y;
-  const BiState& S = st[rhs];
+  BiState& S = st[rhs];
   if (!S.active) return;
   long o = rhs * N;
-  zd al = S.alpha, om = S.omega, mom = mkc<double>(-S.omega.x, -S.omega.y);
+  __shared__ double sh[4][kBlock / 64];
+  zd dot[2];
+  part_sum<2>(near_part + (long)rhs * kSlots * nnear, nnear, dot, sh);
+  const double tt = dot[1].x;
+  zd om = mkc<double>(dot[0].x / tt, dot[0].y / tt);
+  if (zabs(dot[0]) < 1e-200 && tt < 1e-200) om = mkc<double>(1.0, 0.0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) S.omega = om;
+  const zd al = S.alpha, mom = mkc<double>(-om.x, -om.y);
   zd acc[2] = {mkc<double>(0, 0), mkc<double>(0, 0)};
   ISG_VEC_LOOP(N) {
     zd sv = ldv(s, o + i);
@@ -125,27 +99,11 @@ __global__ void __launch_bounds__(kBlock) k_bi_fin(int phase, BiState* __restric
   BiState& S = st[rhs];
   if (phase != PH_INIT && !S.active) return;
   const double tol = (phase == PH_INIT) ? tolv[rhs] : S.tol;
-  const double2* pr = part + (long)rhs * kSlots * nblk;
-  int ns = (phase == PH_ALPHA) ? 1 : 2;
   __shared__ double sh[4][kBlock / 64];
-  double v[4] = {0, 0, 0, 0};
-  for (int s = 0; s < ns; s++)
-    for (int j = threadIdx.x; j < nblk; j += kBlock) {
-      double2 q = pr[s * nblk + j];
-      v[2 * s] += q.x;
-      v[2 * s + 1] += q.y;
-    }
-  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int s = 0; s < 4; s++) {
-    double a = wave_sum(v[s]);
-    if (lane == 0) sh[s][w] = a;
-  }
-  __syncthreads();
+  zd dot[2];
+  part_sum<2>(part + (long)rhs * kSlots * nblk, nblk, dot, sh);
   if (threadIdx.x != 0) return;
-  double tot[4] = {0, 0, 0, 0};
-  for (int s = 0; s < 4; s++)
-    for (int i = 0; i < kBlock / 64; i++) tot[s] += sh[s][i];
-  zd s0 = mkc<double>(tot[0], tot[1]), s1 = mkc<double>(tot[2], tot[3]);
+  const zd s0 = dot[0], s1 = dot[1];
   if (phase == PH_INIT) {
     double bn = sqrt(s0.x);
     if (bn < 1e-20) bn = 1;
@@ -171,12 +129,6 @@ __global__ void __launch_bounds__(kBlock) k_bi_fin(int phase, BiState* __restric
       S.status = (S.err < tol) ? 0 : 1;
       S.active = 0;
     }
-  } else if (phase == PH_ALPHA) {
-    S.alpha = zdiv(S.rho, s0);
-  } else if (phase == PH_OMEGA) {
-    double tt = s1.x;
-    S.omega = mkc<double>(s0.x / tt, s0.y / tt);
-    if (zabs(s0) < 1e-200 && tt < 1e-200) S.omega = mkc<double>(1.0, 0.0);
   } else {
     S.err = sqrt(s0.x) / S.bnrm;
     if (S.err < tol) {
