@@ -60,16 +60,6 @@ __device__ __forceinline__ float max3_abs(float m, float a, float b) {
   return r;
 }
 
-// Maximum of non-negative values over the 16 lanes of a row.
-__device__ __forceinline__ float row_max(float v) {
-  unsigned m = __builtin_bit_cast(unsigned, v);  // ordered as the floats are (a NaN above all)
-  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x128, 0xf, 0xf, false));  // row_ror:8, 4, 2, 1
-  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x124, 0xf, 0xf, false));
-  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x122, 0xf, 0xf, false));
-  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x121, 0xf, 0xf, false));
-  return __builtin_bit_cast(float, m);
-}
-
 // Buffer descriptor of `bytes` bytes at p (raw, 32-bit offsets; a load past the
 // end returns 0) and an 8-byte load through it.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t down_rsrc(const void* p, unsigned bytes) {

@@ -318,6 +318,7 @@ Engine::Engine(const EngineConfig& cfg) : cfg_(cfg) {
   plan_interp(op64_, m2m64_, l2l64_);
   if (has32_) plan_interp(op32_, m2m32_, l2l32_);
   build_down();
+  if (has32_) build_up16();
   for (auto& row : tune_)
     for (auto& t : row) {
       t.m2l.assign(P_.L, -1);
@@ -512,6 +513,44 @@ void Engine::build_split16() {
   ISG_HIP(hipStreamSynchronize(stream_));
 }
 
+// Table of the leaf level's M2M inside k_p2m_h16: the interpolator's band in
+// blocks of 16 parent samples, the window of child samples starting at a
+// multiple of 8, split into FP16 in the layout of the matrix operand.  Left
+// empty (separate kernels) for windows and sample counts that do not fit.
+void Engine::build_up16() {
+  if (!ok() || !p2m16_ || P_.L < 4) return;
+  const int Lf = P_.L - 1, Sc = P_.nsamp[Lf], Sp = P_.nsamp[Lf - 1], ni = cfg_.plan.ninter, nck = (Sp + 15) / 16;
+  if (Sc < kUpMinS || Sc > kUpMaxS || nck > 4 * kUpRounds) return;
+  const std::vector<int>& first = P_.interp0[Lf - 1];
+  const std::vector<double>& wt = P_.interpT[Lf - 1];
+  std::vector<int> s0(nck);
+  double m = 0;
+  for (double v : wt) m = std::max(m, std::fabs(v));
+  up16_ec_ = h16_scale_exp((float)m);
+  std::vector<_Float16> tab((size_t)nck * 4 * 64 * 8, (_Float16)0.f);
+  for (int ck = 0; ck < nck; ck++) {
+    s0[ck] = ((first[16 * ck] % Sc) + Sc) % Sc / 8 * 8;
+    for (int c = 0; c < 16 && 16 * ck + c < Sp; c++) {
+      const int k = 16 * ck + c, off = (((first[k] - s0[ck]) % Sc) + Sc) % Sc;
+      if (off + ni > kUpWin) return;
+      for (int t = 0; t < ni; t++) {
+        const int j = off + t;  // window element: chunk j / 32, lane group (j % 32) / 8, element j % 8
+        const double v = std::ldexp(wt[(size_t)t * Sp + k], up16_ec_);
+        const _Float16 hi = (_Float16)(float)v, lo = (_Float16)(float)(v - (double)(float)hi);
+        const size_t e = ((((size_t)ck * 2 + j / 32) * 2) * 64 + (j % 32 / 8) * 16 + c) * 8 + j % 8;
+        tab[e] = hi;
+        tab[e + 64 * 8] = lo;
+      }
+    }
+  }
+  up16_s0_ = (int*)dalloc(nck * sizeof(int));
+  void* t = dalloc(tab.size() * sizeof(_Float16));
+  if (!ok()) return;
+  ISG_HIP(hipMemcpy(up16_s0_, s0.data(), nck * sizeof(int), hipMemcpyHostToDevice));
+  ISG_HIP(hipMemcpy(t, tab.data(), tab.size() * sizeof(_Float16), hipMemcpyHostToDevice));
+  up16_ = t;
+}
+
 // Tables of the fused downward kernels for levels 3 .. leaf: the band blocks of
 // each level's anterpolator (k_down64), and for the FP32 operator those with the
 // four child shifts folded in, split into FP16 (k_down_h16).  Left empty
@@ -659,7 +698,7 @@ int Engine::interp_kind(const InterpShape& sh, int np, int nrhs) const {
 // --------------------------------------------------------------- launches
 // leaf radiation patterns on the matrix cores
 template <typename T, typename TI>
-void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, const P2mStep<TI>* step) {
+bool Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, const P2mStep<TI>* step, bool up) {
   const int Lf = P_.L - 1, S = P_.nsamp[Lf], B = P_.B;
   const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).p2m_nb;
   // built-in rule: 32-box tiles once they fill the chip, else 16 (64 px, one system: 12.9 -> 9.6 us)
@@ -676,9 +715,22 @@ void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
     if constexpr (sizeof(T) == 4 && sizeof(TI) == 4) {
       if (mode != 1 && B % 32 == 0 && p2m16_ && (nrhs >= 4 || force == kNearSplit)) {
         dim3 grid(B / 32, (nrhs + 1) / 2);
-        auto k = mode == 0 ? k_p2m_h16<0> : (mode == 2 ? k_p2m_h16<2> : k_p2m_h16<3>);
-        k<<<grid, blk, 0, stream_>>>(y, P_.N, out, as, (const v8h*)p2m16_, p2m16_ec_, S, nrhs, act, st);
-        return;
+        P2mUp u;
+        up = up && up16_;
+        if (up) {
+          u.par = d.agm + lvl_off_[Lf - 1];
+          u.ps = (long)lvl_size_[Lf - 1];
+          u.tab = (const v8h*)up16_;
+          u.s0 = up16_s0_;
+          u.shift = d.shiftM[Lf - 1];
+          u.Sp = P_.nsamp[Lf - 1];
+          u.ec = up16_ec_;
+        }
+        auto k = mode == 0 ? (up ? k_p2m_h16<0, true> : k_p2m_h16<0, false>)
+                           : (mode == 2 ? (up ? k_p2m_h16<2, true> : k_p2m_h16<2, false>)
+                                        : (up ? k_p2m_h16<3, true> : k_p2m_h16<3, false>));
+        k<<<grid, blk, 0, stream_>>>(y, P_.N, out, as, (const v8h*)p2m16_, p2m16_ec_, S, nrhs, act, st, u);
+        return up;
       }
     }
     nb = B >= 32 ? 32 : 16;
@@ -694,14 +746,25 @@ void Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
     if (nb == 32) return go(k_p2m_mfma<T, TI, 32, M>);
     go(k_p2m_mfma<T, TI, 16, M>);
   };
-  if (mode == 0) return tile(std::integral_constant<int, 0>());
-  if constexpr (sizeof(T) == sizeof(TI)) {
-    // the solver's vector steps; contrast weighting alone (mode 1) serves the FP64 residual check
-    if (mode == 2) return tile(std::integral_constant<int, 2>());
-    if (mode == 3) return tile(std::integral_constant<int, 3>());
-    if constexpr (sizeof(T) == 8) return tile(std::integral_constant<int, 1>());
+  if (mode == 0) {
+    tile(std::integral_constant<int, 0>());
+    return false;
   }
-  set_error("P2M: no kernel for this step on vectors of this type");
+  // the solver's vector steps; contrast weighting alone (mode 1) serves the FP64 residual check
+  bool done = false;
+  if constexpr (sizeof(T) == sizeof(TI)) {
+    done = true;
+    if (mode == 2)
+      tile(std::integral_constant<int, 2>());
+    else if (mode == 3)
+      tile(std::integral_constant<int, 3>());
+    else if constexpr (sizeof(T) == 8)
+      tile(std::integral_constant<int, 1>());
+    else
+      done = false;
+  }
+  if (!done) set_error("P2M: no kernel for this step on vectors of this type");
+  return false;
 }
 
 // child level i+1 -> parent level i
@@ -989,10 +1052,10 @@ void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, con
     step = &weight;
   }
   prof_begin(KT_P2M);
-  launch_p2m<T, TI>(y, nrhs, act, -1, step);
+  const bool up = launch_p2m<T, TI>(y, nrhs, act, -1, step, true);
   prof_end(KT_P2M);
   prof_begin(KT_INTERP);
-  for (int i = L - 2; i >= 2; i--) launch_m2m<T>(i, nrhs, act);
+  for (int i = up ? L - 3 : L - 2; i >= 2; i--) launch_m2m<T>(i, nrhs, act);
   prof_end(KT_INTERP);
   const int kt = sizeof(T) == 4 ? KT_M2L32 : KT_M2L;
   const int fuse = fuse_level(tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).leaf, nrhs);

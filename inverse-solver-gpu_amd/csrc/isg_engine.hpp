@@ -191,6 +191,7 @@ class Engine {
   // split-FP16 tables of the FP32 operator (k_near_h16, k_p2m_h16)
   void build_split16();
   void build_down();
+  void build_up16();
   // operator with tables / multipoles of type T on vectors of type TI
   template <typename T, typename TI>
   void apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, const NearPost<TI>* post = nullptr,
@@ -198,7 +199,9 @@ class Engine {
   // `force` >= 0 overrides the tuned / built-in choice (autotuner)
   template <typename T, typename TI>
   // prep (mode 3): y is the iterate x and P2M loads prep(x) (FP64 only)
-  void launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force = -1, const P2mStep<TI>* step = nullptr);
+  // up: M2M of the leaf level may be done as well; returns whether it was
+  bool launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force = -1, const P2mStep<TI>* step = nullptr,
+                  bool up = false);
   template <typename T>
   void launch_m2m(int i, int nrhs, const int* act, int force = -1);
   template <typename T>
@@ -270,6 +273,10 @@ class Engine {
   // k_p2m_h16 table ([2][4][4][16 ceil(S / 16)] groups of 8 FP16; null for S > 96) and its exponent
   void* p2m16_ = nullptr;
   int p2m16_ec_ = 0;
+  // leaf M2M inside k_p2m_h16: split table, window starts, scale exponent (null: not available)
+  void* up16_ = nullptr;
+  int* up16_s0_ = nullptr;
+  int up16_ec_ = 0;
   // fused downward kernels: per level (3 .. leaf) the band blocks, their window
   // starts and length, and the FP32 operator's split table with its scale exponent
   struct DownLevel {

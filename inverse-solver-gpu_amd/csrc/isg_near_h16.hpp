@@ -455,6 +455,16 @@ k_near_h16(const zf* __restrict__ y, long ys, const zf* __restrict__ loc, long l
   near_epilogue<float, float, 64, POST>(tile, r, rs, b0, rhs, post);
 }
 
+// Maximum of non-negative values over the 16 lanes of a row.
+__device__ __forceinline__ float row_max(float v) {
+  unsigned m = __builtin_bit_cast(unsigned, v);  // ordered as the floats are (a NaN above all)
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x128, 0xf, 0xf, false));  // row_ror:8, 4, 2, 1
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x124, 0xf, 0xf, false));
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x122, 0xf, 0xf, false));
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x121, 0xf, 0xf, false));
+  return __builtin_bit_cast(float, m);
+}
+
 // P2M of the FP32 operator on split FP16: agm[box][s] = sum_n coeffT[n][s]
 // y[box 64 + n] for 32 Morton-consecutive boxes of two right-hand sides.
 // The workgroup's input (2 x 32 boxes x 64 pixels) is loaded once into
@@ -470,13 +480,37 @@ k_near_h16(const zf* __restrict__ y, long ys, const zf* __restrict__ loc, long l
 // straight from the accumulators to HBM: lane li stores sample 16 cb + li of
 // box 16 j + 4 (lane / 16) + i, 16 consecutive samples per row.
 // Grid (B / 32, ceil(nrhs / 2)), kBlock threads.
+//
+// UP: the interpolation to the parents (M2M of the leaf level) follows in the
+// same workgroup, from the multipoles in registers (P2mUp).  They are scaled by
+// their box's largest component, split again and staged in LDS, real parts
+// first, then imaginary parts, with the first samples repeated past the end so
+// that a window never wraps.  Rows of the matrix product are boxes, 16 of them
+// the children of four parents, columns 16 parent samples, K the window of child
+// samples (<= kUpWin, from a multiple of 8, padded to 64 by zeros of the table);
+// wave w takes the parent samples 16 w + 64 u of all four row blocks.  A lane
+// ends with the four children of one parent: shifted and summed in registers.
+// HBM bounds both: alone, P2M wrote the multipoles in 239 us and M2M, on FP32
+// matrix products, read them again in 289 us (1024 px x 64); together 376 us, and
+// with STEP 2 or 3 620 and 566 instead of 557 + 289 and 485 + 289.
 constexpr int kP2mH16MaxCB = 6;  // column blocks held per wave (S <= 96)
+constexpr int kUpWin = 48, kUpPitch = 120, kUpRounds = 2, kUpCB = 5;
+// kUpCB column blocks exactly; a window from any 8 j < S ends inside what is staged
+constexpr int kUpMinS = 16 * kUpCB - 15, kUpMaxS = kUpPitch - kUpWin;
+struct P2mUp {
+  zf* par = nullptr;  // parents, ps between systems, Sp samples
+  long ps = 0;
+  const v8h* tab = nullptr;  // [sample block 16][k chunk 32][hi, lo][lane], scale 2^ec
+  const int* s0 = nullptr;   // window start of each sample block
+  const zf* shift = nullptr;  // [4][Sp]
+  int Sp = 0, ec = 0;
+};
 // (at least 4 waves per SIMD: unbounded, the compiler hoists every
 // coefficient fragment of both K chunks and takes 256 registers)
-template <int STEP>
+template <int STEP, bool UP>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as, const v8h* __restrict__ coef, int ec, int S,
-          int nrhs, const int* __restrict__ act, P2mStep<float> step) {
+          int nrhs, const int* __restrict__ act, P2mStep<float> step, P2mUp up) {
   __shared__ v8h hal[2 * 4 * 8 * 32];
   __shared__ float red[4][kBlock / 64];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -490,7 +524,7 @@ k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as, cons
   const bool mine = sel2(on, rw);
   const int rv[2] = {on[0] ? rhs[0] : rhs[1], on[1] ? rhs[1] : rhs[0]};
   const long b0 = (long)xcd_block() * 32;
-  const int ncb = (S + 15) / 16, ncolp = 16 * ncb;
+  const int ncb = UP ? kUpCB : (S + 15) / 16, ncolp = 16 * ncb;
   // load c of this thread: pixels 2 pr and 2 pr + 1 of group g8 of box bx + 8 c, so
   // that a wave's load and store instructions cover whole lines
   const int bx = tid >> 5, g8 = (tid >> 2) & 7, pr = tid & 3;
@@ -573,7 +607,7 @@ k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as, cons
     }
   }
   __syncthreads();
-  if (!mine) return;  // no barrier follows
+  if (!UP && !mine) return;  // no barrier follows
   v4f cr[kP2mH16MaxCB], ci[kP2mH16MaxCB];
 #pragma unroll
   for (int c = 0; c < kP2mH16MaxCB; c++) {
@@ -589,6 +623,7 @@ k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as, cons
 #pragma unroll
     for (int cb = 0; cb < kP2mH16MaxCB; cb++) {
       if (cb < ncb) {
+        if constexpr (UP) __builtin_amdgcn_sched_barrier(0);
         v8h b[4], nb[2];
 #pragma unroll
         for (int P = 0; P < 4; P++) b[P] = tl[(long)(kc * 4 + P) * 4 * ncolp + 16 * cb];
@@ -603,9 +638,110 @@ k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as, cons
 #pragma unroll
   for (int cb = 0; cb < kP2mH16MaxCB; cb++) {
     const int sm = 16 * cb + li;
-    if (cb < ncb && sm < S) {
+    if (mine && cb < ncb && sm < S) {
 #pragma unroll
       for (int i = 0; i < 4; i++) out[(long)i * S + sm] = mkc<float>(ldexpf(cr[cb][i], n), ldexpf(ci[cb][i], n));
+    }
+  }
+  if constexpr (UP) {
+    // ---- M2M: row block w of the workgroup is this wave's 16 boxes
+    __shared__ int exs[64];
+    _Float16* hl = reinterpret_cast<_Float16*>(hal);  // [row block 4][hi, lo][box 16][kUpPitch]
+    float sc[4];
+    int ex[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float m = 0.f;
+#pragma unroll
+      for (int cb = 0; cb < kUpCB; cb++) m = fmaxf(m, fmaxf(fabsf(cr[cb][i]), fabsf(ci[cb][i])));
+      ex[i] = h16_scale_exp(row_max(m));
+      sc[i] = ldexpf(1.f, ex[i]);
+    }
+    auto put = [&](const v4f (&c)[kP2mH16MaxCB]) {
+#pragma unroll
+      for (int cb = 0; cb < kUpCB; cb++) {
+        const int k = 16 * cb + li;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float x = c[cb][i] * sc[i];
+          const _Float16 hi = (_Float16)x, lo = (_Float16)(x - (float)hi);
+          _Float16* d = hl + (w * 32 + 4 * lk + i) * kUpPitch + k;
+          if (k < S) {
+            d[0] = hi;
+            d[16 * kUpPitch] = lo;
+            if (k + S < kUpPitch) {
+              d[S] = hi;
+              d[S + 16 * kUpPitch] = lo;
+            }
+          }
+        }
+      }
+    };
+    const int nck = (up.Sp + 15) / 16;
+    // products of sample block ck with the staged parts of all row blocks
+    auto band = [&](int ck, v4f (&acc)[4]) {
+      const v8h* tb = up.tab + ck * 256 + lane;
+      v8h b[2][2];
+#pragma unroll
+      for (int kc = 0; kc < 2; kc++)
+#pragma unroll
+        for (int P = 0; P < 2; P++) b[kc][P] = tb[(kc * 2 + P) * 64];
+      const int s0 = up.s0[ck];
+#pragma unroll
+      for (int rb = 0; rb < 4; rb++) {
+        acc[rb] = v4f{0, 0, 0, 0};
+        const _Float16* d = hl + (rb * 32 + li) * kUpPitch + s0;
+#pragma unroll
+        for (int kc = 0; kc < 2; kc++) {
+          // (past the window the table is zero; any staged value will do)
+          const int k = kc == 0 ? 8 * lk : 32 + 8 * (lk & 1);
+          const v8h hi = *reinterpret_cast<const v8h*>(d + k), lo = *reinterpret_cast<const v8h*>(d + 16 * kUpPitch + k);
+          acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, b[kc][0], acc[rb], 0, 0, 0);
+          acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, b[kc][1], acc[rb], 0, 0, 0);
+          acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, b[kc][0], acc[rb], 0, 0, 0);
+        }
+      }
+    };
+    __syncthreads();  // the input is no longer read
+    __builtin_amdgcn_sched_barrier(0);
+    if (li == 0)
+#pragma unroll
+      for (int i = 0; i < 4; i++) exs[16 * w + 4 * lk + i] = ex[i];
+    put(cr);
+    __syncthreads();
+    v4f re[kUpRounds][4];
+#pragma unroll
+    for (int u = 0; u < kUpRounds; u++) {
+      if (w + 4 * u < nck) band(w + 4 * u, re[u]);
+      __builtin_amdgcn_sched_barrier(0);  // (rounds interleaved would not fit the registers)
+    }
+    __syncthreads();
+    put(ci);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kUpRounds; u++) {
+      const int ck = w + 4 * u, col = 16 * ck + li;
+      if (ck < nck) {
+        v4f im[4];
+        band(ck, im);
+        __builtin_amdgcn_sched_barrier(0);
+        zf sh[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) sh[i] = up.shift[i * up.Sp + min(col, up.Sp - 1)];
+#pragma unroll
+        for (int rb = 0; rb < 4; rb++) {
+          const int n0 = -(es[rb >> 1] + ec + up.ec);
+          zf o = mkc<float>(0.f, 0.f);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int e = n0 - exs[16 * rb + 4 * lk + i];
+            o = cfma(sh[i], mkc<float>(ldexpf(re[u][rb][i], e), ldexpf(im[rb][i], e)), o);
+          }
+          if (on[rb >> 1] && col < up.Sp)
+            up.par[(long)rhs[rb >> 1] * up.ps + ((b0 >> 2) + 4 * (rb & 1) + lk) * up.Sp + col] = o;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
     }
   }
 }
