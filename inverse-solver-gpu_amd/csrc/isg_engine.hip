@@ -17,6 +17,7 @@
 #include "isg_kernels.hpp"
 #include "isg_near_h16.hpp"
 #include "isg_near_sym.hpp"
+#include "isg_p2m_sym.hpp"
 #include "isg_setup_kernels.hpp"
 #include "isg_solver_kernels.hpp"
 
@@ -227,7 +228,9 @@ void Engine::upload(DevOp<T>& d) {
   const int Sl = P_.nsamp[L - 1];
   d.sym_near = (cplx<T>*)dalloc((size_t)4 * kSymK * 16 * sizeof(cplx<T>));
   d.sym_l2p = (cplx<T>*)dalloc((size_t)4 * sym_reps(Sl) * 16 * sizeof(cplx<T>));
+  if constexpr (sizeof(T) == 8) d.sym_p2m = (double*)dalloc((size_t)4 * 16 * 32 * sizeof(double));
   if (ok()) {
+    if (sizeof(T) == 8 && Sl <= kP2mSymS) k_sym_p2m_table<<<8, 256, 0, stream_>>>(op64_.coeffT, Sl, d.sym_p2m);
     k_sym_tables<T><<<64, 256, 0, stream_>>>(op64_.near, op64_.basisT, Sl, d.sym_near, d.sym_l2p);
     ISG_HIP(hipGetLastError());
     ISG_HIP(hipStreamSynchronize(stream_));
@@ -701,8 +704,10 @@ template <typename T, typename TI>
 bool Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, const P2mStep<TI>* step, bool up) {
   const int Lf = P_.L - 1, S = P_.nsamp[Lf], B = P_.B;
   const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).p2m_nb;
-  // built-in rule: 32-box tiles once they fill the chip, else 16 (64 px, one system: 12.9 -> 9.6 us)
-  int nb = force > 0 ? force : (tuned > 0 ? tuned : ((long)(B / 32) * nrhs >= 256 ? 32 : 16));
+  // built-in rule: 32-box tiles once they fill the chip, else 16 (64 px, one system: 12.9 -> 9.6 us); the
+  // FP64 mirror-symmetric kernel 16 everywhere (512 px x 16: 55 us, 32-box tiles 61; 1024 px x 64: 870, 910)
+  const bool sym = sizeof(T) == 8 && S <= kP2mSymS;
+  int nb = force > 0 ? force : (tuned > 0 ? tuned : (!sym && (long)(B / 32) * nrhs >= 256 ? 32 : 16));
   DevOp<T>& d = ops<T>();
   cplx<T>* out = d.agm + lvl_off_[Lf];
   long as = (long)lvl_size_[Lf];
@@ -738,17 +743,38 @@ bool Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
   if (nb == 64 && sizeof(T) != 4) nb = 32;  // 64-box tiles: FP32 only (LDS)
   if (B % nb != 0) nb = 16;
   const dim3 grid(B / nb, nrhs);
-  auto go = [&](auto k) { k<<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act, st); };
+  // FP64: the mirror-symmetric kernel, with M2M of the leaf level for windows that the parents' band has
+  up = up && sym && m2m64_[Lf - 1].ncb > 0 && m2m64_[Lf - 1].kb <= kSymBand;
+  auto tile_nb = [&](auto m, auto n) {
+    constexpr int M = decltype(m)::value, NB = decltype(n)::value;
+    if constexpr (sizeof(T) == 8) {
+      if (S <= kP2mSymS) {
+        SymUp u;
+        if (up) {
+          u.par = d.agm + lvl_off_[Lf - 1];
+          u.ps = (long)lvl_size_[Lf - 1];
+          u.ab = d.band_m2m[Lf - 1];
+          u.s0 = d.bs0_m2m[Lf - 1];
+          u.shift = d.shiftM[Lf - 1];
+          u.Sp = P_.nsamp[Lf - 1];
+          u.kb = m2m64_[Lf - 1].kb;
+        }
+        auto k = up ? k_p2m_sym<NB, M, true> : k_p2m_sym<NB, M, false>;
+        k<<<grid, blk, p2m_sym_lds(NB, S), stream_>>>(y, P_.N, out, as, d.sym_p2m, S, act, st, u);
+        return;
+      }
+    }
+    k_p2m_mfma<T, TI, NB, M><<<grid, blk, 0, stream_>>>(y, P_.N, out, as, d.coeffT, S, act, st);
+  };
   auto tile = [&](auto m) {
-    constexpr int M = decltype(m)::value;
     if constexpr (sizeof(T) == 4)
-      if (nb == 64) return go(k_p2m_mfma<T, TI, 64, M>);
-    if (nb == 32) return go(k_p2m_mfma<T, TI, 32, M>);
-    go(k_p2m_mfma<T, TI, 16, M>);
+      if (nb == 64) return tile_nb(m, std::integral_constant<int, 64>());
+    if (nb == 32) return tile_nb(m, std::integral_constant<int, 32>());
+    tile_nb(m, std::integral_constant<int, 16>());
   };
   if (mode == 0) {
     tile(std::integral_constant<int, 0>());
-    return false;
+    return up;
   }
   // the solver's vector steps; contrast weighting alone (mode 1) serves the FP64 residual check
   bool done = false;
@@ -764,7 +790,7 @@ bool Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
       done = false;
   }
   if (!done) set_error("P2M: no kernel for this step on vectors of this type");
-  return false;
+  return up;
 }
 
 // child level i+1 -> parent level i
@@ -1052,7 +1078,7 @@ void Engine::apply(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, con
     step = &weight;
   }
   prof_begin(KT_P2M);
-  const bool up = launch_p2m<T, TI>(y, nrhs, act, -1, step, true);
+  const bool up = launch_p2m<T, TI>(y, nrhs, act, -1, step, L > 3);
   prof_end(KT_P2M);
   prof_begin(KT_INTERP);
   for (int i = up ? L - 3 : L - 2; i >= 2; i--) launch_m2m<T>(i, nrhs, act);
@@ -1124,8 +1150,8 @@ void Engine::aggregate(const zd* x, zd* r, int nrhs) {
     rx_apply(x, r, nrhs);
   } else {
     const int L = P_.L;
-    launch_p2m<double, double>(x, nrhs, nullptr);
-    for (int i = L - 2; i >= 0; i--) launch_m2m<double>(i, nrhs, nullptr);
+    const bool up = launch_p2m<double, double>(x, nrhs, nullptr, -1, nullptr, true);
+    for (int i = up ? L - 3 : L - 2; i >= 0; i--) launch_m2m<double>(i, nrhs, nullptr);
     int R = cfg_.plan.numrx;
     k_rx_interp<double><<<dim3(nblocks(R), nrhs), dim3(kBlock), 0, stream_>>>(
         op64_.agm + lvl_off_[0], (long)lvl_size_[0], r, R, op64_.rxT, rx0_, P_.nsamp[0], R, cfg_.plan.ninter);

@@ -58,6 +58,7 @@ struct DevOp {
   cplx<T>* basisT = nullptr;   // [S_leaf][64]
   cplx<T>* sym_near = nullptr;  // mirror-symmetric classes of both (k_sym_tables)
   cplx<T>* sym_l2p = nullptr;
+  double* sym_p2m = nullptr;  // k_sym_p2m_table (FP64)
   std::vector<T*> interpT, anterpT, band_m2m, band_l2l;  // band blocks [nrb][KB][16]
   std::vector<int*> bs0_m2m, bs0_l2l;                    // window start of each band block
   std::vector<cplx<T>*> shiftM, shiftL, trans;

@@ -989,34 +989,13 @@ k_m2l_par(M2LSet<T> set, const int* __restrict__ act) {
   for (int c = 0; c < 4; c++) out[(long)c * S + B.k0 + kk] = acc[c];
 }
 
-// P2M on the matrix cores: agm[box][k] = sum_n coeffT[n][k] y[box*64+n] for a
-// tile of NB boxes.  The work is cut into units of 16 rows k x 16 boxes, dealt
-// round-robin to the 4 waves: with S = 68 (5 row blocks) and 64-box tiles
-// every wave gets 5 units (whole row blocks per wave would leave three waves
-// idle half the time).  STEP: the vector step of P2mStep while loading; y is
-// unused then.
-// With S <= kP2mRows (at most 5 row blocks) the units' results stay in
-// registers until every wave is done, then go through LDS so that the tile's
-// contiguous output range [b0 S, (b0 + NB) S) is written with whole,
-// coalesced lines (stored from the MFMA layout, a box's row blocks came from
-// different waves and partial lines reached HBM separately).
-constexpr int kP2mRows = 80;
-template <typename T, typename TI, int NB, int STEP = 0>
-__global__ void __launch_bounds__(kBlock) k_p2m_mfma(const cplx<TI>* __restrict__ y, long ys,
-                                                     cplx<T>* __restrict__ agm, long as,
-                                                     const cplx<T>* __restrict__ coeffT, int S,
-                                                     const int* __restrict__ act, P2mStep<TI> step) {
-  typedef typename Mfma<T>::v4 v4;
-  constexpr int NN = NB / 16;
-  constexpr int MAXU = (5 * NN + 3) / 4;  // units per wave with 5 row blocks
-  __shared__ cplx<T> tile[NB * kP2mRows];  // input rows of 65, later the output rows of S
-  const int rhs = blockIdx.y;
-  if (rhs_off(act, rhs)) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const long b0 = (long)xcd_block() * NB;
+// Input of P2M: the NB x 64 pixels of boxes b0 .. of system rhs to tile[box][65],
+// or the vector step of P2mStep, which forms them (y is unused then).  Loads are
+// issued in groups ahead of their LDS stores.
+template <typename T, typename TI, int NB, int STEP>
+__device__ __forceinline__ void p2m_stage(cplx<T>* tile, const cplx<TI>* __restrict__ y, long ys, long b0, int rhs,
+                                          const P2mStep<TI>& step) {
   const cplx<TI>* yr = y + rhs * ys + b0 * 64;
-  // loads issued in groups ahead of their LDS stores
   if constexpr (STEP == 0) {
     stage<sizeof(T) == 4 ? 8 : 4, cplx<TI>>(
         NB * 64, [&](int idx) { return yr[idx]; },
@@ -1037,6 +1016,35 @@ __global__ void __launch_bounds__(kBlock) k_p2m_mfma(const cplx<TI>* __restrict_
           tile[(idx >> 6) * 65 + (idx & 63)] = ccast<T>(yv);
         });
   }
+}
+
+// P2M on the matrix cores: agm[box][k] = sum_n coeffT[n][k] y[box*64+n] for a
+// tile of NB boxes.  The work is cut into units of 16 rows k x 16 boxes, dealt
+// round-robin to the 4 waves: with S = 68 (5 row blocks) and 64-box tiles
+// every wave gets 5 units (whole row blocks per wave would leave three waves
+// idle half the time).  STEP: the vector step of P2mStep while loading; y is
+// unused then.  FP64 up to kP2mSymS samples goes to k_p2m_sym.
+// With S <= kP2mRows (at most 5 row blocks) the units' results stay in
+// registers until every wave is done, then go through LDS so that the tile's
+// contiguous output range [b0 S, (b0 + NB) S) is written with whole,
+// coalesced lines (stored from the MFMA layout, a box's row blocks came from
+// different waves and partial lines reached HBM separately).
+constexpr int kP2mRows = 80;
+template <typename T, typename TI, int NB, int STEP = 0>
+__global__ void __launch_bounds__(kBlock) k_p2m_mfma(const cplx<TI>* __restrict__ y, long ys,
+                                                     cplx<T>* __restrict__ agm, long as,
+                                                     const cplx<T>* __restrict__ coeffT, int S,
+                                                     const int* __restrict__ act, P2mStep<TI> step) {
+  typedef typename Mfma<T>::v4 v4;
+  constexpr int NN = NB / 16;
+  constexpr int MAXU = (5 * NN + 3) / 4;  // units per wave with 5 row blocks
+  __shared__ cplx<T> tile[NB * kP2mRows];  // input rows of 65, later the output rows of S
+  const int rhs = blockIdx.y;
+  if (rhs_off(act, rhs)) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  const long b0 = (long)xcd_block() * NB;
+  p2m_stage<T, TI, NB, STEP>(tile, y, ys, b0, rhs, step);
   __syncthreads();
   const int nrb = (S + 15) / 16, nunit = nrb * NN;
   const bool staged = S <= kP2mRows;
