@@ -304,18 +304,21 @@ k_down_h16(const zf* __restrict__ agm, zf* __restrict__ agl, long st, const zf* 
 // registers, the 27 operators are loaded once; per right-hand side the source
 // boxes and the parents' windows go to LDS.  Wave w owns child position w; the
 // rows of the matrix product are permuted so that a lane (li, lk) receives
-// parents 4 lk .. +3, a 2 x 2 block, as in k_down_h16.
+// parents 4 lk .. +3, a 2 x 2 block, as in k_down_h16.  FAR = false: the
+// interpolation alone (the transposed receiver product has no translations;
+// levels 3 .. 6 at 512 px x 16, 149 us as band and chunked kernels, 100 here).
 // FP64 work bounds it (an FP64 product of this chip's vector or matrix units
 // either way): 1024 px x 64 right-hand sides, M2L and L2L of levels 2 .. 7, 3140
 // us as separate kernels (M2L 1100, L2L 2040), 1940 here, of which about 1000 is
 // arithmetic at the rate of a large matrix product; 512 px x 16, 195 -> 168 us.
 // Grid (tiles * ceil(S / 16), ceil(nrhs / per)); level >= 3; KB <= kDownK.
+template <bool FAR>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
 k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __restrict__ trans, int lev, int S,
          const zd* __restrict__ par, long ps, int Sp, const double* __restrict__ AB, const int* __restrict__ s0v, int KB,
          const zd* __restrict__ shift, int nrhs, int per, const int* __restrict__ act) {
   typedef Mfma<double>::v4 v4;
-  constexpr int NS = kDownSB * kDownSB * kDownKC, NW = 16 * kDownK / kBlock, WP = kDownK + 1;
+  constexpr int NS = FAR ? kDownSB * kDownSB * kDownKC : 1, NW = 16 * kDownK / kBlock, WP = kDownK + 1;
   __shared__ zd src[NS], win[16 * WP], sh[4 * kDownK];  // win[parent][window]
   __shared__ double ab[kDownK * 16];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -335,7 +338,7 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
   const int ks = min(k0 + (tid & 15), S - 1);  // (samples past S are computed and not stored)
   unsigned soff[9];  // byte offsets; past the end (zeros) for boxes outside the grid
 #pragma unroll
-  for (int u = 0; u < 9; u++) {
+  for (int u = 0; FAR && u < 9; u++) {
     const int b = (tid >> 4) + 16 * u, bx = X0 - 2 + b % kDownSB, by = Y0 - 2 + b / kDownSB;
     const bool ok = bx >= 0 && by >= 0 && bx < nb && by < nb;
     soff[u] = ok ? (morton2(bx, by) * S + ks) * (unsigned)sizeof(zd) : 0xffffff00u;
@@ -358,12 +361,14 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
   }
   for (int e = tid; e < 16 * KB; e += kBlock) ab[e] = AB[(long)chunk * KB * 16 + e];
   zd t[kDownFar];
-  const int kt = min(k0 + li, S - 1);
-  switch (w) {
-    case 0: down_load_t<0, 0>(trans, S, kt, t); break;
-    case 1: down_load_t<1, 0>(trans, S, kt, t); break;
-    case 2: down_load_t<0, 1>(trans, S, kt, t); break;
-    default: down_load_t<1, 1>(trans, S, kt, t); break;
+  if constexpr (FAR) {
+    const int kt = min(k0 + li, S - 1);
+    switch (w) {
+      case 0: down_load_t<0, 0>(trans, S, kt, t); break;
+      case 1: down_load_t<1, 0>(trans, S, kt, t); break;
+      case 2: down_load_t<0, 1>(trans, S, kt, t); break;
+      default: down_load_t<1, 1>(trans, S, kt, t); break;
+    }
   }
   const unsigned mbytes = (unsigned)nb * nb * S * (unsigned)sizeof(zd), pbytes = (unsigned)nb * nb / 4 * Sp * (unsigned)sizeof(zd);
   const unsigned ooff = ((m0 + 16 * lk + w) * S + k0 + li) * (unsigned)sizeof(zd), ostep = 4 * S * (unsigned)sizeof(zd);
@@ -379,14 +384,14 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
       const __amdgpu_buffer_rsrc_t a = down_rsrc(agm + (long)r * st, mbytes), p = down_rsrc(par + (long)r * ps, pbytes);
       zd sv[9], wv[NW];
 #pragma unroll
-      for (int u = 0; u < 9; u++)
+      for (int u = 0; FAR && u < 9; u++)
         sv[u] = __builtin_bit_cast(zd, __builtin_amdgcn_raw_buffer_load_b128(a, (int)soff[u], 0, 0));
 #pragma unroll
       for (int u = 0; u < NW; u++)
         wv[u] = __builtin_bit_cast(zd, __builtin_amdgcn_raw_buffer_load_b128(p, (int)woff[u], 0, 0));
       __syncthreads();  // the previous right-hand side's sources are no longer read
 #pragma unroll
-      for (int u = 0; u < 9; u++) src[tid + kBlock * u] = sv[u];
+      for (int u = 0; FAR && u < 9; u++) src[tid + kBlock * u] = sv[u];
 #pragma unroll
       for (int u = 0; u < NW; u++) win[wdst[u]] = wv[u];  // (the clamped last ones repeat one element)
     }
@@ -401,17 +406,20 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
       ci = Mfma<double>::mac(v.y, a, ci);
     }
     // ---- translations
-    zd acc[4], first[4];
+    zd acc[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) acc[i] = mkc<double>(cr[i], ci[i]);
-    const zd* s = src + (4 * (lk >> 1) * kDownSB + 4 * (lk & 1)) * kDownKC + li;
+    if constexpr (FAR) {
+      zd first[4];
+      const zd* s = src + (4 * (lk >> 1) * kDownSB + 4 * (lk & 1)) * kDownKC + li;
 #pragma unroll
-    for (int x = 0; x < 4; x++) first[x] = s[x * kDownKC];
-    switch (w) {
-      case 0: down_m2l<0, 0, 4>(s, t, first, acc); break;
-      case 1: down_m2l<1, 0, 4>(s, t, first, acc); break;
-      case 2: down_m2l<0, 1, 4>(s, t, first, acc); break;
-      default: down_m2l<1, 1, 4>(s, t, first, acc); break;
+      for (int x = 0; x < 4; x++) first[x] = s[x * kDownKC];
+      switch (w) {
+        case 0: down_m2l<0, 0, 4>(s, t, first, acc); break;
+        case 1: down_m2l<1, 0, 4>(s, t, first, acc); break;
+        case 2: down_m2l<0, 1, 4>(s, t, first, acc); break;
+        default: down_m2l<1, 1, 4>(s, t, first, acc); break;
+      }
     }
     if (store) {
       char* o = reinterpret_cast<char*>(agl + (long)r * st);

@@ -606,7 +606,7 @@ int Engine::fuse_level(int choice, int nrhs) const {
 // M2L of level i and the L2L into it.  Right-hand sides per workgroup: as many
 // as leave four workgroups per CU, 8 at most.
 template <typename T>
-void Engine::launch_down(int i, int nrhs, const int* act) {
+void Engine::launch_down(int i, int nrhs, const int* act, bool far) {
   const int S = P_.nsamp[i], nb = 1 << i, blocks = nb * nb / (kDownTS * kDownTS) * ((S + kDownKC - 1) / kDownKC);
   const int per = (int)std::min<long>(8, std::max<long>(1, (long)blocks * nrhs / 1024));
   const DownLevel& d = down_[i];
@@ -619,8 +619,9 @@ void Engine::launch_down(int i, int nrhs, const int* act) {
     k_down_h16<<<grid, blk, 0, stream_>>>(m, l, st, o.trans[i], i, S, par, ps, P_.nsamp[i - 1], (const v8h*)d.tab, d.s0,
                                           d.kb, d.ec, nrhs, per, act);
   else
-    k_down64<<<grid, blk, 0, stream_>>>(m, l, st, o.trans[i], i, S, par, ps, P_.nsamp[i - 1], d.ab, d.s0,
-                                                       d.kb, o.shiftL[i - 1], nrhs, per, act);
+    (far ? k_down64<true> : k_down64<false>)<<<grid, blk, 0, stream_>>>(m, l, st, o.trans[i], i, S, par, ps,
+                                                                      P_.nsamp[i - 1], d.ab, d.s0, d.kb,
+                                                                      o.shiftL[i - 1], nrhs, per, act);
 }
 
 // ------------------------------------------------------- interpolation plan
@@ -1153,7 +1154,7 @@ void Engine::aggregate(const zd* x, zd* r, int nrhs) {
     const bool up = launch_p2m<double, double>(x, nrhs, nullptr, -1, nullptr, true);
     for (int i = up ? L - 3 : L - 2; i >= 0; i--) launch_m2m<double>(i, nrhs, nullptr);
     int R = cfg_.plan.numrx;
-    k_rx_interp<double><<<dim3(nblocks(R), nrhs), dim3(kBlock), 0, stream_>>>(
+    k_rx_interp<double><<<dim3((R + 63) / 64, nrhs), dim3(kBlock), 0, stream_>>>(
         op64_.agm + lvl_off_[0], (long)lvl_size_[0], r, R, op64_.rxT, rx0_, P_.nsamp[0], R, cfg_.plan.ninter);
     ISG_HIP(hipGetLastError());
   }
@@ -1171,10 +1172,12 @@ void Engine::aggregateh(const zd* r, zd* x, int nrhs) {
     const int L = P_.L;
     int R = cfg_.plan.numrx;
     double sc = (double)R * cfg_.plan.res * cfg_.plan.res;
-    k_rx_anterp<double><<<dim3(nblocks(P_.nsamp[0]), nrhs), dim3(kBlock), 0, stream_>>>(
+    k_rx_anterp<double><<<dim3((P_.nsamp[0] + 63) / 64, nrhs), dim3(kBlock), 0, stream_>>>(
         r, R, op64_.agl + lvl_off_[0], (long)lvl_size_[0], op64_.rxaT, rxaI_, P_.nsamp[0], 2 * cfg_.plan.ninter,
         sc);
-    for (int i = 0; i <= L - 2; i++) launch_l2l<double>(i, false, nrhs, nullptr);
+    const int fuse = fuse_level(tune(PREC_FP64, nrhs).leaf, nrhs);
+    for (int i = 0; i + 1 < std::min(fuse, L); i++) launch_l2l<double>(i, false, nrhs, nullptr);
+    for (int i = fuse; i < L; i++) launch_down<double>(i, nrhs, nullptr, false);
     launch_near<double, double>(nullptr, x, nrhs, nullptr, false);
     ISG_HIP(hipGetLastError());
   }

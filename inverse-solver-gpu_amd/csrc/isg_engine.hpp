@@ -213,7 +213,7 @@ class Engine {
   void launch_m2l_variant(int i, int nrhs, const int* act, int v);
   int fuse_level(int choice, int nrhs) const;
   template <typename T>
-  void launch_down(int i, int nrhs, const int* act);
+  void launch_down(int i, int nrhs, const int* act, bool far = true);  // far: with M2L (FP64 only without)
   template <typename T, typename TI>
   // returns the number of workgroups per right-hand side (partial sums of a post step)
   int launch_near(const cplx<TI>* y, cplx<TI>* r, int nrhs, const int* act, bool with_near, int force = -1,

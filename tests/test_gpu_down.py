@@ -50,3 +50,31 @@ def test_fused_downward_pass_matches_oracle(isg, level, ninter, nrhs):
             s.synchronize()
             check(r.cpu().numpy(), 1e-5 if prec else 1e-12, "FP%d leaf %d" % (32 if prec else 64, leaf))
         s.close()
+
+
+# receivers: 16, one more and one fewer than a workgroup's 64 outputs
+@pytest.mark.parametrize("level,ninter,nrhs,numrx", [(3, 30, 2, 65), (4, 24, 115, 63), (5, 30, 5, 16), (5, 40, 29, 64),
+                                                     (6, 30, 8, 65)])
+def test_receiver_products_match_oracle(isg, level, ninter, nrhs, numrx):
+    """aggregate and aggregateh (no translations on the way down) at the same sizes; bar 1e-12."""
+    import torch
+    print("receivers level", level, "ninter", ninter, "nrhs", nrhs, "numrx", numrx, flush=True)
+    o = oracle_for(level, numrx=numrx, ninter=ninter)
+    xs = [rand_c(np.random.default_rng(140 + k), o.N) for k in range(3)]
+    rs = [rand_c(np.random.default_rng(150 + k), numrx) for k in range(3)]
+    down, up = [o.aggregateh(v) for v in rs], [o.aggregate(v) for v in xs]
+    s = isg.Solver(level=level, numrx=numrx, max_rhs=nrhs, ninter=ninter)
+    x = torch.from_numpy(np.stack([xs[k % 3] for k in range(nrhs)])).cuda()
+    r = torch.from_numpy(np.stack([rs[k % 3] for k in range(nrhs)])).cuda()
+    xo, ro = torch.empty_like(x), torch.empty_like(r)
+    torch.cuda.synchronize()
+    for leaf in (-1, 1, 0):
+        s.tuning_set(0, 1 if nrhs >= 16 else 0, "leaf", 0, leaf)
+        s.aggregate_dev(x.data_ptr(), ro.data_ptr(), nrhs)
+        s.aggregateh_dev(xo.data_ptr(), r.data_ptr(), nrhs)
+        s.synchronize()
+        X, R = xo.cpu().numpy(), ro.cpu().numpy()
+        errs = [max(relerr(X[k], down[k % 3]), relerr(R[k], up[k % 3])) for k in range(nrhs)]
+        print("leaf %d: max relative difference %.2e" % (leaf, max(errs)), flush=True)
+        assert max(errs) < 1e-12, (leaf, errs)
+    s.close()
