@@ -75,8 +75,9 @@ typedef struct isg_config {
   double mixed_margin; /* mixed precision only: the FP32 solve runs to mixed_margin * toli on its
                           recursive residual before the FP64 check, so that the check rarely
                           needs a defect-correction round; 0 < mixed_margin <= 1 (default 0.5) */
-  int graph;       /* 1 (default): each BiCGSTAB iteration is captured once per solve as a HIP graph
-                      and replayed; 0: launched kernel by kernel.  Results are identical. */
+  int graph;       /* 1 (default): the BiCGSTAB iterations of small solves are captured as a HIP graph
+                      and replayed once the solve has taken several; 0: always launched kernel by
+                      kernel.  Results are identical. */
   double radius;   /* 0 (default): plane-wave transmitters and far-field receivers, as the reference
                       (setup_born.cpp:62-65, matvec_gpu.cu:351-361).  > 0: line-source transmitters
                       and point receivers equispaced on a circle of this radius (wavelengths):

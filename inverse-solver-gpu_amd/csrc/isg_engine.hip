@@ -131,6 +131,9 @@ int build_band(int M, int K, int nt, const std::vector<int>& first, const std::v
   return KB;
 }
 constexpr int kRefineRounds = 3;
+// BiCGSTAB iterations go to a graph after kGraphAfter of them, in solves of at most kGraphMaxElems elements.
+constexpr int kGraphAfter = 8;
+constexpr long kGraphMaxElems = 8192;
 
 // Largest LDS window (source samples) of a target chunk for the chunked
 // interpolation kernels, or -1 when the first-tap indices of some chunk are
@@ -1271,10 +1274,16 @@ void Engine::run_bicgs(zd* x, const zd* g, long gs, const zd* b, bool herm, int 
   k_bi_init<V><<<grid, blk, 0, stream_>>>(x, op, g, gs, b, r0, r, rt, N, h, x_zero ? 1 : 0, part_);
   k_bi_fin<<<dim3(nrhs), blk, 0, stream_>>>(PH_INIT, state_, active_, part_, nblk_, tolv_, maxit);
   maxit_ = maxit;
-  // one iteration = bicgs_body; with graphs it is captured once per call and
-  // replayed, the host reading the activity flags after each replay
+  // One iteration = bicgs_body, launched kernel by kernel: its ~20 launches take
+  // the host less than the kernels take the GPU.  Only below that, in the smallest
+  // solves, is an iteration cheaper as a graph, and capturing it costs 100 to 200 us,
+  // so it is captured when the solve turns out to be long.  us an iteration, launched /
+  // replayed: 64 px x 1 101 / 87, 128 px x 1 142 / 141, 256 px x 1 148 / 163, 512 px
+  // x 15 527 / 545; a solve of 2 iterations with a graph from the start, 64 px 226 ->
+  // 329 us, 256 px 341 -> 381, 512 px 446 -> 561.
   hipGraphExec_t exec = nullptr;
-  if (cfg_.graph && !prof_) {
+  const bool graph = cfg_.graph && !prof_ && N * nrhs <= kGraphMaxElems;
+  auto capture = [&] {
     hipGraph_t gr = nullptr;
     ISG_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     bicgs_body<V>(x, g, gs, herm, nrhs, prec);
@@ -1283,8 +1292,7 @@ void Engine::run_bicgs(zd* x, const zd* g, long gs, const zd* b, bool herm, int 
       ISG_HIP(hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0));
       (void)hipGraphDestroy(gr);
     }
-    if (!ok()) return;
-  }
+  };
   ISG_HIP(hipMemcpyAsync(active_h_, active_, nrhs * sizeof(int), hipMemcpyDeviceToHost, stream_));
   for (int it = 0; it <= maxit; it++) {
     ISG_HIP(hipStreamSynchronize(stream_));
@@ -1293,6 +1301,8 @@ void Engine::run_bicgs(zd* x, const zd* g, long gs, const zd* b, bool herm, int 
     int nact = 0;
     for (int i = 0; i < nrhs; i++) nact += active_h_[i] != 0;
     if (nact == 0) break;
+    if (graph && it == kGraphAfter) capture();
+    if (!ok()) break;
     if (exec)
       ISG_HIP(hipGraphLaunch(exec, stream_));
     else
