@@ -646,8 +646,7 @@ __global__ void __launch_bounds__(kBlock) k_interp_band(const cplx<T>* __restric
       pre[q] = mkc<T>(0, 0);
       if (k < Mrows) {
         if (MODE == 0) {
-          if (!Mfma<T>::kRowsAcrossLanes || q == 0)
-            pre[q] = shift[(Mfma<T>::kRowsAcrossLanes ? lk : q) * Mrows + k];
+          pre[q] = shift[q * Mrows + k];
         } else if (accumulate) {
           pre[q] = dst[rhs * ds + (4 * p0 + 16 * cb0 + Mfma<T>::row(lk, q)) * (long)Mrows + k];
         }
@@ -656,7 +655,9 @@ __global__ void __launch_bounds__(kBlock) k_interp_band(const cplx<T>* __restric
 #pragma unroll
     for (int cc = 0; cc < CPI; cc++) {
       const int cb = cb0 + cc;
-      const cplx<T>* tcol = tile + (16 * cb + li) * row;
+      // M2M: columns in the order that leaves the 4 siblings of parent 4 cb + lk to a lane
+      const int ci = MODE == 0 && Mfma<T>::kRowsAcrossLanes ? 4 * (li & 3) + (li >> 2) : li;
+      const cplx<T>* tcol = tile + (16 * cb + ci) * row;
       v4 cr0 = v4{0, 0, 0, 0}, ci0 = v4{0, 0, 0, 0};
 #pragma unroll
       for (int q = 0; q < KQ; q++) {
@@ -671,31 +672,15 @@ __global__ void __launch_bounds__(kBlock) k_interp_band(const cplx<T>* __restric
       // D[col][k]: lane li holds target sample k = 16 rb + li; col = 16 cb + row(lk, q)
       if (MODE == 0) {
         // parent = sum over the 4 sibling columns of shiftM[c][k] * D[col][k]
-        if (Mfma<T>::kRowsAcrossLanes) {
-          // col = 16cb + lk + 4q: sibling c = lk, parent 4cb + q
-          const cplx<T> s1 = pre[0];
+        T xr = 0, xi = 0;
 #pragma unroll
-          for (int q = 0; q < 4; q++) {
-            T vr = cr0[q], vi = ci0[q];
-            T xr = vr * s1.x - vi * s1.y, xi = vr * s1.y + vi * s1.x;
-            xr += __shfl_xor(xr, 16, 64);
-            xi += __shfl_xor(xi, 16, 64);
-            xr += __shfl_xor(xr, 32, 64);
-            xi += __shfl_xor(xi, 32, 64);
-            if (lk == 0 && k < Mrows) dst[rhs * ds + (p0 + 4 * cb + q) * Mrows + k] = mkc<T>(xr, xi);
-          }
-        } else {
-          // col = 16cb + 4lk + q: sibling c = q, parent 4cb + lk
-          T xr = 0, xi = 0;
-#pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const cplx<T> sq = pre[q];
-            T vr = cr0[q], vi = ci0[q];
-            xr += vr * sq.x - vi * sq.y;
-            xi += vr * sq.y + vi * sq.x;
-          }
-          if (k < Mrows) dst[rhs * ds + (p0 + 4 * cb + lk) * Mrows + k] = mkc<T>(xr, xi);
+        for (int q = 0; q < 4; q++) {
+          const cplx<T> sq = pre[q];
+          const T vr = cr0[q], vi = ci0[q];
+          xr += vr * sq.x - vi * sq.y;
+          xi += vr * sq.y + vi * sq.x;
         }
+        if (k < Mrows) dst[rhs * ds + (p0 + 4 * cb + lk) * Mrows + k] = mkc<T>(xr, xi);
       } else if (k < Mrows) {
 #pragma unroll
         for (int q = 0; q < 4; q++) {
