@@ -22,6 +22,7 @@ constexpr int kDownTS = 8, kDownSB = kDownTS + 4, kDownKC = 16;
 constexpr int kDownK = 96;                // window slots (three MFMA chunks)
 constexpr int kDownG = kDownK / 8;        // groups of 8 slots
 constexpr int kDownFrag = 4 * kDownG * 16;  // v8h fragments of a window: [part][group][parent]
+constexpr int kDownPer = 16;  // most right-hand sides of a workgroup (bits of `live`)
 constexpr int kDownFar = 27;
 
 // Table of one level: out[rb][c][part][g][col] = 8 FP16 parts of
@@ -353,6 +354,16 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
     woff[u] = (((m0 >> 2) + p) * Sp + j) * (unsigned)sizeof(zd);
     wdst[u] = p * WP + jj;
   }
+  const unsigned mbytes = (unsigned)nb * nb * S * (unsigned)sizeof(zd), pbytes = (unsigned)nb * nb / 4 * Sp * (unsigned)sizeof(zd);
+  zd wv[NW];
+  auto load_window = [&](int r) {
+    const __amdgpu_buffer_rsrc_t p = down_rsrc(par + (long)r * ps, pbytes);
+#pragma unroll
+    for (int u = 0; u < NW; u++)
+      wv[u] = __builtin_bit_cast(zd, __builtin_amdgcn_raw_buffer_load_b128(p, (int)woff[u], 0, 0));
+  };
+  int r = rg + __builtin_ctz(live);
+  load_window(r);
   for (int e = tid; e < 4 * KB; e += kBlock) {
     const int c = e / KB;
     int j = s0 + e - c * KB;
@@ -370,32 +381,29 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
       default: down_load_t<1, 1>(trans, S, kt, t); break;
     }
   }
-  const unsigned mbytes = (unsigned)nb * nb * S * (unsigned)sizeof(zd), pbytes = (unsigned)nb * nb / 4 * Sp * (unsigned)sizeof(zd);
   const unsigned ooff = ((m0 + 16 * lk + w) * S + k0 + li) * (unsigned)sizeof(zd), ostep = 4 * S * (unsigned)sizeof(zd);
   const bool store = k0 + li < S;
   const zd* wrow = win + (4 * (li & 3) + (li >> 2)) * WP + lk;  // this lane's row of the product
   const zd* srow = sh + w * KB + lk;
   const double* arow = ab + lk * 16 + li;
   const int nkq = KB >> 2;
-  while (live) {
-    const int r = rg + __builtin_ctz(live);
+  // The sources of a right-hand side and the next one's windows are in flight
+  // during the interpolation.
+#pragma unroll
+  for (int u = 0; u < NW; u++) win[wdst[u]] = wv[u];  // (the clamped last ones repeat one element)
+  __syncthreads();
+  for (;;) {
     live &= live - 1;
-    {
-      const __amdgpu_buffer_rsrc_t a = down_rsrc(agm + (long)r * st, mbytes), p = down_rsrc(par + (long)r * ps, pbytes);
-      zd sv[9], wv[NW];
+    const bool more = live != 0;
+    const int rn = more ? rg + __builtin_ctz(live) : r;
+    zd sv[9];
+    if constexpr (FAR) {
+      const __amdgpu_buffer_rsrc_t a = down_rsrc(agm + (long)r * st, mbytes);
 #pragma unroll
-      for (int u = 0; FAR && u < 9; u++)
+      for (int u = 0; u < 9; u++)
         sv[u] = __builtin_bit_cast(zd, __builtin_amdgcn_raw_buffer_load_b128(a, (int)soff[u], 0, 0));
-#pragma unroll
-      for (int u = 0; u < NW; u++)
-        wv[u] = __builtin_bit_cast(zd, __builtin_amdgcn_raw_buffer_load_b128(p, (int)woff[u], 0, 0));
-      __syncthreads();  // the previous right-hand side's sources are no longer read
-#pragma unroll
-      for (int u = 0; FAR && u < 9; u++) src[tid + kBlock * u] = sv[u];
-#pragma unroll
-      for (int u = 0; u < NW; u++) win[wdst[u]] = wv[u];  // (the clamped last ones repeat one element)
     }
-    __syncthreads();
+    if (more) load_window(rn);
     // ---- interpolation: rows = parents, columns = samples
     v4 cr = v4{0, 0, 0, 0}, ci = v4{0, 0, 0, 0};
 #pragma unroll 4
@@ -405,6 +413,16 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
       cr = Mfma<double>::mac(v.x, a, cr);
       ci = Mfma<double>::mac(v.y, a, ci);
     }
+    if (FAR || more) __syncthreads();  // windows and the previous right-hand side's sources are no longer read
+    if constexpr (FAR) {
+#pragma unroll
+      for (int u = 0; u < 9; u++) src[tid + kBlock * u] = sv[u];
+    }
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < NW; u++) win[wdst[u]] = wv[u];
+    }
+    if (FAR || more) __syncthreads();
     // ---- translations
     zd acc[4];
 #pragma unroll
@@ -426,6 +444,8 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
 #pragma unroll
       for (int i = 0; i < 4; i++) *reinterpret_cast<zd*>(o + (ooff + i * ostep)) = acc[i];
     }
+    if (!more) break;
+    r = rn;
   }
 }
 

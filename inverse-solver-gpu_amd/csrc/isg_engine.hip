@@ -606,12 +606,32 @@ int Engine::fuse_level(int choice, int nrhs) const {
   return choice == 1 || (long)P_.B * nrhs < 7168 ? P_.L - 1 : 3;
 }
 
-// M2L of level i and the L2L into it.  Right-hand sides per workgroup: as many
-// as leave four workgroups per CU, 8 at most.
+// Right-hand sides per workgroup of the fused downward kernels, of `blocks`
+// workgroups each: a workgroup's tables cost about as much as 1.5 right-hand sides
+// and two workgroups fit a CU, so the choice with the fewest rounds x (1.5 + per).
+// Against as many as leave four workgroups per CU (8 at most): 512 px x 15 FP32 96.5
+// -> 90.6 us, 256 px x 7 37 -> 34, 1024 px x 64 1087 -> 1040, 512 px x 16 FP64 164 ->
+// 160 (weights from 0.7 to 4 measured alike).
+static int down_per(int blocks, int nrhs) {
+  const long slots = 512;
+  int best = 1;
+  double cost = 0;
+  for (int per = 1; per <= std::min(kDownPer, nrhs); per++) {
+    const long groups = (nrhs + per - 1) / per, rounds = (blocks * groups + slots - 1) / slots;
+    const double c = rounds * (1.5 + per);
+    if (per == 1 || c < cost) {
+      cost = c;
+      best = per;
+    }
+  }
+  return best;
+}
+
+// M2L of level i and the L2L into it.
 template <typename T>
 void Engine::launch_down(int i, int nrhs, const int* act, bool far) {
   const int S = P_.nsamp[i], nb = 1 << i, blocks = nb * nb / (kDownTS * kDownTS) * ((S + kDownKC - 1) / kDownKC);
-  const int per = (int)std::min<long>(8, std::max<long>(1, (long)blocks * nrhs / 1024));
+  const int per = down_per(blocks, nrhs);
   const DownLevel& d = down_[i];
   DevOp<T>& o = ops<T>();
   const dim3 grid(blocks, (nrhs + per - 1) / per), blk(kBlock);
