@@ -310,8 +310,8 @@ k_down_h16(const zf* __restrict__ agm, zf* __restrict__ agl, long st, const zf* 
 // levels 3 .. 6 at 512 px x 16, 149 us as band and chunked kernels, 100 here).
 // FP64 work bounds it (an FP64 product of this chip's vector or matrix units
 // either way): 1024 px x 64 right-hand sides, M2L and L2L of levels 2 .. 7, 3140
-// us as separate kernels (M2L 1100, L2L 2040), 1940 here, of which about 1000 is
-// arithmetic at the rate of a large matrix product; 512 px x 16, 195 -> 168 us.
+// us as separate kernels (M2L 1100, L2L 2040), 1890 here, of which about 1000 is
+// arithmetic at the rate of a large matrix product; 512 px x 16, 195 -> 150 us.
 // Grid (tiles * ceil(S / 16), ceil(nrhs / per)); level >= 3; KB <= kDownK.
 template <bool FAR>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
@@ -364,13 +364,20 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
   };
   int r = rg + __builtin_ctz(live);
   load_window(r);
-  for (int e = tid; e < 4 * KB; e += kBlock) {
-    const int c = e / KB;
+  // (the tables' loads are all issued before the first is stored: as loops of load
+  // and store they were six waits in a row, half of a small level's time)
+  constexpr int NA = 16 * kDownK / kBlock, NH = (4 * kDownK + kBlock - 1) / kBlock;
+  double av[NA];
+  zd hv[NH];
+#pragma unroll
+  for (int u = 0; u < NH; u++) {
+    const int e = min(tid + kBlock * u, 4 * KB - 1), c = e / KB;
     int j = s0 + e - c * KB;
     if (j >= Sp) j -= Sp;
-    sh[e] = shift[c * Sp + j];
+    hv[u] = shift[c * Sp + j];
   }
-  for (int e = tid; e < 16 * KB; e += kBlock) ab[e] = AB[(long)chunk * KB * 16 + e];
+#pragma unroll
+  for (int u = 0; u < NA; u++) av[u] = AB[(long)chunk * KB * 16 + min(tid + kBlock * u, 16 * KB - 1)];
   zd t[kDownFar];
   if constexpr (FAR) {
     const int kt = min(k0 + li, S - 1);
@@ -381,6 +388,10 @@ k_down64(const zd* __restrict__ agm, zd* __restrict__ agl, long st, const zd* __
       default: down_load_t<1, 1>(trans, S, kt, t); break;
     }
   }
+#pragma unroll
+  for (int u = 0; u < NH; u++) sh[min(tid + kBlock * u, 4 * KB - 1)] = hv[u];
+#pragma unroll
+  for (int u = 0; u < NA; u++) ab[min(tid + kBlock * u, 16 * KB - 1)] = av[u];
   const unsigned ooff = ((m0 + 16 * lk + w) * S + k0 + li) * (unsigned)sizeof(zd), ostep = 4 * S * (unsigned)sizeof(zd);
   const bool store = k0 + li < S;
   const zd* wrow = win + (4 * (li & 3) + (li >> 2)) * WP + lk;  // this lane's row of the product
