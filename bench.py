@@ -32,9 +32,8 @@ Paths, all from the same measurements:
           first-order start (isg_dbim field_start 3);
   fast    the same with the first-order total-field start alone (no network);
   plain   FP64 operator, one right-hand side at a time, every solve from zero:
-          the reference's loop on this library's kernels, each BiCGSTAB
-          iteration replayed as a HIP graph, the dense receiver operator
-          applied once per phase for all transmitters.
+          the reference's loop on this library's kernels, the dense receiver
+          operator applied once per phase for all transmitters.
 The reference geometry (plane waves, far-field receivers; --radius 0) is timed
 as well, one 5-iteration cycle per path ("reference_geometry").
 
@@ -199,9 +198,9 @@ def run_paths(isg, args, wl, common, otrue, mes, paths, warmup, steps, timing):
         if p == "plain":
             s = isg.Solver(max_rhs=1, **common)
             d = isg.Dbim(s, otrue, field_start=0, measurements=mes)
-            # timed at its best: without live kernel timers, so that each BiCGSTAB iteration
-            # replays as a HIP graph (its single-RHS kernels are short enough for launch
-            # overhead to show), unless it is the only path and supplies the roofline figures
+            # timed at its best: without live kernel timers (its single-RHS kernels are short
+            # enough for their events to show), unless it is the only path and supplies the
+            # roofline figures
             ptime = timing and paths == ["plain"]
         else:
             s = isg.Solver(**fast_kw, **common)
@@ -217,9 +216,9 @@ def run_paths(isg, args, wl, common, otrue, mes, paths, warmup, steps, timing):
                 s.close()
                 continue
             ptime = timing
-            # M2L and L2L of a level in one kernel: the leaf (1) or, FP32, every level (-1, the built-in rule)
+            # M2L and L2L of a level in one kernel: the leaf (1) or every level (-1, the built-in rule at these sizes)
             leaf = s.tuning_get(fast_prec, 1, "leaf")
-            fused = fused or leaf == 1 or (leaf == -1 and fast_prec == 1)
+            fused = fused or leaf in (-1, 1)
             # the split-FP16 near field k_near_h16 (tuning values 128 and 256) serves grids of >= 8 x 8
             # leaf boxes; the built-in rule (-1) takes it from 256 workgroups of 64 boxes on
             nv = s.tuning_get(1, 1 if batch >= 16 else 0, "near")
@@ -332,8 +331,8 @@ def main():
     ap.add_argument("--tuning", default="committed",
                     help="kernel-variant cache: 'committed' (inverse-solver-gpu_amd/tuning), 'none' or a path")
     ap.add_argument("--kernel-timing", default="on", choices=["on", "off"],
-                    help="live HIP-event kernel timing in the batched paths' timed regions (off: BiCGSTAB "
-                         "iterations replay as HIP graphs, no roofline figures)")
+                    help="live HIP-event kernel timing in the batched paths' timed regions (off: no "
+                         "roofline figures)")
     ap.add_argument("--radius", type=float, default=None,
                     help="transmitter/receiver circle radius in wavelengths (0: plane waves, far-field "
                          "receivers; default: the workload's, 60 at 1024^2)")
@@ -499,7 +498,8 @@ def main():
     }
     if timing:
         # GPU time of the live-timed kernel groups per step (HIP events on the solver's stream;
-        # near/m2l are the FP64 operator, *_fp32 the FP32 one, p2m/interp either precision,
+        # near/m2l are the FP64 operator (m2l with the L2L of its levels), *_fp32 the FP32 one,
+        # p2m (with the leaf level's M2M and the solver's p and s updates) / interp either precision,
         # receivers the receiver operator calls)
         out["kernel_timers_ms_per_step"] = {k: round(v[0] / args.steps, 3) for k, v in prof.items() if v[1] > 0}
     if main_path == "learned":

@@ -33,9 +33,9 @@ struct EngineConfig {
   int max_rhs = 1;        // right-hand sides solved together
   int precision = 0;      // PREC_MIXED also builds the FP32 operator
   double mixed_margin = 0.5;  // FP32 solve target = mixed_margin * tol before the FP64 check
-  bool graph = true;          // replay each BiCGSTAB iteration as one captured HIP graph
-                              // (not while live kernel timing is on: HIP events recorded
-                              // by graph nodes carry no timestamps)
+  bool graph = true;          // replay the BiCGSTAB iterations of long small solves as a
+                              // captured HIP graph (not while live kernel timing is on: HIP
+                              // events recorded by graph nodes carry no timestamps)
   int rx_rhs = 0;             // finite-radius receivers: right-hand sides one aggregate /
                               // aggregateh call may take (at least max_rhs), so that a
                               // caller solving one transmitter at a time can still apply

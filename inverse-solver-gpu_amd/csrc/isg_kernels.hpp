@@ -2,10 +2,12 @@
 // vector algebra, written for gfx950 (64-lane wavefronts, 256-thread blocks).
 //
 // Operator stages (reference counterparts in parentheses):
-//   k_p2m_mfma   leaf radiation patterns on the matrix cores (kernels.cu:6-30)
-//   k_m2m_lds    child -> parent interpolate+shift  (kernels.cu:83-136)
-//   k_m2l_tile   diagonal translation               (kernels.cu:239-266)
-//   k_l2l_lds    parent -> child shift+anterpolate  (kernels.cu:137-238)
+//   k_p2m_mfma, k_p2m_sym (isg_p2m_sym.hpp), k_p2m_h16 (isg_near_h16.hpp)
+//                leaf radiation patterns on the matrix cores (kernels.cu:6-30)
+//   k_interp_band, k_m2m_chunk, k_m2m   child -> parent interpolate+shift (kernels.cu:83-136)
+//   k_m2l_par, k_m2l_tile, k_m2l_reg    diagonal translation (kernels.cu:239-266)
+//   k_interp_band, k_l2l_chunk, k_l2l   parent -> child shift+anterpolate (kernels.cu:137-238)
+//   k_down_h16, k_down64 (isg_down.hpp) translation and anterpolation of a level in one
 //   k_near_mfma (isg_near_sym.hpp)  near field + leaf receiving patterns on the
 //                matrix cores                     (kernels.cu:32-81, :292-319)
 //   k_rx_*    receiver interpolation / anterpolation (matvec_gpu.cu:351-361, :395-401)

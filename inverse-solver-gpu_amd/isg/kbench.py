@@ -6,7 +6,7 @@ Runs `reps` batched matvecs (nrhs right-hand sides; FP64 operator, FP32
 operator on FP64 vectors, or with --vec32 the FP32 operator on FP32 vectors
 as the mixed-precision solver runs it) with live kernel timing and prints
 one JSON line with the near-field, M2L, P2M and interpolation (M2M + L2L)
-launch times.  --copy-mib adds a
+launch times (the leaf level's M2M counts with P2M, fused L2L with M2L).  --copy-mib adds a
 plain device-to-device copy of that many MiB, whose memory counters
 calibrate FETCH_SIZE / WRITE_SIZE readings of the same profiler run.
 Device buffers come from torch, imported before the library starts HIP.
@@ -30,8 +30,8 @@ def main():
     ap.add_argument("--reps", type=int, default=3)
     ap.add_argument("--copy-mib", type=int, default=0)
     ap.add_argument("--near", type=int, default=None,
-                    help="force the near-field variant (16, 32 or 64 boxes per tile; 128: the split-FP16 kernel of the FP32 "
-                         "operator on pairs of right-hand sides, 256: the same on 128-box tiles of one)")
+                    help="force the near-field variant (16, 32 or 64 boxes per tile; 128 or 256: the split-FP16 kernel of "
+                         "the FP32 operator)")
     ap.add_argument("--p2m", type=int, default=None,
                     help="force the P2M variant (16, 32 or 64 boxes per tile; 128: the split-FP16 kernel of the FP32 "
                          "operator)")
