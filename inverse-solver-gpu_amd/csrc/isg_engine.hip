@@ -728,24 +728,31 @@ template <typename T, typename TI>
 bool Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, const P2mStep<TI>* step, bool up) {
   const int Lf = P_.L - 1, S = P_.nsamp[Lf], B = P_.B;
   const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).p2m_nb;
-  // built-in rule: 32-box tiles once they fill the chip, else 16 (64 px, one system: 12.9 -> 9.6 us); the
-  // FP64 mirror-symmetric kernel 16 everywhere (512 px x 16: 55 us, 32-box tiles 61; 1024 px x 64: 870, 910)
+  // built-in rule: where a kernel does the leaf level's M2M along with P2M, that one -- FP32: the split-FP16
+  // kernel, a product of 64 px x 1 38 -> 30 us, 128 px x 1 62 -> 54, 256 px x 1 54.5 -> 51, x 7 70 -> 68.5,
+  // 512 px x 1 65.7 -> 66.5, x 8 135 -> 121, 1024 px x 2 146 -> 133; FP64: the mirror-symmetric one on 16-box
+  // tiles (512 px x 16: 55 us, 32-box tiles 61; 1024 px x 64: 870, 910) --, else the dense kernel on 32-box
+  // tiles once they fill the chip and 16 below (64 px, one system: 12.9 -> 9.6 us)
   const bool sym = sizeof(T) == 8 && S <= kP2mSymS;
-  int nb = force > 0 ? force : (tuned > 0 ? tuned : (!sym && (long)(B / 32) * nrhs >= 256 ? 32 : 16));
+  const int mode = step ? step->mode : 0;
+  const bool h16 = sizeof(T) == 4 && sizeof(TI) == 4 && mode != 1 && B % 32 == 0 && p2m16_;
+  const bool h16_up = h16 && up && up16_;
+  int nb = force > 0 ? force
+                     : (tuned > 0 ? tuned
+                                  : (h16_up ? kNearSplit : (!sym && (long)(B / 32) * nrhs >= 256 ? 32 : 16)));
   DevOp<T>& d = ops<T>();
   cplx<T>* out = d.agm + lvl_off_[Lf];
   long as = (long)lvl_size_[Lf];
-  const int mode = step ? step->mode : 0;
   const P2mStep<TI> st = step ? *step : P2mStep<TI>();
   const dim3 blk(kBlock);
   if (nb == kNearSplit) {
-    // split-FP16 P2M: FP32 operator on FP32 vectors, 32-box tiles of two
-    // right-hand sides (below 4 the workgroups are few and half idle)
+    // split-FP16 P2M: FP32 operator on FP32 vectors, 32-box tiles of two right-hand sides (without the
+    // M2M not below 4: the workgroups are few and half idle)
     if constexpr (sizeof(T) == 4 && sizeof(TI) == 4) {
-      if (mode != 1 && B % 32 == 0 && p2m16_ && (nrhs >= 4 || force == kNearSplit)) {
+      if (h16 && (nrhs >= 4 || h16_up || force == kNearSplit)) {
         dim3 grid(B / 32, (nrhs + 1) / 2);
         P2mUp u;
-        up = up && up16_;
+        up = h16_up;
         if (up) {
           u.par = d.agm + lvl_off_[Lf - 1];
           u.ps = (long)lvl_size_[Lf - 1];
@@ -1671,7 +1678,10 @@ void Engine::autotune_prec(int nrhs, int reps) {
     if (c == 3) return sizeof(T) == 4 && P_.B % 32 == 0 && p2m16_ != nullptr;
     return P_.B % widths[c] == 0 && (widths[c] < 64 || sizeof(T) == 4);
   };
-  c = pick(4, p2m_ok, [&](int c) { launch_p2m<T, T>((const cplx<T>*)y, nrhs, nullptr, widths[c]); });
+  c = pick(4, p2m_ok, [&](int c) {  // with the leaf level's M2M, which some of them do themselves
+    if (!launch_p2m<T, T>((const cplx<T>*)y, nrhs, nullptr, widths[c], nullptr, L > 3) && L > 3)
+      launch_m2m<T>(L - 2, nrhs, nullptr);
+  });
   tu.p2m_nb = c < 0 ? -1 : widths[c];
   for (int i = 2; i <= Lf; i++)
     tu.m2l[i] = pick(
