@@ -54,19 +54,6 @@ __device__ __forceinline__ void h16_split(float v, v8h& hi, v8h& lo, int e) {
   lo[e] = (_Float16)(v - (float)h);  // exact difference: at most 13 significant bits
 }
 
-// Four complex values (two float4) scaled by s and split into the four parts
-// (re hi, re lo, im hi, im lo), elements e0 .. e0 + 3 of each part.
-__device__ __forceinline__ void h16_split4(float4 a, float4 b, float s, v8h (&ph)[4], int e0) {
-  h16_split(a.x * s, ph[0], ph[1], e0);
-  h16_split(a.y * s, ph[2], ph[3], e0);
-  h16_split(a.z * s, ph[0], ph[1], e0 + 1);
-  h16_split(a.w * s, ph[2], ph[3], e0 + 1);
-  h16_split(b.x * s, ph[0], ph[1], e0 + 2);
-  h16_split(b.y * s, ph[2], ph[3], e0 + 2);
-  h16_split(b.z * s, ph[0], ph[1], e0 + 3);
-  h16_split(b.w * s, ph[2], ph[3], e0 + 3);
-}
-
 __device__ __forceinline__ float h16_absmax(float4 v) {
   return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
