@@ -139,7 +139,8 @@ struct P2mStep {
   long gs = 0;
   int herm = 0;
   BiState* st = nullptr;
-  const double2* part = nullptr;  // mode 3: nblk partial sums per system
+  const double2* part = nullptr;  // mode 3: nblk partial sums per system, pstride apart
+  long pstride = 0;
   int nblk = 0;
 };
 

@@ -134,6 +134,14 @@ constexpr int kRefineRounds = 3;
 // BiCGSTAB iterations go to a graph after kGraphAfter of them, in solves of at most kGraphMaxElems elements.
 constexpr int kGraphAfter = 8;
 constexpr long kGraphMaxElems = 8192;
+// The near field's partials are summed by every workgroup that needs the sum, up to
+// this many partials read a launch; from there on by k_bi_reduce beforehand.  Left to
+// the workgroups the reads grow with the square of the domain (FP64, one system:
+// 2^20 at 1024^2, 2^32 at 8192^2).  Iteration, summed by all / beforehand: 512^2 x 1
+// (2^16) 203 / 206 us, 1024^2 x 4 (2^22) 954 / 956, 1024^2 x 16 and 2048^2 x 1 (2^24)
+// alike, 4096^2 x 1 (2^28) 3.81 / 3.64 ms, 8192^2 x 1 (2^32) 17.9 / 14.4 ms; FP32
+// 1024^2 x 64 (2^23) and 2048^2 x 13 (2^24.7) alike.
+constexpr long kPartReads = 1L << 24;
 
 // Largest LDS window (source samples) of a target chunk for the chunked
 // interpolation kernels, or -1 when the first-tap indices of some chunk are
@@ -1342,6 +1350,15 @@ void Engine::run_bicgs(zd* x, const zd* g, long gs, const zd* b, bool herm, int 
   ISG_HIP(hipStreamSynchronize(stream_));
 }
 
+template <int NS>
+Engine::NearPart Engine::near_part(int nrhs, long readers) {
+  const int n = near_blocks_;
+  const long stride = (long)kSlots * n;
+  if (n < 2 || NS * n * readers * nrhs < kPartReads) return {part_, stride, n};
+  k_bi_reduce<NS><<<dim3(nrhs), dim3(kBlock), 0, stream_>>>(part_, n, active_);
+  return {part_ + 2 * n, stride, 1};
+}
+
 // One BiCGSTAB iteration for every active system (bicgs_gpu.cu:146-213),
 // ending with the copy of the activity flags to the host.  No memset: the
 // sequence is captured into a graph.
@@ -1376,8 +1393,10 @@ void Engine::bicgs_body(zd* x, const zd* g, long gs, bool herm, int nrhs, int pr
   apply_vec<V>(y, v, nrhs, active_, prec, &post, &step);
   step.mode = 3;
   step.p = s;
-  step.part = part_;
-  step.nblk = near_blocks_;
+  const NearPart pa = near_part<1>(nrhs, P_.B / (sizeof(V) == 4 ? 32 : 16));  // P2M's tiles
+  step.part = pa.part;
+  step.pstride = pa.stride;
+  step.nblk = pa.n;
   post.mode = 2;
   post.x = s;
   post.rt = nullptr;
@@ -1385,8 +1404,9 @@ void Engine::bicgs_body(zd* x, const zd* g, long gs, bool herm, int nrhs, int pr
   // omega's partials are in part_, so the residual's go to y, which is free until
   // the next product (kSlots nblk_ of 16 bytes; N >= 1024 nblk_ or nblk_ = 1)
   double2* rpart = reinterpret_cast<double2*>(y);
+  const NearPart po = near_part<2>(nrhs, nblk_);
   prof_begin(KT_VEC);
-  k_bi_xrupd<V><<<grid, blk, 0, stream_>>>(x, p, s, t, r, rt, N, state_, part_, near_blocks_, rpart);
+  k_bi_xrupd<V><<<grid, blk, 0, stream_>>>(x, p, s, t, r, rt, N, state_, po.part, po.stride, po.n, rpart);
   prof_end(KT_VEC);
   k_bi_fin<<<dim3(nrhs), blk, 0, stream_>>>(PH_RESID, state_, active_, rpart, nblk_, tolv_, maxit_);
   ISG_HIP(hipMemcpyAsync(active_h_, active_, nrhs * sizeof(int), hipMemcpyDeviceToHost, stream_));

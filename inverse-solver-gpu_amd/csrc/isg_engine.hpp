@@ -252,6 +252,14 @@ class Engine {
   void prof_begin(int id, bool new_set = true);
   void prof_end(int id);
   void harvest();
+  // the near field's partial sums of a post step, for `readers` workgroups per system
+  struct NearPart {
+    const double2* part;
+    long stride;  // between systems
+    int n;        // per system and slot
+  };
+  template <int NS>
+  NearPart near_part(int nrhs, long readers);
   template <typename V>
   void bicgs_body(zd* x, const zd* g, long gs, bool herm, int nrhs, int prec);
   void* dalloc(size_t bytes);

@@ -263,8 +263,9 @@ __device__ __forceinline__ void part_sum(const double2* __restrict__ pr, int nbl
 // The vector step of P2mStep, element by element (o: the system's offset,
 // element i of it; load only loads, so that a group's loads are in flight
 // together).  Every element belongs to one workgroup.  alpha is summed by each
-// workgroup from at most B / 16 partials in L2 (a kernel of one workgroup per
-// system between the two products cost 5 us of latency); the first stores it.
+// workgroup from the near field's partials (a kernel of one workgroup per system
+// between the two products costs 5 us of latency; where the workgroups are too
+// many for that, k_bi_reduce has left one partial per system); the first stores it.
 template <typename V>
 struct StepIn {
   cplx<V> r, p, v;
@@ -285,7 +286,7 @@ __device__ __forceinline__ StepCoef step_coef(const P2mStep<V>& q, int rhs, void
     c.first = S.first != 0;
   } else if constexpr (STEP == 3) {
     zd t[1];
-    part_sum<1>(q.part + (long)rhs * kSlots * q.nblk, q.nblk, t, static_cast<double(*)[kBlock / 64]>(lds));
+    part_sum<1>(q.part + rhs * q.pstride, q.nblk, t, static_cast<double(*)[kBlock / 64]>(lds));
     const zd al = zdiv(q.st[rhs].rho, t[0]);
     if (blockIdx.x == 0 && threadIdx.x == 0) q.st[rhs].alpha = al;
     c.a = mkc<double>(-al.x, -al.y);

@@ -55,21 +55,36 @@ __global__ void __launch_bounds__(kBlock) k_bi_init(const zd* __restrict__ x, co
   block_store<2>(acc, part + (long)rhs * kSlots * gridDim.x, gridDim.x, blockIdx.x);
 }
 
-// omega = <t,s> / <t,t> from the near field's partials (nnear per system, summed
-// by every workgroup; the first stores it).  part must not overlap them.
+// Sums of slots 0 .. NS - 1 of each system's nblk partials, in part_sum's order,
+// into the first elements of its slot 2 (nblk >= NS), which the near field's post
+// steps leave alone.  Every reader of the partials would form them otherwise.
+template <int NS>
+__global__ void __launch_bounds__(kBlock) k_bi_reduce(double2* part, int nblk, const int* __restrict__ act) {
+  const int rhs = blockIdx.x;
+  if (rhs_off(act, rhs)) return;
+  __shared__ double sh[2 * NS][kBlock / 64];
+  double2* pr = part + (long)rhs * kSlots * nblk;
+  zd tot[NS];
+  part_sum<NS>(pr, nblk, tot, sh);
+  if (threadIdx.x == 0)
+    for (int s = 0; s < NS; s++) pr[2 * nblk + s] = make_double2(tot[s].x, tot[s].y);
+}
+
+// omega = <t,s> / <t,t> from nnear partials per system, nstride apart (summed by
+// every workgroup; the first stores it).  part must not overlap them.
 template <typename V>
 __global__ void __launch_bounds__(kBlock) k_bi_xrupd(zd* __restrict__ x, const cplx<V>* __restrict__ p,
                                                      const cplx<V>* __restrict__ s, const cplx<V>* __restrict__ t,
                                                      cplx<V>* __restrict__ r, const cplx<V>* __restrict__ rt, long N,
                                                      BiState* __restrict__ st, const double2* __restrict__ near_part,
-                                                     int nnear, double2* __restrict__ part) {
+                                                     long nstride, int nnear, double2* __restrict__ part) {
   int rhs = blockIdx.y;
   BiState& S = st[rhs];
   if (!S.active) return;
   long o = rhs * N;
   __shared__ double sh[4][kBlock / 64];
   zd dot[2];
-  part_sum<2>(near_part + (long)rhs * kSlots * nnear, nnear, dot, sh);
+  part_sum<2>(near_part + rhs * nstride, nnear, dot, sh);
   const double tt = dot[1].x;
   zd om = mkc<double>(dot[0].x / tt, dot[0].y / tt);
   if (zabs(dot[0]) < 1e-200 && tt < 1e-200) om = mkc<double>(1.0, 0.0);
