@@ -178,6 +178,8 @@ int isg_stage(isg_context* ctx, int which, int level, int rhs, double* out);
  * out[0] single-RHS matvecs (mom.cpp:61), out[1] solves, out[2] solver iterations,
  * out[3] matvecs with the FP32 operator, out[4] defect-correction solves (5 entries) */
 int isg_counters(const isg_context* ctx, long long* out);
+/* solver iterations since creation that ran as replays of a captured HIP graph (isg_config.graph) */
+int isg_graph_replays(const isg_context* ctx, long long* out);
 
 /* ---- DBIM / nonlinear-CG inversion (mom.cpp:222-400, setup_born.cpp) ---- */
 typedef struct isg_dbim_stats {

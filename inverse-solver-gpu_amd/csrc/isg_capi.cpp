@@ -365,6 +365,12 @@ int isg_counters(const isg_context* c, long long* out) {
   return ISG_OK;
 }
 
+int isg_graph_replays(const isg_context* c, long long* out) {
+  if (!c || !c->eng || !out) return ISG_E_ARG;
+  *out = c->eng->graph_replays;
+  return ISG_OK;
+}
+
 static void fill_stats(const isg::DbimStats& s, isg_dbim_stats* o) {
   if (!o) return;
   o->alpha = s.alpha;

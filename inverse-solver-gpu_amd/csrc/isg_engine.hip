@@ -1338,10 +1338,12 @@ void Engine::run_bicgs(zd* x, const zd* g, long gs, const zd* b, bool herm, int 
     if (nact == 0) break;
     if (graph && it == kGraphAfter) capture();
     if (!ok()) break;
-    if (exec)
+    if (exec) {
       ISG_HIP(hipGraphLaunch(exec, stream_));
-    else
+      graph_replays++;
+    } else {
       bicgs_body<V>(x, g, gs, herm, nrhs, prec);
+    }
     matvecs += 2 * nact;
     matvecs32 += f32 * 2 * nact;
   }

@@ -130,6 +130,7 @@ class Engine {
   long long matvecs = 0;       // single-rhs operator applications
   long long matvecs32 = 0;     // ... of which with the FP32 operator
   long long solves = 0, solve_iters = 0, refinements = 0;
+  long long graph_replays = 0;  // solver iterations run as a captured graph
 
   void launch_prep(const zd* x, const zd* g, long g_stride, zd* y, bool herm, int nrhs);
 

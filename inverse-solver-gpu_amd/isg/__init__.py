@@ -109,6 +109,7 @@ _SIGS = {
                                             ctypes.c_int, _P(SolveInfo)]),
     "isg_stage": (ctypes.c_int, [_V, ctypes.c_int, ctypes.c_int, ctypes.c_int, _D]),
     "isg_counters": (ctypes.c_int, [_V, _P(ctypes.c_longlong)]),
+    "isg_graph_replays": (ctypes.c_int, [_V, _P(ctypes.c_longlong)]),
     "isg_dbim_setup": (ctypes.c_int, [_V, _D, ctypes.c_int, _P(DbimStats)]),
     "isg_dbim_setup_measured": (ctypes.c_int, [_V, _D, _D, ctypes.c_int, _P(DbimStats)]),
     "isg_profile": (ctypes.c_int, [_V, ctypes.c_int]),
@@ -353,6 +354,12 @@ class Solver:
         self._err(self.lib.isg_counters(self.h, out), "isg_counters")
         return {"matvecs": out[0], "solves": out[1], "solve_iters": out[2], "matvecs_fp32": out[3],
                 "refinements": out[4]}
+
+    def graph_replays(self):
+        """Solver iterations so far that ran as replays of a captured HIP graph."""
+        n = ctypes.c_longlong()
+        self._err(self.lib.isg_graph_replays(self.h, ctypes.byref(n)), "isg_graph_replays")
+        return n.value
 
     # ---- device-pointer surface (pointers are integers, e.g. torch data_ptr())
     def mlfma_dev(self, x_ptr, r_ptr, nrhs=1):
