@@ -83,6 +83,14 @@ __device__ __forceinline__ void block_max(float (&m)[N], float (*red)[kBlock / 6
   }
 }
 
+// 16-byte load from a caller's vector: complex FP32 elements, aligned to 8 bytes
+// only (the loads are the same instructions, which take any such address).
+typedef float v4f_8 __attribute__((ext_vector_type(4), aligned(8)));
+__device__ __forceinline__ float4 h16_load(const zf* p, int i) {  // elements 2 i, 2 i + 1
+  const v4f_8 v = reinterpret_cast<const v4f_8*>(p)[i];
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+
 // a[q] for a runtime q without indexing a private array (which would live in scratch)
 template <typename T>
 __device__ __forceinline__ T sel2(const T (&a)[2], int q) {
@@ -253,14 +261,14 @@ k_near_h16(const zf* __restrict__ y, long ys, const zf* __restrict__ loc, long l
   int es;
   {
     constexpr int NU = 13;  // 100 boxes x 32 float4
-    const float4* yq = reinterpret_cast<const float4*>(y + (long)rhs * ys);
+    const zf* yq = y + (long)rhs * ys;
     float4 v[NU];
     float m[1] = {0.f};
 #pragma unroll
     for (int u = 0; u < NU; u++) {
       const int e = tid + u * kBlock, ec = e < 3200 ? e : 3199;
       const int off = hoff[ec >> 5];
-      v[u] = yq[((off < 0 ? 0 : off) >> 1) + (ec & 31)];
+      v[u] = h16_load(yq, ((off < 0 ? 0 : off) >> 1) + (ec & 31));
       if (off < 0) v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
@@ -521,7 +529,7 @@ k_p2m_h16(const zf* __restrict__ y, long ys, zf* __restrict__ agm, long as, cons
     const long o = (long)sel2(rv, q) * ys + b0 * 64 + 2 * tid;  // + 512 c
     if constexpr (STEP == 0) {
 #pragma unroll
-      for (int c = 0; c < 4; c++) v[q][c] = *reinterpret_cast<const float4*>(y + o + 512 * c);
+      for (int c = 0; c < 4; c++) v[q][c] = h16_load(y + o + 512 * c, 0);
     } else {
       // (a switched-off system's vectors stay as they are)
       if (!sel2(on, q)) {
