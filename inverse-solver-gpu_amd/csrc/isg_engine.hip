@@ -205,9 +205,11 @@ void Engine::upload(DevOp<T>& d) {
   d.shiftL.assign(L, nullptr);
   d.trans.assign(L, nullptr);
   if (cfg_.plan.host_tables) {
-    d.near = up_c(P_.near);
     d.coeffT = up_c(P_.coeffT);
-    d.basisT = up_c(P_.basisT);
+    if constexpr (sizeof(T) == 8) {
+      d.near = up_c(P_.near);
+      d.basisT = up_c(P_.basisT);
+    }
     for (int i = 0; i < L; i++) {
       if (!P_.shiftM[i].empty()) d.shiftM[i] = up_c(P_.shiftM[i]);
       if (!P_.shiftL[i].empty()) d.shiftL[i] = up_c(P_.shiftL[i]);
@@ -224,9 +226,7 @@ void Engine::upload(DevOp<T>& d) {
       return p;
     };
     const int Sl = P_.nsamp[L - 1];
-    d.near = cvt(op64_.near, (size_t)9 * 64 * 64);
     d.coeffT = cvt(op64_.coeffT, (size_t)64 * Sl);
-    d.basisT = cvt(op64_.basisT, (size_t)Sl * 64);
     for (int i = 0; i < L; i++) {
       if (op64_.shiftM[i]) d.shiftM[i] = cvt(op64_.shiftM[i], (size_t)4 * P_.nsamp[i]);
       if (op64_.shiftL[i]) d.shiftL[i] = cvt(op64_.shiftL[i], (size_t)4 * P_.nsamp[i]);

@@ -53,9 +53,9 @@ struct SolveStat {
 // precision T.
 template <typename T>
 struct DevOp {
-  cplx<T>* near = nullptr;     // [9][64][64]
+  cplx<T>* near = nullptr;     // [9][64][64] (FP64; the symmetric tables are formed from it and basisT)
   cplx<T>* coeffT = nullptr;   // [64][S_leaf]
-  cplx<T>* basisT = nullptr;   // [S_leaf][64]
+  cplx<T>* basisT = nullptr;   // [S_leaf][64] (FP64)
   cplx<T>* sym_near = nullptr;  // mirror-symmetric classes of both (k_sym_tables)
   cplx<T>* sym_l2p = nullptr;
   double* sym_p2m = nullptr;  // k_sym_p2m_table (FP64)

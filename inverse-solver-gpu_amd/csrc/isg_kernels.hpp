@@ -140,12 +140,6 @@ struct Mfma<double> {
   }
   static __device__ __forceinline__ int row(int g, int q) { return g + 4 * q; }
   // cr + i ci += d * a   (d data, A operand; a table, B operand; nai = -a.y)
-  static __device__ __forceinline__ void cmac(cplx<double> d, cplx<double> a, double nai, v4& cr, v4& ci) {
-    cr = mac(d.x, a.x, cr);
-    cr = mac(d.y, nai, cr);
-    ci = mac(d.x, a.y, ci);
-    ci = mac(d.y, a.x, ci);
-  }
   // three-product form (Gauss): p1 += dr ar, p2 += di ai, p3 += (dr + di)(ar + ai)
   // with asum = ar + ai; then d a = (p1 - p2) + i (p3 - p1 - p2)
   static __device__ __forceinline__ void cmac3(cplx<double> d, cplx<double> a, double asum, v4& p1, v4& p2, v4& p3) {
@@ -162,12 +156,6 @@ struct Mfma<float> {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int g, int q) { return 4 * g + q; }
-  static __device__ __forceinline__ void cmac(cplx<float> d, cplx<float> a, float nai, v4& cr, v4& ci) {
-    cr = mac(d.x, a.x, cr);
-    cr = mac(d.y, nai, cr);
-    ci = mac(d.x, a.y, ci);
-    ci = mac(d.y, a.x, ci);
-  }
   static __device__ __forceinline__ void cmac3(cplx<float> d, cplx<float> a, float asum, v4& p1, v4& p2, v4& p3) {
     p1 = mac(d.x, a.x, p1);
     p2 = mac(d.y, a.y, p2);
