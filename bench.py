@@ -102,12 +102,22 @@ def measured_traffic(split):
     return None
 
 
-def m2l_bytes_per_rhs(level, numsamp, cbytes, fused=False):
+def fused_from(level, leaf, nrhs):
+    """First level whose M2L and L2L run as one kernel, by the tuning stage
+    "leaf" (0 none, 1 the leaf, -1 the built-in rule: every level from 3 on,
+    the leaf alone below 7168 leaf boxes x right-hand sides); None: separate."""
+    if leaf == 0 or level < 4:
+        return None
+    return level - 1 if leaf == 1 or 4 ** (level - 1) * nrhs < 7168 else 3
+
+
+def m2l_bytes_per_rhs(level, numsamp, cbytes, first=None):
     """Read every multipole once and write every local once, levels 2..leaf;
-    with the fused M2L + L2L kernels also read the parent locals they interpolate."""
+    the fused M2L + L2L kernels of levels first..leaf also read the parent
+    locals they interpolate."""
     b = sum(2 * cbytes * 4 ** i * numsamp[i] for i in range(2, level))
-    if fused:
-        b += sum(cbytes * 4 ** (i - 1) * numsamp[i - 1] for i in range(3, level))
+    if first is not None:
+        b += sum(cbytes * 4 ** (i - 1) * numsamp[i - 1] for i in range(first, level))
     return b
 
 
@@ -184,15 +194,15 @@ def synthesize(isg, common, batch, otrue, iti):
 def run_paths(isg, args, wl, common, otrue, mes, paths, warmup, steps, timing):
     """Time the requested paths from the same measurements; returns a dict:
     res (per path: s/step, stats, kernel timers), contrast (per path), fused
-    (leaf M2L + L2L fused), split (the FP32 near field ran on the split-FP16
+    (per path: fused_from of its operator), split (the FP32 near field ran on the split-FP16
     kernel) and errors (paths skipped)."""
     batch = wl.get("batch", wl["numtx"])
     fast_prec = 1 if args.fast_precision == "mixed" else 0
     fast_kw = dict(max_rhs=batch, precision=fast_prec, mixed_margin=args.mixed_margin,
                    products=1 if args.fast_products == "fp32" and fast_prec == 1 else 0,
                    solve_start=1 if args.fast_solve_start == "previous" else 0)
-    res, contrast, errors = {}, {}, {}
-    fused = split = False
+    res, contrast, errors, fused = {}, {}, {}, {}
+    split = False
     side = 8 << (wl["level"] - 1)
     for p in paths:
         if p == "plain":
@@ -216,9 +226,6 @@ def run_paths(isg, args, wl, common, otrue, mes, paths, warmup, steps, timing):
                 s.close()
                 continue
             ptime = timing
-            # M2L and L2L of a level in one kernel: the leaf (1) or every level (-1, the built-in rule at these sizes)
-            leaf = s.tuning_get(fast_prec, 1, "leaf")
-            fused = fused or leaf in (-1, 1)
             # the split-FP16 near field k_near_h16 (tuning values 128 and 256) serves grids of >= 8 x 8
             # leaf boxes; the built-in rule (-1) takes it from 256 workgroups of 64 boxes on
             nv = s.tuning_get(1, 1 if batch >= 16 else 0, "near")
@@ -226,6 +233,8 @@ def run_paths(isg, args, wl, common, otrue, mes, paths, warmup, steps, timing):
                 nv = 128
             if fast_prec == 1 and nv in (128, 256) and wl["level"] >= 4:
                 split = split or nv
+        prec, nrhs = (0, 1) if p == "plain" else (fast_prec, batch)
+        fused[p] = fused_from(wl["level"], s.tuning_get(prec, 1 if nrhs >= 16 else 0, "leaf"), nrhs)
         res[p] = run_path(s, d, warmup, steps, p, ptime)
         contrast[p] = d.get("o")
         del d
@@ -392,7 +401,7 @@ def main():
 
     runs = run_paths(isg, args, wl, common, otrue, mes, paths, args.warmup, args.steps, timing)
     res, contrast, errors = runs["res"], runs["contrast"], runs["errors"]
-    fast_leaf_fused, fast_split = runs["fused"], runs["split"]
+    fast_split = runs["split"]
     if not res:
         print(json.dumps({"metric": METRIC, "value": None, "error": errors}), flush=True)
         sys.exit(1)
@@ -412,7 +421,7 @@ def main():
         n_near, prec, cb = matvecs, "f64", 16
     vec_ms, vec_n = prof["bicgs_update"]
     achieved = n_near * flops_mv / (near_ms * 1e-3) / 1e12 if near_ms > 0 else 0.0
-    fused = main_path != "plain" and fast_leaf_fused
+    fused = runs["fused"][main_path]
     m2l_gbs = (n_near * m2l_bytes_per_rhs(level, numsamp, cb, fused) / (m2l_ms * 1e-3) / 1e9
                if m2l_ms > 0 else 0.0)
     iters = sum(s["solve_iters"] for s in stats)
@@ -480,7 +489,7 @@ def main():
         },
         "m2l": {"achieved_GBs": round(m2l_gbs, 1), "peak_GBs": PEAK_HBM_GBS, "frac": round(m2l_gbs / PEAK_HBM_GBS, 4),
                 "ms_per_matvec_launchset": round(m2l_ms / max(m2l_n, 1), 4),
-                "leaf_l2l_fused": fused},
+                "leaf_l2l_fused": fused is not None, "fused_from_level": fused},
         # x/r update reads x, p, s, t, r~ and writes x, r: x is FP64 (16 B), the
         # work vectors FP64 (plain) or FP32 (mixed): 7 x 16 B or 2 x 16 + 5 x 8 B per unknown
         "bicgs_update": {"GBs": round((72 if mixed else 112) * side * side * iters / max(vec_ms * 1e-3, 1e-12) / 1e9, 1),
