@@ -53,6 +53,10 @@ import numpy as np  # noqa: E402
 
 METRIC = "s per DBIM iteration, 1024² px ×64 Tx, rel-res 1e-6: plain vs batched+learned"
 PEAK_TFLOPS = {"f64": 78.6, "f32": 157.3, "f16": 2500.0}
+# matrix-core flops that the near-field kernels execute per flop of the dense blocks (8 per complex
+# multiply-add): a quarter of the multiplications in the mirror-symmetric basis, 24 flops each in
+# the split-FP16 kernel (four real products of three part products), 6 in the three-product form
+EXECUTED_PER_DENSE = {"split": 24 / 8 / 4, "three-product": 6 / 8 / 4}
 PEAK_HBM_GBS = 8000.0
 CYCLE = 5  # DBIM iterations of one inversion (the workload's 5; --cycle sets it)
 
@@ -428,6 +432,7 @@ def main():
     split = fast_split if mixed else False
     traffic = measured_traffic(split) if (mixed and level == 8 and ntx == 64) else None
     peak = PEAK_TFLOPS["f16" if split else prec]
+    executed = achieved * EXECUTED_PER_DENSE["split" if split else "three-product"]
     geom = (("on a circle of radius %g lambda (line sources)" % args.radius) if args.radius > 0
             else "(plane waves, far-field receivers)")
 
@@ -476,13 +481,12 @@ def main():
                               "(rocprofv3 FETCH_SIZE x2 + WRITE_SIZE x1, copy-calibrated)"
                               if traffic else None,
             "flops_per_rhs_launch": flops_mv,
-            "note": ("achieved counts the dense blocks' 8 flops per complex multiply-add; the mirror-symmetric basis "
-                     "needs a quarter of those multiplications, and the split kernel executes each real product as "
-                     "three FP16 products (hi.hi + hi.lo + lo.hi) in the four-product complex form: its executed MFMA "
-                     "rate is 0.75 x achieved (0.83 x with the padding of its k-chunks)" if split else
-                     "achieved counts the dense blocks' 8 flops per complex multiply-add; the mirror-symmetric basis "
-                     "needs a quarter of those multiplications, the three-product form 6 of the 8 flops: the executed "
-                     "MFMA rate is 0.19 x achieved"),
+            "executed": round(executed, 2),
+            "executed_frac": round(executed / peak, 4),
+            "note": ("achieved, frac and frac_of_split_ceiling (3 x frac) are dense-equivalent: they count the dense "
+                     "blocks' 8 flops per complex multiply-add, of which the mirror-symmetric basis leaves a quarter of "
+                     "the multiplications, so they may exceed 1.  executed is the rate of the matrix-core flops that "
+                     "run, without the padding of the kernels' k-steps, and executed_frac its share of the peak"),
             "frac_of_split_ceiling": round(3 * achieved / peak, 4) if split else None,
             "avg_launch_ms": round(near_ms / max(near_n, 1), 4),
             "launches": near_n,

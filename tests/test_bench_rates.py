@@ -3,6 +3,10 @@
 M2L: the bytes are every multipole read and every local written once, and the
 parents' locals of the levels whose M2L and L2L are one kernel -- the leaf alone,
 or every level from 3 on, whichever the solver was told.
+
+Near field: achieved and frac count the dense blocks' flops; the matrix cores run
+a quarter of the complex multiplications, of 24 FP16 flops each in the split
+kernel and 6 otherwise, and executed / executed_frac say so.
 """
 import pytest
 
@@ -43,3 +47,12 @@ def test_json_line_counts_the_leaf_alone(bench, monkeypatch):
     want = 500 * bench.m2l_bytes_per_rhs(6, ns, 8, 5) / 10e-3 / 1e9
     assert abs(d["m2l"]["achieved_GBs"] - want) < 0.1
     assert d["m2l"]["leaf_l2l_fused"] is True and d["m2l"]["fused_from_level"] == 5
+
+
+@pytest.mark.parametrize("split,per_dense", [(128, 24 / 32), (0, 6 / 32)])
+def test_executed_rate_counts_the_symmetric_products(monkeypatch, split, per_dense):
+    r = run_bench(monkeypatch, "--workload", "dbim-256", "--steps", "2", "--warmup", "0", "--cpu-baseline", "off",
+                  "--ref-geometry", "off", split=split)["roofline"]
+    assert abs(r["executed"] - per_dense * r["achieved"]) < 0.02
+    assert abs(r["executed_frac"] - r["executed"] / r["peak"]) < 1e-3
+    assert r["executed_frac"] < r["frac"]
