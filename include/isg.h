@@ -261,22 +261,29 @@ int isg_raster_bin_write(const char* path, int numunk, const double* raster);
 int isg_raster_bin_read(const char* path, int numunk, double* raster);
 
 /* ---- autotuner (kernel variants per stage and level, measured on the device) ----
- * stage 0 near-field tile width (16, 32 or 64 boxes; 64 for the FP32
- * operator only; 128 or 256, FP32 operator only: the split-FP16 kernel, 64-box
- * tiles on the FP16 matrix cores with FP32 operands carried as hi + lo), 1 P2M
- * tile width (16, 32 or 64; 128, FP32 operator only: the split-FP16 P2M, 32-box
- * tiles of two right-hand sides, 4 or more right-hand sides), 2 M2L tile
- * variant of `level` (0: 4x4 boxes x 8 samples, 1: 8x8 x 8, 2: 8x8 x 16,
- * 3: 16x16 x 8, 4: 8x8 x 32, 5: 16x16 x 16; 6, 7, 8: 8x8 x 16, 32, 8 with the
- * operators held in registers; 9: 8x8 x 16, one thread per parent, one launch
- * for all levels that have it, and the built-in rule; 4, 5 and 7 FP32 only), 3 / 4
- * M2M / L2L kernel of `level` (0 band MFMA, 1 chunked LDS, 2 direct, 3 / 4 band
- * MFMA with 16 / 32 columns per workgroup), 5 fusion (`level` ignored; FP32
- * operator: M2L and the L2L into a level as one kernel that writes each local
- * expansion once, -1: every level from 3 on, 1: the leaf level, 0: none; the FP64
- * operator runs them separately); value -1 = built-in
- * rule.  precision 0 = FP64 operator, 1 = FP32 operator of the mixed path;
- * batch_class 0 for fewer than 16 right-hand sides, 1 otherwise.
+ * precision 0 = FP64 operator, 1 = FP32 operator of the mixed path; batch_class 0
+ * for fewer than 16 right-hand sides, 1 otherwise; value -1 = built-in rule.
+ *   stage 0  near field: boxes per tile (16, 32 or 64; 64 FP32 operator only), or
+ *            128 or 256 (FP32 operator only): the split-FP16 kernel, 64-box tiles on
+ *            the FP16 matrix cores with FP32 operands carried as hi + lo
+ *   stage 1  P2M: boxes per tile (16, 32 or 64; 64 FP32 operator only), or 128 (FP32
+ *            operator only): the split-FP16 kernel, 32-box tiles of two right-hand
+ *            sides, at every batch size where it also does the leaf level's M2M
+ *            (four and more tree levels, 65 to 72 leaf samples), else from 4
+ *            right-hand sides on.  The FP64 kernel does that M2M at either width
+ *   stage 2  M2L of `level`, where it is not fused (stage 5): 0: 4x4 boxes x 8
+ *            samples, 1: 8x8 x 8, 2: 8x8 x 16, 3: 16x16 x 8, 4: 8x8 x 32, 5: 16x16 x
+ *            16; 6, 7, 8: 8x8 x 16, 32, 8 with the operators held in registers; 9: 8x8
+ *            x 16, one thread per parent, one launch for all levels that have it, and
+ *            the built-in rule; 4, 5 and 7 FP32 only
+ *   stage 3, 4  M2M / L2L of `level`: 0 band MFMA, 1 chunked LDS, 2 direct, 3 / 4 band
+ *            MFMA with 16 / 32 columns per workgroup (L2L: where it is not fused; M2M:
+ *            not of the leaf level where P2M does it)
+ *   stage 5  fusion, either operator (`level` ignored): M2L and the L2L into a level as
+ *            one kernel that writes each local expansion once.  0: none, 1: the leaf
+ *            level, -1: every level from 3 on, the leaf level alone below 7168 leaf
+ *            boxes x right-hand sides; none where an interpolation window of some
+ *            level exceeds 96 samples
  * isg_autotune times every admissible variant (reps launches each) and keeps
  * the fastest for batch_class(nrhs) and every operator precision the context has.
  * The file holds lines "tree-depth precision batch_class stage level value";
@@ -290,11 +297,12 @@ int isg_tuning_load(isg_context* ctx, const char* path);
 /* ---- live kernel timing (HIP events on the context's stream; the reference
  * times whole matvecs with cudaEvents, matvec_gpu.cu:117-122) ----
  * kernel 0: near field + L2P on the matrix cores, one launch per matvec
- * kernel 1: M2L over all levels of one matvec
+ * kernel 1: M2L over all levels of one matvec, with the L2L that is fused with it
  * kernel 2: BiCGSTAB x/r update with its two dot products
  * kernel 3, 4: as 0, 1 for the FP32 operator of the mixed path
- * kernel 5: P2M of one matvec (either precision)
- * kernel 6: M2M and L2L interpolation of one matvec (either precision)
+ * kernel 5: P2M of one matvec (either precision), with the leaf level's M2M and the
+ *           solver's p and s updates where P2M does them
+ * kernel 6: the other M2M and L2L interpolation of one matvec (either precision)
  * kernel 7: receiver operator (isg_aggregate / isg_aggregateh and the DBIM
  *           loop's receiver products), one launch set per call
  * isg_profile(ctx, 1) clears the totals and starts recording. */

@@ -1,12 +1,13 @@
-// isg_down.hpp -- downward pass of one level of the FP32 operator: its
-// translations (M2L) and the interpolation of the parents' locals (L2L) in one
-// kernel, the interpolation on the FP16 matrix cores with split operands.
+// isg_down.hpp -- downward pass of one level: its translations (M2L) and the
+// interpolation of the parents' locals (L2L) in one kernel.  k_down_h16: the FP32
+// operator, interpolating on the FP16 matrix cores with split operands; k_down64:
+// the FP64 operator, on the FP64 ones.
 //
 // local_i[box][k] = sum over the 27 far boxes of T[k] multipole_i[box'][k]
 //                 + sum_j A[k][j] shiftL[c][j] local_{i-1}[parent][j]
 // Reference counterpart: kernels.cu:239-266 and :137-238.
 //
-// The shift of child position c is folded into the anterpolator (a complex
+// FP32: the shift of child position c is folded into the anterpolator (a complex
 // table per child position), so that the operand is the parents' locals
 // themselves: 16 parents x the window of 16 samples, split once into FP16 hi +
 // lo (isg_near_h16.hpp) under one power-of-two scale per parent, for four child

@@ -605,10 +605,14 @@ void Engine::build_down() {
 // tuning stage "leaf": 0 none, 1 the leaf alone, -1 the rule.  A workgroup takes
 // 64 boxes and the levels above the leaf have few of those, each with many
 // sample chunks that repeat the set-up, so a small product fuses the leaf only.
-// All levels / the leaf / none, us a product: FP64 256 px x 1 70 / 64 / 64, x 4
-// 82 / 76 / 89, x 8 99 / 100 / 125, 512 px x 1 95 / 87 / 88, x 4 149 / 161 / 158,
-// x 16 393 / 409 / 428; FP32 256 px x 1 58 / 55 / 54, x 7 72 / 72 / 80, 512 px x 1
-// 72 / 68 / 72.
+// All levels / the leaf alone, us a product by boxes x right-hand sides: FP64 4096
+// (128 px x 16) 66.8 / 66.9, (256 px x 4) 71.9 / 69.1, (512 px x 1) 83.3 / 80.1; 5120
+// (256 px x 5) 78.7 / 78.8; 6144 79.2 / 80.6; 7168 82.1 / 86.2; 8192 86.8 / 90.5, (512
+// px x 2) 99 / 101.  FP32 4096 60.8 / 57.8 (256 px x 4), 71.3 / 67.4 (512 px x 1); 6144
+// 66.2 / 65.5 (256 px x 6), 71.2 / 71.9 (128 px x 24); 7168 68.3 / 69.0; 8192 70.8 /
+// 71.0, 80.7 / 80.5; 12288 77.8 / 79.5.  One line for both: where the slower of them,
+// FP32 at 256 px, crosses.  Neither fused: FP64 256 px x 8 125 instead of 99, FP32 256
+// px x 7 80 instead of 72 (an earlier state of the kernels).
 int Engine::fuse_level(int choice, int nrhs) const {
   if (down_.empty() || choice == 0) return P_.L;
   return choice == 1 || (long)P_.B * nrhs < 7168 ? P_.L - 1 : 3;
@@ -737,8 +741,9 @@ bool Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
   const int Lf = P_.L - 1, S = P_.nsamp[Lf], B = P_.B;
   const int tuned = tune(sizeof(T) == 4 ? PREC_MIXED : PREC_FP64, nrhs).p2m_nb;
   // built-in rule: where a kernel does the leaf level's M2M along with P2M, that one -- FP32: the split-FP16
-  // kernel, a product of 64 px x 1 38 -> 30 us, 128 px x 1 62 -> 54, 256 px x 1 54.5 -> 51, x 7 70 -> 68.5,
-  // 512 px x 1 65.7 -> 66.5, x 8 135 -> 121, 1024 px x 2 146 -> 133; FP64: the mirror-symmetric one on 16-box
+  // kernel, a product of 64 px x 1 38 -> 30 us, 128 px x 1 62 -> 54, 256 px x 1 54.4 -> 51.0, x 7 70 -> 68.5,
+  // 512 px x 3 92.6 -> 91.2, x 8 135 -> 121, 1024 px x 1 109.6 -> 106.8, x 2 146 -> 133 (alike at 512 px x 1,
+  // 66.1 -> 66.2, and 1 % slower at x 2, 80.0 -> 80.9); FP64: the mirror-symmetric one on 16-box
   // tiles (512 px x 16: 55 us, 32-box tiles 61; 1024 px x 64: 870, 910) --, else the dense kernel on 32-box
   // tiles once they fill the chip and 16 below (64 px, one system: 12.9 -> 9.6 us)
   const bool sym = sizeof(T) == 8 && S <= kP2mSymS;

@@ -143,10 +143,10 @@ class Engine {
   void profile_read(int id, double& ms, long long& launches);
 
   // Kernel-variant choices per operator precision and batch class (nrhs < 16
-  // or >= 16); -1 = the built-in rule.  Stages: near/P2M tile width (16 or 32
-  // boxes), M2L tile variant per level (kM2LVariants), M2M/L2L kernel kind per
-  // level (0 band MFMA, 1 chunked LDS, 2 direct, 3 / 4 band MFMA with 16 / 32
-  // columns per workgroup).
+  // or >= 16); -1 = the built-in rule.  Stages: near/P2M tile width (16, 32 or 64
+  // boxes, or the split-FP16 kernel), M2L variant per level (kM2LVariants), M2M/L2L
+  // kernel kind per level (0 band MFMA, 1 chunked LDS, 2 direct, 3 / 4 band MFMA with
+  // 16 / 32 columns per workgroup), fusion of M2L and L2L.
   enum { ST_NEAR = 0, ST_P2M = 1, ST_M2L = 2, ST_M2M = 3, ST_L2L = 4, ST_LEAF = 5, ST_COUNT = 6 };
   struct Tuning {
     int near_nb = -1, p2m_nb = -1;

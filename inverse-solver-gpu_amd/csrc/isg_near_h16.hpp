@@ -4,9 +4,14 @@
 //
 // Every FP32 operand x is carried as two FP16 numbers, hi = rne16(2^e x) and
 // lo = rne16(2^e x - hi), with a power-of-two scale 2^e chosen so that
-// |2^e x| < 2^14 -- per table, and per workgroup and right-hand side for the
-// data.  hi + lo holds x to 2^-22 relative (elements below 2^-16 of the
-// largest one, whose lo is subnormal, to 2^-38 of the largest, absolutely).  A product x a is formed
+// |2^e x| < 2^14 -- per table, and for the data per workgroup and right-hand side
+// (the leaf level's M2M: per box; k_down_h16: per parent).  hi + lo holds x to 2^-22
+// relative (elements below 2^-16 of the largest one, whose lo is subnormal, to 2^-38
+// of the largest, absolutely; the largest one's field reaches every output of the
+// workgroup, so that does not show: with amplitudes over 30 and 40 octaves and with
+// point sources 2^24 above the rest, the error of each leaf box relative to its own
+// field is that of the FP32 kernels or less, 1 to 15 right-hand sides, 64 to 2048
+// px).  A product x a is formed
 // as hi.hi + hi.lo + lo.hi in FP32 accumulators (the dropped lo.lo term is
 // below 2^-22 relative): three FP16 MFMAs, each 16 times the FP32 rate, for
 // one FP32 MFMA's worth of products.  Complex products take the four-product
@@ -467,8 +472,8 @@ __device__ __forceinline__ float row_max(float v) {
 // between lanes, with three to five arrays in flight, ran from L2: 697 -> 557 us
 // for STEP 2 at 1024 px x 64), its largest component per
 // right-hand side sets the data scale, and it is staged split in LDS as
-// [rhs][part][pixel group 8][box 32] x 8 FP16 (boxes XOR 2 (g mod 4), as in
-// k_near_h16).  Wave w owns right-hand side w / 2, row block w % 2 (16
+// [rhs][part][pixel group 8][box 32] x 8 FP16 (boxes XOR 2 (g mod 4) against
+// bank conflicts).  Wave w owns right-hand side w / 2, row block w % 2 (16
 // boxes) and all ceil(S / 16) column blocks (samples); K = 64 pixels in two
 // MFMA chunks of 32.  The coefficient table coef[kc][part][g][s] (s padded to
 // 16 ceil(S / 16), zero beyond S) carries its own scale 2^ec.  Results go
@@ -486,7 +491,7 @@ __device__ __forceinline__ float row_max(float v) {
 // wave w takes the parent samples 16 w + 64 u of all four row blocks.  A lane
 // ends with the four children of one parent: shifted and summed in registers.
 // HBM bounds both: alone, P2M wrote the multipoles in 239 us and M2M, on FP32
-// matrix products, read them again in 289 us (1024 px x 64); together 376 us, and
+// matrix products, read them again in 289 us (1024 px x 64); together 361 us, and
 // with STEP 2 or 3 620 and 566 instead of 557 + 289 and 485 + 289.
 constexpr int kP2mH16MaxCB = 6;  // column blocks held per wave (S <= 96)
 constexpr int kUpWin = 48, kUpPitch = 120, kUpRounds = 2, kUpCB = 5;
