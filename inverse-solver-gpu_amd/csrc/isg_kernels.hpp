@@ -377,8 +377,8 @@ __device__ __forceinline__ void near_epilogue(const cplx<T>* tile, cplx<TI>* __r
 // The upper levels have little work (16 parents of 1036 samples at 1024^2) and
 // these kernels were bound by the latency of their serial tap loop, each tap
 // waiting for its weight from L2: the weights, shifts and first-tap indices of a
-// thread are now loaded into registers before the staging (NT taps, compiled in;
-// 0: any count, loaded tap by tap), and the staging steps its indices instead of
+// thread are now loaded into registers before the staging (NT taps, compiled in for
+// the default 30 and 60; 0: any count, loaded along the way), and the staging steps its indices instead of
 // dividing.  Per launch at 512^2 x 15 right-hand sides (FP32): M2M 14.5 -> 8.5 us,
 // L2L 19.6 -> 17.4 us.
 
@@ -439,24 +439,38 @@ __global__ void __launch_bounds__(kBlock) k_m2m_chunk(const cplx<T>* __restrict_
   int d = ik - base;
   if (d < 0) d += Sc;
   cplx<T> acc = mkc<T>(0, 0);
+  if constexpr (NT > 0) {
 #pragma unroll
-  for (int c = 0; c < 4; c++) {
-    const cplx<T>* src = lds + (4 * g + c) * W + d;
-    cplx<T> red = mkc<T>(0, 0);
-    if constexpr (NT > 0) {
+    for (int c = 0; c < 4; c++) {
+      const cplx<T>* src = lds + (4 * g + c) * W + d;
+      cplx<T> red = mkc<T>(0, 0);
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         red.x += w[t] * src[t].x;
         red.y += w[t] * src[t].y;
       }
-    } else {
-      for (int t = 0; t < ntap; t++) {
-        const T wt = wT[t * Sp + k];
-        red.x += wt * src[t].x;
-        red.y += wt * src[t].y;
+      acc = cfma(red, sh[c], acc);
+    }
+  } else {
+    // a weight is loaded once for the four children, several in flight (M2M above the
+    // leaf at 512 px x 2, 28 taps: child by child FP64 59 us and FP32 43, with two taps
+    // in flight 45 and 41, with four 34 and 47)
+    constexpr int U = sizeof(T) == 8 ? 4 : 2;
+    const cplx<T>* src = lds + 4 * g * W + d;
+    cplx<T> red[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) red[c] = mkc<T>(0, 0);
+#pragma unroll U
+    for (int t = 0; t < ntap; t++) {
+      const T wt = wT[t * Sp + k];
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        red[c].x += wt * src[c * W + t].x;
+        red[c].y += wt * src[c * W + t].y;
       }
     }
-    acc = cfma(red, sh[c], acc);
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc = cfma(red[c], sh[c], acc);
   }
   par[rhs * ps + (p0 + g) * Sp + k] = acc;
 }
