@@ -744,15 +744,17 @@ bool Engine::launch_p2m(const cplx<TI>* y, int nrhs, const int* act, int force, 
   // kernel, a product of 64 px x 1 38 -> 30 us, 128 px x 1 62 -> 54, 256 px x 1 54.4 -> 51.0, x 7 70 -> 68.5,
   // 512 px x 3 92.6 -> 91.2, x 8 135 -> 121, 1024 px x 1 109.6 -> 106.8, x 2 146 -> 133 (alike at 512 px x 1,
   // 66.1 -> 66.2, and 1 % slower at x 2, 80.0 -> 80.9); FP64: the mirror-symmetric one on 16-box
-  // tiles (512 px x 16: 55 us, 32-box tiles 61; 1024 px x 64: 870, 910) --, else the dense kernel on 32-box
-  // tiles once they fill the chip and 16 below (64 px, one system: 12.9 -> 9.6 us)
+  // tiles (512 px x 16: 55 us, 32-box tiles 61; 1024 px x 64: 870, 910).  Else, in FP32, the split kernel
+  // alone once its workgroups fill the chip (36 taps, dense / split: 256 px x 8, 128 workgroups, 95.9 / 96.9 us;
+  // 512 px x 4, 256, 123.4 / 123.2; x 5, 384, 143.6 / 141.5; 1024 px x 16 961 / 924), and the dense kernel on
+  // 32-box tiles once they fill the chip and 16 below (64 px, one system: 12.9 -> 9.6 us)
   const bool sym = sizeof(T) == 8 && S <= kP2mSymS;
   const int mode = step ? step->mode : 0;
   const bool h16 = sizeof(T) == 4 && sizeof(TI) == 4 && mode != 1 && B % 32 == 0 && p2m16_;
   const bool h16_up = h16 && up && up16_;
+  const bool split = h16_up || (h16 && nrhs >= 4 && (long)(B / 32) * ((nrhs + 1) / 2) >= 256);
   int nb = force > 0 ? force
-                     : (tuned > 0 ? tuned
-                                  : (h16_up ? kNearSplit : (!sym && (long)(B / 32) * nrhs >= 256 ? 32 : 16)));
+                     : (tuned > 0 ? tuned : (split ? kNearSplit : (!sym && (long)(B / 32) * nrhs >= 256 ? 32 : 16)));
   DevOp<T>& d = ops<T>();
   cplx<T>* out = d.agm + lvl_off_[Lf];
   long as = (long)lvl_size_[Lf];
