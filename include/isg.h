@@ -269,8 +269,9 @@ int isg_raster_bin_read(const char* path, int numunk, double* raster);
  *   stage 1  P2M: boxes per tile (16, 32 or 64; 64 FP32 operator only), or 128 (FP32
  *            operator only): the split-FP16 kernel, 32-box tiles of two right-hand
  *            sides, at every batch size where it also does the leaf level's M2M
- *            (four and more tree levels, 65 to 72 leaf samples), else from 4
- *            right-hand sides on.  The FP64 kernel does that M2M at either width
+ *            (four and more tree levels, 65 to 72 leaf samples, 30 taps at the
+ *            default resolution), else from 4 right-hand sides on.  The FP64 kernel
+ *            does that M2M at either width (124 leaf samples, 38 taps)
  *   stage 2  M2L of `level`, where it is not fused (stage 5): 0: 4x4 boxes x 8
  *            samples, 1: 8x8 x 8, 2: 8x8 x 16, 3: 16x16 x 8, 4: 8x8 x 32, 5: 16x16 x
  *            16; 6, 7, 8: 8x8 x 16, 32, 8 with the operators held in registers; 9: 8x8
